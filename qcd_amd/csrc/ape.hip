@@ -21,76 +21,131 @@ using C = Cx<double>;
 __device__ __forceinline__ C cm(C a, C b) { return C{fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)}; }
 __device__ __forceinline__ C cj(C a) { return C{a.re, -a.im}; }
 
-// c = a b (DA: a^+, DB: b^+)
-template <bool DA, bool DB>
+// c (+)= a b (DA: a^+, DB: b^+; ADD: added to c): a chain of fused
+// multiply-adds per element, 108 instructions
+template <bool DA, bool DB, bool ADD = false>
 __device__ __forceinline__ void mm3(C c[9], const C a[9], const C b[9]) {
 #pragma unroll
   for (int i = 0; i < 3; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-      C s{0.0, 0.0};
+      double re, im;
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         const C x = DA ? cj(a[3 * k + i]) : a[3 * i + k];
         const C y = DB ? cj(b[3 * j + k]) : b[3 * k + j];
-        const C p = cm(x, y);
-        s = C{s.re + p.re, s.im + p.im};
+        if (k == 0 && !ADD) {
+          re = x.re * y.re;
+          im = x.re * y.im;
+        } else {
+          re = fma(x.re, y.re, k == 0 ? c[3 * i + j].re : re);
+          im = fma(x.re, y.im, k == 0 ? c[3 * i + j].im : im);
+        }
+        re = fma(-x.im, y.im, re);
+        im = fma(x.im, y.re, im);
       }
-      c[3 * i + j] = s;
+      c[3 * i + j] = C{re, im};
     }
 }
 
-__device__ __forceinline__ C det3(const C a[9]) {
-  C d{0.0, 0.0};
-#pragma unroll
-  for (int c = 0; c < 3; c++) {   // expansion along row 0, cyclic minors carry their sign
-    const C t = cm(a[3 + (c + 1) % 3], a[6 + (c + 2) % 3]);
-    const C s = cm(a[3 + (c + 2) % 3], a[6 + (c + 1) % 3]);
-    d = C{d.re + a[c].re * (t.re - s.re) - a[c].im * (t.im - s.im), d.im + a[c].re * (t.im - s.im) + a[c].im * (t.re - s.re)};
-  }
-  return d;
+// 1 / x and 1 / sqrt(x) for normal x > 0: the hardware's approximation and
+// two Newton steps.  Zero, infinity and NaN give infinity, zero or NaN.
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double rsqrt_pos(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
 }
 
-// SU(3) projection in place
-__device__ void project_su3(C m[9]) {
+// cofactor of element (r, c) of a 3x3 matrix
+__device__ __forceinline__ C cof3(const C x[9], int r, int c) {
+  const int r1 = (r + 1) % 3, r2 = (r + 2) % 3, c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+  const C p = x[3 * r1 + c1], q = x[3 * r2 + c2], u = x[3 * r1 + c2], v = x[3 * r2 + c1];
+  return C{fma(p.re, q.re, fma(-p.im, q.im, fma(-u.re, v.re, u.im * v.im))),
+           fma(p.re, q.im, fma(p.im, q.re, fma(-u.re, v.im, -(u.im * v.re))))};
+}
+
+// SU(3) projection in place: Newton's iteration X <- (g X + X^-+ / g) / 2.
+//
+// The FP64 arithmetic of this loop and of the staples bounds the smearing
+// kernels, so a step spends nothing that the result does not need:
+//  * any positive factors in place of g and 1/g leave the polar factor as it
+//    is, so the Frobenius scaling (|X^-1| / |X|)^1/2 is a single-precision
+//    fourth root with the exponents split off (it cannot over- or underflow),
+//    taken while the last change was above 1e-2 per unit;
+//  * an unscaled step that changed X by D leaves an error of |D|^2 / 2, so
+//    the loop ends at |D|^2 <= 1e-17 without a step that confirms it;
+//  * the phase exp(-i arg(det M) / 3) starts from single precision and takes two
+//    Newton steps z <- z (4 - z^3 conj(w)) / 3 for z^3 = w, |w| = 1.
+// 24^3x48: an APE step 446-468 -> 322 us with these and the fused products.
+__device__ __forceinline__ void project_su3(C m[9]) {
   C x[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) x[k] = m[k];
+  C w{0.0, 0.0};   // conj(det M) / |det M|
+  double diff = 1.0;
   for (int it = 0; it < 100; it++) {
     // y = (x^-1)^+ = conj(cofactor(x)) / conj(det x)
-    const C d = det3(x);
-    const double rdd = 1.0 / (d.re * d.re + d.im * d.im);
     C y[9];
-    double nx = 0.0, ny = 0.0;
 #pragma unroll
     for (int r = 0; r < 3; r++)
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const int r1 = (r + 1) % 3, r2 = (r + 2) % 3, c1 = (c + 1) % 3, c2 = (c + 2) % 3;
-        const C t = cm(x[3 * r1 + c1], x[3 * r2 + c2]);
-        const C s = cm(x[3 * r1 + c2], x[3 * r2 + c1]);
-        const C cof{t.re - s.re, t.im - s.im};
-        // cof / det, then conjugate
-        const C q{(cof.re * d.re + cof.im * d.im) * rdd, (cof.im * d.re - cof.re * d.im) * rdd};
-        y[3 * r + c] = cj(q);
-        nx += x[3 * r + c].re * x[3 * r + c].re + x[3 * r + c].im * x[3 * r + c].im;
-        ny += q.re * q.re + q.im * q.im;
+      for (int c = 0; c < 3; c++) y[3 * r + c] = cof3(x, r, c);
+    C d = cm(x[0], y[0]);
+#pragma unroll
+    for (int c = 1; c < 3; c++)
+      d = C{fma(x[c].re, y[c].re, fma(-x[c].im, y[c].im, d.re)), fma(x[c].re, y[c].im, fma(x[c].im, y[c].re, d.im))};
+    const double dd = fma(d.re, d.re, d.im * d.im);
+    if (it == 0) {
+      const double rd = rsqrt_pos(dd);
+      w = C{d.re * rd, -(d.im * rd)};
+    }
+    const double rdd = recip(dd);
+    double g = 0.5, rg = 0.5;
+    const bool scale = !(diff <= 1e-4);
+    if (scale) {
+      double nx = 0.0, ny = 0.0;
+#pragma unroll
+      for (int k = 0; k < 9; k++) {
+        nx = fma(x[k].re, x[k].re, fma(x[k].im, x[k].im, nx));
+        ny = fma(y[k].re, y[k].re, fma(y[k].im, y[k].im, ny));
       }
-    const double g = it < 8 ? sqrt(sqrt(ny / nx)) : 1.0, rg = 1.0 / g;
-    double diff = 0.0;
+      ny *= rdd;   // |X^-1|^2
+      // ny / nx = 2^(4 q) f with f in (1/2, 16): g = 2^q f^1/4
+      const int e = __builtin_amdgcn_frexp_exp(ny) - __builtin_amdgcn_frexp_exp(nx), q = e >> 2;
+      const float f = ldexpf((float)__builtin_amdgcn_frexp_mant(ny) *
+                                 __builtin_amdgcn_rcpf((float)__builtin_amdgcn_frexp_mant(nx)),
+                             e - 4 * q);
+      const float h = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(f));
+      g = ldexp((double)h, q - 1);
+      rg = ldexp((double)__builtin_amdgcn_rcpf(h), -q - 1);
+    }
+    // conj(cof / d) rg = conj(cof) d rdd rg
+    const C s{d.re * rdd * rg, d.im * rdd * rg};
+    diff = 0.0;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
-      const C n{0.5 * (g * x[k].re + y[k].re * rg), 0.5 * (g * x[k].im + y[k].im * rg)};
-      diff += (n.re - x[k].re) * (n.re - x[k].re) + (n.im - x[k].im) * (n.im - x[k].im);
+      const C q = cm(cj(y[k]), s);
+      const C n{fma(g, x[k].re, q.re), fma(g, x[k].im, q.im)};
+      const double dr = n.re - x[k].re, di = n.im - x[k].im;
+      diff = fma(dr, dr, fma(di, di, diff));
       x[k] = n;
     }
-    if (diff <= 1e-30) break;   // a fixed point of the scaled step is unitary
+    if (!scale && diff <= 1e-17) break;
   }
-  const C d = det3(m);
-  const double ph = atan2(d.im, d.re) / 3.0;
-  const C e{cos(ph), -sin(ph)};
+  const float ph = -atan2f((float)-w.im, (float)w.re) / 3.0f;
+  C z{(double)__cosf(ph), (double)__sinf(ph)};
 #pragma unroll
-  for (int k = 0; k < 9; k++) m[k] = cm(x[k], e);
+  for (int i = 0; i < 2; i++) {
+    const C t = cm(cm(cm(z, z), z), cj(w));
+    z = cm(z, C{(4.0 - t.re) * (1.0 / 3.0), t.im * (-1.0 / 3.0)});
+  }
+#pragma unroll
+  for (int k = 0; k < 9; k++) m[k] = cm(x[k], z);
 }
 
 // Plaquette sum of one site over the 6 planes mu < nu (qcd_observables.c:15-36):
@@ -135,54 +190,103 @@ __device__ __forceinline__ double stout_xi0(double w) {
 
 // m <- exp(i m) for Hermitian traceless m: f0 + f1 Q + f2 Q^2 with the
 // Cayley-Hamilton coefficients of Peardon & Morningstar (hep-lat/0311018
-// eqs. 19, 29-34; qcd_smearing.c:293-370).  Where the reference divides 0 by
-// 0 (tr Q^2 / 2 below 1e-24, e.g. the unit gauge field) this uses
-// 1 + iQ - Q^2/2, exact to double precision there; where rounding puts the
-// argument of acos above 1 (two equal eigenvalues) it is clamped to 1.  The
-// reference returns NaN in both cases.
-__device__ void stout_exp(C m[9]) {
-  C m2[9], m3[9];
-  mm3<false, false>(m2, m, m);
-  mm3<false, false>(m3, m2, m);
-  double c0 = (m3[0].re + m3[4].re + m3[8].re) / 3.0;
-  const double c1 = (m2[0].re + m2[4].re + m2[8].re) / 2.0;
-  if (c1 < 1e-24) {
+// eqs. 19, 29-34; qcd_smearing.c:293-370).  Where rounding puts the argument
+// of acos above 1 (two equal eigenvalues) it is clamped to 1; at Q = 0 the
+// reference divides 0 by 0.  It returns NaN in both cases.
+//
+// For tr Q^2 / 2 <= 3/4 the eigenvalues are at most 1 in size and the
+// coefficients come from the exponential series instead: Q^3 = c1 Q + c0 gives
+// Q^n = a_n + b_n Q + d_n Q^2 with a' = c0 d, b' = a + c1 d, d' = b (real), and
+// 21 orders reach 1/21! = 2e-20.  No trigonometric functions, no division by
+// 9 u^2 - w^2 (which is small for nearly equal eigenvalues).  A step of
+// rho = 0.1 stays below it on any SU(3) field (|Q| <= 0.6).
+__device__ __forceinline__ void stout_exp(C m[9]) {
+  // Q^2, Hermitian
+  C m2[9];
 #pragma unroll
-    for (int k = 0; k < 9; k++)
-      m[k] = C{(k % 4 == 0 ? 1.0 : 0.0) - m[k].im - 0.5 * m2[k].re, m[k].re - 0.5 * m2[k].im};
-    return;
+  for (int i = 0; i < 3; i++) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) t = fma(m[3 * i + k].re, m[3 * i + k].re, fma(m[3 * i + k].im, m[3 * i + k].im, t));
+    m2[4 * i] = C{t, 0.0};
+#pragma unroll
+    for (int j = i + 1; j < 3; j++) {
+      C q = cm(m[3 * i], m[j]);
+#pragma unroll
+      for (int k = 1; k < 3; k++) {
+        const C x = m[3 * i + k], y = m[3 * k + j];
+        q = C{fma(x.re, y.re, fma(-x.im, y.im, q.re)), fma(x.re, y.im, fma(x.im, y.re, q.im))};
+      }
+      m2[3 * i + j] = q;
+      m2[3 * j + i] = cj(q);
+    }
   }
-  const bool neg = c0 < 0.0;
-  if (neg) c0 = -c0;
-  const double c0max = 2.0 * pow(c1 / 3.0, 1.5);
-  const double theta = acos(c0 < c0max ? c0 / c0max : 1.0);   // degenerate spectra: rounding can exceed 1
-  const double u = sqrt(c1 / 3.0) * cos(theta / 3.0);
-  const double w = sqrt(c1) * sin(theta / 3.0);
-  const double xi = stout_xi0(w), cw = cos(w);
-  const C e2iu{cos(2 * u), sin(2 * u)}, emiu{cos(u), -sin(u)};
-  const C h0 = [&] {
-    const C a = cm(C{u * u - w * w, 0.0}, e2iu), b = cm(emiu, C{8 * u * u * cw, 2 * u * (3 * u * u + w * w) * xi});
-    return C{a.re + b.re, a.im + b.im};
-  }();
-  const C h1 = [&] {
-    const C a = cm(C{2 * u, 0.0}, e2iu), b = cm(emiu, C{2 * u * cw, -(3 * u * u - w * w) * xi});
-    return C{a.re - b.re, a.im - b.im};
-  }();
-  const C h2 = [&] {
-    const C b = cm(emiu, C{cw, 3 * u * xi});
-    return C{e2iu.re - b.re, e2iu.im - b.im};
-  }();
-  const double fac = 9 * u * u - w * w;
-  // eq. (34): f_j(-c0) = (-1)^j conj(f_j(c0))
-  const C f0 = neg ? C{h0.re / fac, -h0.im / fac} : C{h0.re / fac, h0.im / fac};
-  const C f1 = neg ? C{-h1.re / fac, h1.im / fac} : C{h1.re / fac, h1.im / fac};
-  const C f2 = neg ? C{h2.re / fac, -h2.im / fac} : C{h2.re / fac, h2.im / fac};
+  // c0 = tr Q^3 / 3, c1 = tr Q^2 / 2
+  double c0 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      c0 = fma(m2[3 * i + j].re, m[3 * j + i].re, fma(-m2[3 * i + j].im, m[3 * j + i].im, c0));
+  c0 *= 1.0 / 3.0;
+  const double c1 = (m2[0].re + m2[4].re + m2[8].re) / 2.0;
+  C f0, f1, f2;
+  if (c1 <= 0.75) {
+    // scaled by 1/n!: a, b, d hold a_n / n!
+    double a = 1.0, b = 0.0, d = 0.0;
+    f0 = C{1.0, 0.0};
+    f1 = f2 = C{0.0, 0.0};
+#pragma unroll
+    for (int n = 1; n <= 21; n++) {
+      const double r = 1.0 / n, na = c0 * d * r, nb = fma(c1, d, a) * r, nd = b * r;
+      a = na;
+      b = nb;
+      d = nd;
+      if (n % 2 == 0) {   // i^n real
+        const double sg = n % 4 == 0 ? 1.0 : -1.0;
+        f0.re = fma(sg, a, f0.re);
+        f1.re = fma(sg, b, f1.re);
+        f2.re = fma(sg, d, f2.re);
+      } else {
+        const double sg = n % 4 == 1 ? 1.0 : -1.0;
+        f0.im = fma(sg, a, f0.im);
+        f1.im = fma(sg, b, f1.im);
+        f2.im = fma(sg, d, f2.im);
+      }
+    }
+  } else {
+    const bool neg = c0 < 0.0;
+    if (neg) c0 = -c0;
+    const double c0max = 2.0 * pow(c1 / 3.0, 1.5);
+    const double theta = acos(c0 < c0max ? c0 / c0max : 1.0);   // degenerate spectra: rounding can exceed 1
+    const double u = sqrt(c1 / 3.0) * cos(theta / 3.0);
+    const double w = sqrt(c1) * sin(theta / 3.0);
+    const double xi = stout_xi0(w), cw = cos(w);
+    const C e2iu{cos(2 * u), sin(2 * u)}, emiu{cos(u), -sin(u)};
+    const C h0 = [&] {
+      const C a = cm(C{u * u - w * w, 0.0}, e2iu), b = cm(emiu, C{8 * u * u * cw, 2 * u * (3 * u * u + w * w) * xi});
+      return C{a.re + b.re, a.im + b.im};
+    }();
+    const C h1 = [&] {
+      const C a = cm(C{2 * u, 0.0}, e2iu), b = cm(emiu, C{2 * u * cw, -(3 * u * u - w * w) * xi});
+      return C{a.re - b.re, a.im - b.im};
+    }();
+    const C h2 = [&] {
+      const C b = cm(emiu, C{cw, 3 * u * xi});
+      return C{e2iu.re - b.re, e2iu.im - b.im};
+    }();
+    const double fac = 9 * u * u - w * w;
+    // eq. (34): f_j(-c0) = (-1)^j conj(f_j(c0))
+    f0 = neg ? C{h0.re / fac, -h0.im / fac} : C{h0.re / fac, h0.im / fac};
+    f1 = neg ? C{-h1.re / fac, h1.im / fac} : C{h1.re / fac, h1.im / fac};
+    f2 = neg ? C{h2.re / fac, -h2.im / fac} : C{h2.re / fac, h2.im / fac};
+  }
 #pragma unroll
   for (int k = 0; k < 9; k++) {
-    const C a = cm(f1, m[k]), b = cm(f2, m2[k]);
-    C r{a.re + b.re, a.im + b.im};
-    if (k % 4 == 0) r = C{r.re + f0.re, r.im + f0.im};
-    m[k] = r;
+    const C p = m[k], q = m2[k];
+    C r = k % 4 == 0 ? f0 : C{0.0, 0.0};
+    r = C{fma(f1.re, p.re, fma(-f1.im, p.im, r.re)), fma(f1.re, p.im, fma(f1.im, p.re, r.im))};
+    m[k] = C{fma(f2.re, q.re, fma(-f2.im, q.im, r.re)), fma(f2.re, q.im, fma(f2.im, q.re, r.im))};
   }
 }
 
@@ -198,37 +302,50 @@ __device__ __forceinline__ unsigned bwd_dir(unsigned mu, const Site &st, const D
                                            : mu == 2 ? neighbour<2, -1>(st, a) : neighbour<3, -1>(st, a);
 }
 
-// c += a b (DA: a^+, DB: b^+); each element's product is summed from zero
-// and then added, the rounding of computing a b first
-template <bool DA, bool DB>
-__device__ __forceinline__ void mm3_add(C c[9], const C a[9], const C b[9]) {
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      C s{0.0, 0.0};
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const C x = DA ? cj(a[3 * k + i]) : a[3 * i + k];
-        const C y = DB ? cj(b[3 * j + k]) : b[3 * k + j];
-        const C p = cm(x, y);
-        s = C{s.re + p.re, s.im + p.im};
-      }
-      c[3 * i + j] = C{c[3 * i + j].re + s.re, c[3 * i + j].im + s.im};
-    }
+// Site order of the smearing kernels.  Lane j of the launch takes the sites of
+// one y slab after another, each slab swept along z in (t, x, y) order, and the
+// directions of a block of sites are the fastest block index: an XCD then
+// holds the planes z - 1, z, z + 1 of its slab and the links that the
+// directions share in its L2.  24^3x48, against site order with the directions
+// as separate passes and the same arithmetic (us a step): APE 322 -> 286,
+// stout 440 -> 415.  What bounds them now is traffic between L2 and the fabric
+// (1.6 GB read for 0.29 GB of spatial links an APE step) together with the
+// FP64 pipes, busy 42% of the time.  Tried and slower: rows of the products
+// formed one at a time (fewer registers, 3-4 wavefronts per SIMD), separate
+// loops over backward and forward stout staples (3 wavefronts).
+struct SlabOrder {
+  unsigned by;     // y rows per slab
+  unsigned full;   // sites of a full slab, T X by Z
+};
+__device__ __forceinline__ Site slab_site(unsigned j, const SlabOrder &o, const DslashArgs &a) {
+  const unsigned P = a.L[0] * a.L[1];
+  const unsigned k = j / o.full, y0 = k * o.by, ny = min(o.by, a.L[2] - y0);
+  unsigned r = j - k * o.full;
+  Site st;
+  st.z = r / (P * ny);
+  r -= st.z * P * ny;
+  const unsigned yy = r / P;
+  r -= yy * P;
+  st.y = y0 + yy;
+  st.x = r / a.L[0];
+  st.t = r - st.x * a.L[0];
+  st.s = r + P * (st.y + a.L[2] * st.z);
+  st.valid = true;
+  return st;
 }
 
 // One APE step for the spatial directions, one lane per (site, direction)
-// with the direction mu = 1 + blockIdx.y uniform over the workgroup, so the
-// staple loops do not diverge.  Each staple's three links are loaded as its
+// with the direction uniform over the workgroup, so the staple loops do not
+// diverge.  Each staple's three links are loaded as its
 // products need them, which bounds the live matrices to the staple sum and
 // two factors.  The temporal links are copied by the caller.
 __global__ void __launch_bounds__(kBlock) k_ape3d(DslashArgs a, GaugeIn<QCD_HIP_F64> U, double2 *__restrict__ out,
-                                                  size_t stride, double alpha) {
-  const unsigned s = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (s >= a.V) return;
-  const unsigned mu = 1 + blockIdx.y;
-  const Site st = site_coords(s, a);
+                                                  size_t stride, double alpha, SlabOrder ord) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const unsigned j = lb / 3 * kBlock + threadIdx.x, mu = 1 + lb % 3;   // mu is uniform over the workgroup
+  if (j >= a.V) return;
+  const Site st = slab_site(j, ord, a);
+  const unsigned s = st.s;
   C S[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) S[k] = C{0.0, 0.0};
@@ -247,7 +364,7 @@ __global__ void __launch_bounds__(kBlock) k_ape3d(DslashArgs a, GaugeIn<QCD_HIP_
     }
     C W[9];
     U.load(nu, sf, W);
-    mm3_add<false, true>(S, T, W);
+    mm3<false, true, true>(S, T, W);
   }
 #pragma unroll 1
   for (unsigned nu = 1; nu < 4; nu++) {
@@ -262,7 +379,7 @@ __global__ void __launch_bounds__(kBlock) k_ape3d(DslashArgs a, GaugeIn<QCD_HIP_
     }
     C A[9];
     U.load(nu, sn, A);
-    mm3_add<true, false>(S, A, T);
+    mm3<true, false, true>(S, A, T);
   }
   C m[9];
   U.load(mu, s, m);
@@ -277,16 +394,17 @@ __global__ void __launch_bounds__(kBlock) k_ape3d(DslashArgs a, GaugeIn<QCD_HIP_
 // One stout step (qcd_smearing.c:374-476), one lane per (site, direction):
 // C = sum over nu != mu (nu from START) of the backward staple then the
 // forward one, W = C U^+, A = W - W^+ minus tr(A)/3, Q = -i rho/2 A,
-// U' = exp(iQ) U.  The direction is START + blockIdx.y, uniform over the
-// workgroup; directions below START (the temporal one for 3d stout) are
+// U' = exp(iQ) U.  The direction is uniform over the workgroup; directions below START (the temporal one for 3d stout) are
 // copied by the caller.
 template <unsigned START>
 __global__ void __launch_bounds__(kBlock) k_stout(DslashArgs a, GaugeIn<QCD_HIP_F64> U, double2 *__restrict__ out,
-                                                  size_t stride, double rho) {
-  const unsigned s = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-  if (s >= a.V) return;
-  const unsigned mu = START + blockIdx.y;   // uniform over the workgroup
-  const Site st = site_coords(s, a);
+                                                  size_t stride, double rho, SlabOrder ord) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const unsigned j = lb / (4 - START) * kBlock + threadIdx.x;
+  const unsigned mu = START + lb % (4 - START);   // uniform over the workgroup
+  if (j >= a.V) return;
+  const Site st = slab_site(j, ord, a);
+  const unsigned s = st.s;
   C S[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) S[k] = C{0.0, 0.0};
@@ -306,7 +424,7 @@ __global__ void __launch_bounds__(kBlock) k_stout(DslashArgs a, GaugeIn<QCD_HIP_
       }
       C A[9];
       U.load(nu, sb, A);
-      mm3_add<true, false>(S, A, T);
+      mm3<true, false, true>(S, A, T);
     }
     // forward: [U_nu(x) U_mu(x+nu)] U_nu(x+mu)^+
     {
@@ -319,7 +437,7 @@ __global__ void __launch_bounds__(kBlock) k_stout(DslashArgs a, GaugeIn<QCD_HIP_
       }
       C W[9];
       U.load(nu, sf, W);
-      mm3_add<false, true>(S, T, W);
+      mm3<false, true, true>(S, T, W);
     }
   }
   C m[9], W[9];
@@ -342,30 +460,47 @@ __global__ void __launch_bounds__(kBlock) k_stout(DslashArgs a, GaugeIn<QCD_HIP_
   for (int k = 0; k < 9; k++) o[(size_t)k * kTile] = make_double2(W[k].re, W[k].im);
 }
 
-int stout_step(qcd_hip_field out, qcd_hip_field in, double rho, int ndim, hipStream_t st) {
+// One slab per XCD while its plane of links fits L2 (2.4 MB): 24^3x48 takes 3
+// rows (APE 10 steps 2.92 ms; 2 rows 3.01, 6 rows 3.08, site order 3.27),
+// 32^3x64 2 rows (2 steps 2.34 ms; 4 rows 2.41, site order 2.43), 48^3x96
+// single rows.
+static SlabOrder slab_order(qcd_hip_lattice lat) {
+  const unsigned Y = (unsigned)lat->L[2], row = (unsigned)lat->L[0] * (unsigned)lat->L[1];
+  const unsigned fit = std::max(1u, 2400000u / (row * 576u));
+  const unsigned by = std::min((Y + kNumXcd - 1) / kNumXcd, fit);
+  return SlabOrder{by, row * by * (unsigned)lat->L[3]};
+}
+
+// temporal links of in copied to out: direction 0 is the first 9 stride
+// links of the layout
+static int copy_temporal(qcd_hip_field out, qcd_hip_field in, hipStream_t st) {
+  QH_CHECK(hipMemcpyAsync(out->data, in->data, (size_t)9 * in->lat->stride * sizeof(double2),
+                          hipMemcpyDeviceToDevice, st));
+  return 0;
+}
+
+// keep: out holds the temporal links already (the second and later steps
+// that write one of the two ping-pong fields)
+int stout_step(qcd_hip_field out, qcd_hip_field in, double rho, int ndim, bool keep, hipStream_t st) {
   const DslashArgs a = make_args(in->lat, 0.0, 0.0);
   const int grid = grid_for(in->lat->V);
   if (ndim == 3) {
-    // temporal links copied: direction 0 is the first 9 stride links of the layout
-    QH_CHECK(hipMemcpyAsync(out->data, in->data, (size_t)9 * in->lat->stride * sizeof(double2),
-                            hipMemcpyDeviceToDevice, st));
-    k_stout<1><<<dim3(grid, 3), kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
-                                                 (size_t)in->lat->stride, rho);
+    if (!keep) QH_TRY(copy_temporal(out, in, st));
+    k_stout<1><<<3 * grid, kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
+                                                 (size_t)in->lat->stride, rho, slab_order(in->lat));
   } else {
-    k_stout<0><<<dim3(grid, 4), kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
-                                                 (size_t)in->lat->stride, rho);
+    k_stout<0><<<4 * grid, kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
+                                                 (size_t)in->lat->stride, rho, slab_order(in->lat));
   }
   QH_CHECK(hipGetLastError());
   return 0;
 }
 
-int ape_step(qcd_hip_field out, qcd_hip_field in, double alpha, hipStream_t st) {
+int ape_step(qcd_hip_field out, qcd_hip_field in, double alpha, bool keep, hipStream_t st) {
   const DslashArgs a = make_args(in->lat, 0.0, 0.0);
-  // temporal links: direction 0 is the first 9 stride links of the layout
-  QH_CHECK(hipMemcpyAsync(out->data, in->data, (size_t)9 * in->lat->stride * sizeof(double2),
-                          hipMemcpyDeviceToDevice, st));
-  k_ape3d<<<dim3(grid_for(in->lat->V), 3), kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
-                                                           (size_t)in->lat->stride, alpha);
+  if (!keep) QH_TRY(copy_temporal(out, in, st));
+  k_ape3d<<<3 * grid_for(in->lat->V), kBlock, 0, st>>>(a, GaugeIn<QCD_HIP_F64>::of(in), (double2 *)out->data,
+                                                           (size_t)in->lat->stride, alpha, slab_order(in->lat));
   QH_CHECK(hipGetLastError());
   return 0;
 }
@@ -427,13 +562,13 @@ int qcd_hip_ape_smear(qcd_hip_field out, qcd_hip_field in, double alpha, int nst
     return 0;
   }
   qcd_hip_field tmp = nullptr;
-  if (nsteps > 1) QH_TRY(qcd_hip_gauge_create(&tmp, in->lat, QCD_HIP_F64));
+  if (nsteps > 1) QH_TRY(gauge_create_unfilled(&tmp, in->lat));
   // ping-pong so that the last step writes out
   qcd_hip_field src = in;
   int rc = 0;
   for (int k = 0; k < nsteps && !rc; k++) {
     qcd_hip_field dst = ((nsteps - 1 - k) % 2 == 0) ? out : tmp;
-    rc = ape_step(dst, src, alpha, st);
+    rc = ape_step(dst, src, alpha, k >= 2, st);
     src = dst;
   }
   if (!rc && hipStreamSynchronize(st) != hipSuccess) {
@@ -469,12 +604,12 @@ int qcd_hip_stout_smear(qcd_hip_field out, qcd_hip_field in, double rho, int ndi
     return 0;
   }
   qcd_hip_field tmp = nullptr;
-  if (nsteps > 1) QH_TRY(qcd_hip_gauge_create(&tmp, in->lat, QCD_HIP_F64));
+  if (nsteps > 1) QH_TRY(gauge_create_unfilled(&tmp, in->lat));
   qcd_hip_field src = in;
   int rc = 0;
   for (int k = 0; k < nsteps && !rc; k++) {
     qcd_hip_field dst = ((nsteps - 1 - k) % 2 == 0) ? out : tmp;
-    rc = stout_step(dst, src, rho, ndim, st);
+    rc = stout_step(dst, src, rho, ndim, k >= 2, st);
     src = dst;
   }
   if (!rc && hipStreamSynchronize(st) != hipSuccess) {

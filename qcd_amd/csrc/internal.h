@@ -70,6 +70,7 @@ std::recursive_mutex &state_mutex();
 int ensure_init();
 int dev_alloc(void **p, size_t bytes);
 void dev_free(void *p, size_t bytes);
+int gauge_create_unfilled(qcd_hip_field *f, qcd_hip_lattice lat);
 // a library call wrote new links into gauge field f
 inline void gauge_written(qcd_hip_field f);
 

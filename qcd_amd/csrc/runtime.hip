@@ -379,7 +379,7 @@ void qcd_hip_lattice_destroy(qcd_hip_lattice lat) { delete lat; }
 long qcd_hip_lattice_volume(qcd_hip_lattice lat) { return lat ? lat->V : 0; }
 
 // ------------------------------------------------------------ fields
-static int field_alloc(qcd_hip_field *out, qcd_hip_lattice lat, int kind, int prec, int nrhs) {
+static int field_alloc(qcd_hip_field *out, qcd_hip_lattice lat, int kind, int prec, int nrhs, bool fill = true) {
   *out = nullptr;
   QH_TRY(ensure_init());
   if (!lat) {
@@ -409,6 +409,10 @@ static int field_alloc(qcd_hip_field *out, qcd_hip_lattice lat, int kind, int pr
   }
   f->norm = norm_bytes ? (float *)((char *)f->data + data_bytes) : nullptr;
   f->bytes = data_bytes + norm_bytes;
+  if (!fill) {
+    *out = f;
+    return 0;
+  }
   // complete before returning: the field may next be used on any stream, and
   // the null stream does not order against the library's non-blocking streams
   hipError_t e = hipMemsetAsync(f->data, 0, f->bytes, g_ctx.stream);
@@ -421,6 +425,16 @@ static int field_alloc(qcd_hip_field *out, qcd_hip_lattice lat, int kind, int pr
   *out = f;
   return 0;
 }
+
+}  // extern "C"
+
+// an FP64 gauge field with undefined contents, for work on the library stream
+// that writes every link before it reads one
+int qcdhip::gauge_create_unfilled(qcd_hip_field *f, qcd_hip_lattice lat) {
+  return field_alloc(f, lat, QCD_HIP_GAUGE, QCD_HIP_F64, 1, false);
+}
+
+extern "C" {
 
 int qcd_hip_spinor_create(qcd_hip_field *f, qcd_hip_lattice lat, int prec, int nrhs) {
   return field_alloc(f, lat, QCD_HIP_SPINOR, prec, nrhs);
