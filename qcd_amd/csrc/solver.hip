@@ -7,15 +7,17 @@
 // operator A = Q = i g5 D (as invert.c) or A = D.  For A = Q the system solved
 // is Q x = i g5 b, i.e. D x = b, so the residual is ||b - D x|| either way.
 //
-// GCR iteration k (w_k = A res_k, chi_k = w_k / |w_k|, unnormalised w kept):
-//   multi-dot:   d_j = <w_j, w_k>, j < k                    (reads k+1 vectors)
-//   scalars:     a[k][j] = -s_j d_j, coefficient -s_j^2 d_j  (1 workgroup)
-//   multi-axpy:  w_k += sum_j coef_j w_j, with |w_k|^2 and <w_k, src>
-//   scalars:     s_k = 1/|w_k|, c_k = s_k <w_k, src>, invert.c's recurrence
-//                a[k][j] <- a[k][j] a[j][j] + sum_{l=j+1}^{k-1} a[k][l] a[l][j]
-//   axpy:        res_{k+1} = res_k - c_k s_k w_k
-// After n iterations one multi-axpy forms x = sum_j beta_j res_j with
-// beta_j = sum_{k>=j} c_k a[k][j] (the reference updates x every iteration).
+// GCR iteration k (w_k = A res_k, made orthogonal to the earlier w_j and kept
+// unnormalised):
+//   k_gcr_dots:    d_j = <w_j, w_k>, j < k, |w_k|^2, <w_k, res_k>  (reads k+2
+//                  vectors)
+//   k_gcr_scal:    coef[k][j] and alpha[k] (few sums: formed by k_gcr_update)
+//   k_gcr_update:  w_k += sum_j coef[k][j] w_j, res_{k+1} = res_k + alpha[k] w_k
+//                  (reads k+2 vectors, writes 2; not needed in the last step).
+//                  Q in reduced precision: w_k, then alpha[k] from its own
+//                  sums, then res_{k+1}
+// After n iterations k_solution forms x = sum_j beta_j res_j, beta from coef and
+// alpha (the reference updates x every iteration).
 // All coefficients live in device memory: a cycle needs no host round trip.
 // Right-hand sides are solved in batches of prm.batch that advance in
 // lockstep: every kernel takes a second grid dimension over the batch, and
@@ -27,6 +29,7 @@
 
 #include <chrono>
 #include <cmath>
+#include <type_traits>
 
 namespace qcdhip {
 
@@ -43,13 +46,15 @@ qcd_hip_lattice eo_half_lattice(qcd_hip_lattice full);
 
 constexpr int kN = kMaxKrylov;
 
+// The coefficients of one right-hand side's GCR cycle.  w_k = A res_k +
+// sum_j coef[k][j] w_j, res_{k+1} = res_k + alpha[k] w_k.
 struct GcrScal {
-  double2 a[kN * kN];
-  double2 c[kN];
-  double s[kN];
-  double2 coef[kN];
-  double2 beta[kN];
-  double2 alpha;
+  double2 coef[kN * kN];   // [k][j], j < k
+  double2 alpha[kN];
+  double2 beta[kN];        // the cycle's solution is sum_j beta_j res_j
+  double w2inv[kN];        // 1 / |w_k|^2 of the stored w_k
+  double rmin[kN];         // smallest |res_i|^2, i <= k
+  int stop[kN];            // the cycle's steps from k on are left out
   double rnorm;
   double rscale;
   int bad;
@@ -59,168 +64,151 @@ __device__ __forceinline__ double2 cmul2(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// Sum nvals doubles over the workgroup; lane 0 of the group writes
-// out[v * nb + slot] for v < nvals.  All lanes must call it.
-template <int NV>
-__device__ __forceinline__ void group_sum(double (&v)[NV], double *out, unsigned nb, unsigned slot) {
-  __shared__ double sh[NV][kBlock / 64];
-#pragma unroll
-  for (int i = 0; i < NV; i++)
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v[i] += __shfl_xor(v[i], off, 64);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0)
-#pragma unroll
-    for (int i = 0; i < NV; i++) sh[i][wid] = v[i];
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    double t = 0.0;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; w++) t += sh[threadIdx.x][w];
-    out[(size_t)threadIdx.x * nb + slot] = t;
-  }
-  __syncthreads();
-}
-
 // Batched kernels: grid row y works on right-hand-side slot ids[y]; the
 // Krylov vector j of slot b is vector b*n + j of the Rs / Ws fields; row y
 // writes its partial sums at part + y*rowsz, laid out [value][workgroup].
 
-// d_j = <w_j, w_k> for j < k, in chunks of kDotChunk basis vectors: their
-// loads are in flight together and the workgroup reduces the chunk's sums
-// at once (each d_j is summed exactly as it would be alone)
-constexpr int kDotChunk = 4;
+// ------------------------------------------------------------ chunks
+// A vector is an array of 16-byte chunks: tile after tile, kG groups of 64
+// chunks each (SpinorIn::offset), kC complex components of one site per chunk.
+// A wavefront takes M consecutive groups, lane by lane, so each of its loads
+// is one contiguous 1 KB, and the kernels below see one array whatever the
+// layout.  M = kG is one site per lane.
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <int P>
-__global__ void __launch_bounds__(kBlock) k_multidot(SpinorSet<P> W, int n, int k, const int *ids, unsigned V,
-                                                     double *part, size_t rowsz) {
-  using R = typename Prec<P>::R;
-  const int b = ids[blockIdx.y];
-  double *pr = part + blockIdx.y * rowsz;
-  const unsigned s = blockIdx.x * kBlock + threadIdx.x;
-  const bool ok = s < V;
-  Cx<R> wk[12];
-  if (ok) W.load(b * n + k, s, wk);
-  for (int j0 = 0; j0 < k; j0 += kDotChunk) {
-    double v[2 * kDotChunk];
+struct Chunk {
+  using T = typename Prec<P>::T;
+  static constexpr int kG = 12 * (int)sizeof(T) / 16, kC = 16 / (int)sizeof(T);
+  static __device__ __forceinline__ u32x4 *at(const SpinorSet<P> &v, int j, unsigned q) {
+    return (u32x4 *)(v.base + (size_t)j * v.vstride) + q;
+  }
+  static __device__ __forceinline__ u32x4 load(const SpinorSet<P> &v, int j, unsigned q) {
+    return __builtin_nontemporal_load(at(v, j, q));
+  }
+  static __device__ __forceinline__ float norm(const SpinorSet<P> &v, int j, unsigned s) {
+    if constexpr (P == QCD_HIP_F16) return __builtin_nontemporal_load(&v.norm[(size_t)j * v.nstride + s]);
+    else return 1.0f;
+  }
+  // component i of a chunk as stored (FP16: without the site norm)
+  static __device__ __forceinline__ Cx<typename Prec<P>::R> get(u32x4 q, int i) {
+    using R = typename Prec<P>::R;
+    if constexpr (P == QCD_HIP_F64) {
+      const f64x2 d = __builtin_bit_cast(f64x2, q);
+      return Cx<R>{d.x, d.y};
+    } else if constexpr (P == QCD_HIP_F32) {
+      const f32x4 f = __builtin_bit_cast(f32x4, q);
+      return Cx<R>{f[2 * i], f[2 * i + 1]};
+    } else {
+      return to_cx<R>(as_half2(q[i]));
+    }
+  }
+  // sum over the chunk of conj(a) b, of stored values
+  static __device__ __forceinline__ void dot(u32x4 a, u32x4 b, double &re, double &im) {
 #pragma unroll
-    for (int i = 0; i < 2 * kDotChunk; i++) v[i] = 0.0;
-    if (ok) {
-#pragma unroll
-      for (int i = 0; i < kDotChunk; i++) {
-        if (j0 + i < k) {
-          Cx<R> wj[12];
-          W.load(b * n + j0 + i, s, wj);
-#pragma unroll
-          for (int c = 0; c < 12; c++) {
-            v[2 * i] += (double)wj[c].re * (double)wk[c].re + (double)wj[c].im * (double)wk[c].im;
-            v[2 * i + 1] += (double)wj[c].re * (double)wk[c].im - (double)wj[c].im * (double)wk[c].re;
-          }
-        }
+    for (int i = 0; i < kC; i++) {
+      const auto x = get(a, i), y = get(b, i);
+      if constexpr (P == QCD_HIP_F16) {
+        // a product of two half values is exact in FP32; one rounding per sum
+        re += (double)fmaf(x.im, y.im, x.re * y.re);
+        im += (double)fmaf(-x.im, y.re, x.re * y.im);
+      } else {
+        re = fma((double)x.re, (double)y.re, fma((double)x.im, (double)y.im, re));
+        im = fma((double)x.re, (double)y.im, fma(-(double)x.im, (double)y.re, im));
       }
     }
-    // sums of j >= k are written too (zeros) but never read
-    group_sum<2 * kDotChunk>(v, pr + (size_t)2 * j0 * gridDim.x, gridDim.x, blockIdx.x);
   }
-}
-
-// w_k += sum_j coef_j w_j; partials: |w_k|^2, Re/Im <w_k, src = res_0>
-template <int P>
-__global__ void __launch_bounds__(kBlock) k_multiaxpy_norm(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k,
-                                                           const GcrScal *sc, const int *ids, unsigned V, double *part,
-                                                           size_t rowsz) {
-  using R = typename Prec<P>::R;
-  const int b = ids[blockIdx.y];
-  __shared__ double2 cf[kN];
-  for (int j = threadIdx.x; j < k; j += kBlock) cf[j] = sc[b].coef[j];
-  __syncthreads();
-  const unsigned s = blockIdx.x * kBlock + threadIdx.x;
-  double v[3] = {0.0, 0.0, 0.0};
-  if (s < V) {
-    Cx<R> wk[12];
-    W.load(b * n + k, s, wk);
-    if (k > 0) {
-      Cx<double> acc[12];
+  // |a|^2 of stored values
+  static __device__ __forceinline__ void norm2(u32x4 a, double &re) {
 #pragma unroll
-      for (int c = 0; c < 12; c++) acc[c] = Cx<double>{(double)wk[c].re, (double)wk[c].im};
-#pragma unroll 4
-      for (int j = 0; j < k; j++) {
-        Cx<R> wj[12];
-        W.load(b * n + j, s, wj);
-        const double2 a = cf[j];
-#pragma unroll
-        for (int c = 0; c < 12; c++) {
-          acc[c].re += a.x * (double)wj[c].re - a.y * (double)wj[c].im;
-          acc[c].im += a.x * (double)wj[c].im + a.y * (double)wj[c].re;
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 12; c++) wk[c] = Cx<R>{(R)acc[c].re, (R)acc[c].im};
-      W.store_back(b * n + k, s, wk);   // the norms below are those of the stored (rounded) vector
-    }
-    Cx<R> sv[12];
-    Rs.load(b * n, s, sv);
-#pragma unroll
-    for (int c = 0; c < 12; c++) {
-      const double wr = wk[c].re, wi = wk[c].im;
-      v[0] += wr * wr + wi * wi;
-      v[1] += wr * (double)sv[c].re + wi * (double)sv[c].im;
-      v[2] += wr * (double)sv[c].im - wi * (double)sv[c].re;
+    for (int i = 0; i < kC; i++) {
+      const auto x = get(a, i);
+      if constexpr (P == QCD_HIP_F16) re += (double)fmaf(x.im, x.im, x.re * x.re);
+      else re = fma((double)x.re, (double)x.re, fma((double)x.im, (double)x.im, re));
     }
   }
-  group_sum<3>(v, part + blockIdx.y * rowsz, gridDim.x, blockIdx.x);
-}
-
-// res_{k+1} = res_k + alpha w_k
-template <int P>
-__global__ void __launch_bounds__(kBlock) k_res_update(SpinorSet<P> Rs, SpinorSet<P> W, int n, int k,
-                                                       const GcrScal *sc, const int *ids, unsigned V) {
-  using R = typename Prec<P>::R;
-  const int b = ids[blockIdx.y];
-  const unsigned s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= V) return;
-  const double2 al = sc[b].alpha;
-  Cx<R> r[12], w[12];
-  Rs.load(b * n + k, s, r);
-  W.load(b * n + k, s, w);
+  // acc += c a (FP16: c includes the site norm)
+  static __device__ __forceinline__ void axpy(Cx<double> acc[kC], double2 c, u32x4 a) {
 #pragma unroll
-  for (int c = 0; c < 12; c++) {
-    const double wr = w[c].re, wi = w[c].im;
-    r[c] = Cx<R>{(R)((double)r[c].re + al.x * wr - al.y * wi), (R)((double)r[c].im + al.x * wi + al.y * wr)};
-  }
-  Rs.store(b * n + k + 1, s, r);
-}
-
-// e_b = sum_j beta_j res_j, times |r_b| (the norm the inner source was
-// divided by) when scaled
-template <int P>
-__global__ void __launch_bounds__(kBlock) k_solution(SpinorSet<P> Rs, int n, const GcrScal *sc, SpinorSet<P> E,
-                                                     const int *ids, unsigned V, int scaled) {
-  using R = typename Prec<P>::R;
-  const int b = ids[blockIdx.y];
-  __shared__ double2 bt[kN];
-  const double f = scaled ? sc[b].rnorm : 1.0;
-  for (int j = threadIdx.x; j < n; j += kBlock) bt[j] = make_double2(sc[b].beta[j].x * f, sc[b].beta[j].y * f);
-  __syncthreads();
-  const unsigned s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= V) return;
-  Cx<double> acc[12];
-#pragma unroll
-  for (int c = 0; c < 12; c++) acc[c] = Cx<double>{0.0, 0.0};
-#pragma unroll 4
-  for (int j = 0; j < n; j++) {
-    Cx<R> r[12];
-    Rs.load(b * n + j, s, r);
-    const double2 bb = bt[j];
-#pragma unroll
-    for (int c = 0; c < 12; c++) {
-      acc[c].re += bb.x * (double)r[c].re - bb.y * (double)r[c].im;
-      acc[c].im += bb.x * (double)r[c].im + bb.y * (double)r[c].re;
+    for (int i = 0; i < kC; i++) {
+      const auto x = get(a, i);
+      acc[i].re = fma(c.x, (double)x.re, fma(-c.y, (double)x.im, acc[i].re));
+      acc[i].im = fma(c.x, (double)x.im, fma(c.y, (double)x.re, acc[i].im));
     }
   }
-  Cx<R> o[12];
+};
+
+// first group of this wavefront and its lane's site there
+template <int P, int M>
+struct ChunkLane {
+  unsigned q0, tile, lane;   // chunk of group 0, tile of the wavefront, lane
+  bool valid;
+  // T lanes per workgroup
+  static __device__ __forceinline__ ChunkLane of(unsigned V) {
+    constexpr unsigned kG = Chunk<P>::kG;
+    static_assert(kG % M == 0, "a wavefront stays in one tile");
+    ChunkLane l;
+    l.lane = threadIdx.x & 63u;
+    const unsigned u = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    l.tile = u / (kG / M);
+    l.q0 = u * (M * 64u) + l.lane;
+    l.valid = l.tile * 64u + l.lane < V;
+    return l;
+  }
+  __device__ __forceinline__ unsigned site() const { return tile * 64u + lane; }
+};
+
+// x of the lane that DPP control CTRL selects (within rows of 16 lanes)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+constexpr int kRowMirror = 0x140, kHalfMirror = 0x141, kQuadMirror = 0x1B, kQuadSwap = 0xB1;
+// Sums of a over lanes l and l ^ W where bit W of the lane is clear, of b
+// where it is set (W = 32 or 16): one swap of register halves (rows) and an
+// addition
+template <int W>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  auto swap = [](unsigned p, unsigned q) {
+    if constexpr (W == 32) return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    else return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+  };
+  const auto lo = swap((unsigned)x, (unsigned)y), hi = swap((unsigned)(x >> 32), (unsigned)(y >> 32));
+  return __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]) +
+         __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+}
+// the same across the mirrored half rows (W = 8) or quads (W = 4)
+template <int W>
+__device__ __forceinline__ double mirror_add(double a, double b) {
+  const bool up = (threadIdx.x & W) != 0;
+  const double keep = up ? b : a, send = up ? a : b;
+  return keep + dpp_move<W == 8 ? kRowMirror : kHalfMirror>(send);
+}
+
+// Sum NV (2, 4, 8 or 16) values over the wavefront; lane l returns value
+// l / (64 / NV).  Every exchange halves the values a lane keeps, by register
+// swaps between rows and DPP moves within them: 18 exchanges and additions
+// for 8 values, no LDS latency.
+template <int NV>
+__device__ __forceinline__ double wave_sum_scatter(double (&v)[NV]) {
+  constexpr int H = NV / 2;
 #pragma unroll
-  for (int c = 0; c < 12; c++) o[c] = Cx<R>{(R)acc[c].re, (R)acc[c].im};
-  E.store(b, s, o);
+  for (int i = 0; i < H; i++) v[i] = swap_add<32>(v[i], v[i + H]);
+  constexpr int Q = H > 1 ? H / 2 : 1;
+#pragma unroll
+  for (int i = 0; i < Q; i++) v[i] = swap_add<16>(v[i], H > 1 ? v[i + Q] : v[i]);
+  if constexpr (NV == 16) v[0] = mirror_add<8>(v[0], v[2]), v[1] = mirror_add<8>(v[1], v[3]);
+  else if constexpr (NV == 8) v[0] = mirror_add<8>(v[0], v[1]);
+  else v[0] += dpp_move<kRowMirror>(v[0]);
+  if constexpr (NV == 16) v[0] = mirror_add<4>(v[0], v[1]);
+  else v[0] += dpp_move<kHalfMirror>(v[0]);
+  v[0] += dpp_move<kQuadMirror>(v[0]);
+  v[0] += dpp_move<kQuadSwap>(v[0]);
+  return v[0];
 }
 
 // Sum a [nv][nb] partial array (one wave per value, an order fixed by nb)
@@ -247,80 +235,509 @@ __device__ void wave_sums(const double *part, int nv, unsigned nb, double *sums)
   }
 }
 
-// after the multi-dot of iteration k (one workgroup per slot)
-__global__ void __launch_bounds__(1024) k_scal_dots(GcrScal *scs, const double *part, size_t rowsz, unsigned nb, int k,
-                                                    int n, const int *ids) {
-  __shared__ double sums[2 * kN];
-  GcrScal *sc = scs + ids[blockIdx.x];
-  wave_sums(part + blockIdx.x * rowsz, 2 * k, nb, sums);
-  __syncthreads();
-  for (int j = threadIdx.x; j < k; j += blockDim.x) {
-    const double sj = sc->s[j];
-    const double2 d = make_double2(sums[2 * j], sums[2 * j + 1]);
-    sc->a[k * n + j] = make_double2(-sj * d.x, -sj * d.y);
-    sc->coef[j] = make_double2(-sj * sj * d.x, -sj * sj * d.y);
-  }
-}
-
-// after the multi-axpy of iteration k: normalisation, c_k and the
-// coefficient recurrence of invert.c:83-94
-// Row k is scaled by s_k first; then every a[k][j] is updated from the scaled
-// row and the finished rows l < k, so the j are independent: thread j does
-// one of them, with rows 0..k-1 staged in LDS (packed lower triangle).
-__global__ void __launch_bounds__(1024) k_scal_norm(GcrScal *scs, const double *part, size_t rowsz, unsigned nb, int k,
-                                                    int n, const int *ids) {
-  __shared__ double sums[3];
-  __shared__ double2 rowk[kN];
-  __shared__ double diag[kN];
-  __shared__ double2 tri[kN * (kN - 1) / 2];   // a[l][j], j < l < k, at l (l - 1) / 2 + j
-  GcrScal *sc = scs + ids[blockIdx.x];
-  wave_sums(part + blockIdx.x * rowsz, 3, nb, sums);
-  const int tid = threadIdx.x;
-  for (int base = 0; base < k; base += 1024 / 64) {
-    const int l = base + (tid >> 6), j = tid & 63;
-    if (l < k && j < l) tri[l * (l - 1) / 2 + j] = sc->a[l * n + j];
-  }
-  if (tid < k) diag[tid] = sc->a[tid * n + tid].x;
-  __syncthreads();
-  const double sk = 1.0 / sqrt(sums[0]);
-  if (tid < k) {
-    const double2 a = sc->a[k * n + tid];
-    rowk[tid] = make_double2(a.x * sk, a.y * sk);
-  }
-  __syncthreads();
-  if (tid < k) {
-    const int j = tid;
-    double2 t = rowk[j];
-    t = make_double2(t.x * diag[j], t.y * diag[j]);
-    for (int l = j + 1; l < k; l++) {
-      const double2 p = cmul2(rowk[l], tri[l * (l - 1) / 2 + j]);
-      t = make_double2(t.x + p.x, t.y + p.y);
+// sums[q] = sum over p < np of part[p nv + q], q < nv <= BLK, in an order fixed
+// by np and BLK: BLK / nv lanes per value, each over every (BLK / nv)th p, then
+// a tree over LDS.  The whole workgroup calls it; sums holds BLK values.
+template <int BLK>
+__device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsigned nv, double *sums) {
+  unsigned g = BLK / nv;
+  const unsigned t = threadIdx.x, p0 = t / nv, q = t - p0 * nv;
+  double x = 0.0;
+  if (p0 < g) {
+    const double *a = part + q;
+    unsigned p = p0;
+    for (; p + 7 * g < np; p += 8 * g) {
+      double y[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) y[i] = a[(size_t)(p + i * g) * nv];
+      x += ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
     }
-    sc->a[k * n + j] = t;
+    for (; p < np; p += g) x += a[(size_t)p * nv];
   }
-  if (tid == 0) {
-    if (!(sk == sk) || isinf(sk)) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
-    sc->s[k] = sk;
-    sc->a[k * n + k] = make_double2(sk, 0.0);
-    const double2 ck = make_double2(sk * sums[1], sk * sums[2]);
-    sc->c[k] = ck;
-    sc->alpha = make_double2(-ck.x * sk, -ck.y * sk);
+  sums[t] = x;
+  __syncthreads();
+  while (g > 1) {
+    const unsigned h = (g + 1) / 2;
+    if (p0 + h < g) sums[t] += sums[t + h * nv];
+    g = h;
+    __syncthreads();
   }
 }
 
-// beta_j = sum_{k >= j} c_k a[k][j]; keep_q1 drops the k = 0 term as
-// invert.c:50-53 does
-__global__ void k_scal_beta(GcrScal *scs, int n, int keep_q1, const int *ids) {
+// Smallest |w_k|^2 / |A res_k|^2 that the difference below can tell from
+// rounding of the stored vectors
+template <int P>
+constexpr double gcr_floor() { return P == QCD_HIP_F64 ? 1e-13 : P == QCD_HIP_F32 ? 1e-6 : 1e-4; }
+
+// sums of step k: d_j = <w_j, A res_k> for j < k (re, im), |A res_k|^2,
+// |res_k|^2, <A res_k, res_k> (re, im), |w_{k-1}|^2
+__host__ __device__ constexpr unsigned gcr_values(int k) { return 2 * (unsigned)k + 5; }
+
+// Coefficients of step k from its sums (first wavefront of a workgroup).  The
+// w_j are orthogonal to each other and to res_k, so with
+//   coef_j = -d_j / |w_j|^2,  w_k = A res_k + sum_j coef_j w_j
+// |w_k|^2 = |A res_k|^2 - sum_j |d_j|^2 / |w_j|^2 and <w_k, res_k> =
+// <A res_k, res_k>: the step length alpha = -<w_k, res_k> / |w_k|^2 is known
+// before w_k is formed, and w_k and res_{k+1} come out of one pass.  The
+// solution is formed from the same coef and alpha, so it matches res_{k+1}
+// whatever alpha is; rounding in alpha only makes the step a little shorter or
+// longer than the best one.  Where the difference cancels (A res_k in the span
+// of the w_j) it is bounded below, which shortens the step.  In reduced
+// precision the w_j of a long cycle lose their orthogonality and a step can
+// come out far too long (FP16, 64 steps on 270 sites): |res_k|^2 above four
+// times the smallest before it leaves that step and the rest of the cycle out
+// (alpha = 0).
+// cf[j] = coef_j, cf[k] = alpha, cf[k + 1].x = whether step k - 1 is left out;
+// store: write the results to sc as well.
+template <int P>
+__device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, double2 *cf, bool store) {
+  const int j = threadIdx.x;
+  const double *own = sums + 2 * k;
+  const double wl = own[4], wli = wl > 0.0 ? 1.0 / wl : 0.0, r2 = own[1];
+  const bool stop = k > 0 && (sc->stop[k - 1] || r2 > 4.0 * sc->rmin[k - 1]);
+  double e = 0.0;
+  if (j < k) {
+    const double w = j == k - 1 ? wli : sc->w2inv[j];
+    const double2 d = make_double2(sums[2 * j], sums[2 * j + 1]), c = make_double2(-w * d.x, -w * d.y);
+    cf[j] = c;
+    if (store) sc->coef[k * kN + j] = c;
+    e = (d.x * d.x + d.y * d.y) * w;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+  if (j == 0) {
+    const double n = own[0], t = fmax(n - e, gcr_floor<P>() * n), w = 1.0 / t;
+    const double2 al = stop ? make_double2(0.0, 0.0) : make_double2(-w * own[2], -w * own[3]);
+    cf[k] = al;
+    cf[k + 1] = make_double2(stop ? 1.0 : 0.0, 0.0);
+    if (store) {
+      // Krylov space is sick (invert.c:75-79)
+      if (!stop && (!(w == w) || isinf(w) || !(e == e))) sc->bad = 1;
+      if (k > 0) sc->w2inv[k - 1] = wli;
+      if (stop) sc->alpha[k - 1] = make_double2(0.0, 0.0);
+      sc->rmin[k] = k > 0 ? fmin(sc->rmin[k - 1], r2) : r2;
+      sc->stop[k] = stop;
+      sc->alpha[k] = al;
+    }
+  }
+}
+
+// Step k's sums (gcr_values) with the unorthogonalised w_k = A res_k, one partial
+// per value and workgroup, a workgroup's side by side.
+//
+// Streams k + 2 vectors, J of them in flight at a time (the last group reads
+// its last vector again where k is no multiple of J); PRE: the next group is
+// loaded before the present one is reduced, for launches with few wavefronts
+// per SIMD.  A wavefront adds its sums in its LDS row; the workgroup adds the
+// rows once.
+template <int P, int M, int J, int BLK>
+__global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, const int *ids,
+                                                  unsigned V, double *part, size_t rowsz) {
+  using CH = Chunk<P>;
+  constexpr int NW = BLK / 64, NV = 2 * J;
+  constexpr bool PRE = M == 1;
+  __shared__ double sums[NW][2 * kN + 8];
+  const int b = ids[blockIdx.y];
+  const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
+  const unsigned wid = threadIdx.x >> 6;
+  const int k0 = b * n;
+  struct Group {
+    u32x4 a[J][M];
+    float nj[J];
+  };
+  auto load = [&](Group &g, int j0) {
+    if (!l.valid) return;
+#pragma unroll
+    for (int i = 0; i < J; i++) {
+      const int j = k0 + min(j0 + i, k - 1);
+      g.nj[i] = CH::norm(W, j, l.site());
+#pragma unroll
+      for (int m = 0; m < M; m++) g.a[i][m] = CH::load(W, j, l.q0 + 64 * m);
+    }
+  };
+  u32x4 wk[M];
+  float nk = 0.f;
+  double last[2] = {0.0, 0.0};
+  Group next;
+  {
+    u32x4 r[M];
+    float nr = 0.f;
+    double own[4] = {0.0, 0.0, 0.0, 0.0};
+    if (l.valid) {
+      nk = CH::norm(W, k0 + k, l.site());
+      nr = CH::norm(Rs, k0 + k, l.site());
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        wk[m] = CH::load(W, k0 + k, l.q0 + 64 * m);
+        r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
+      }
+    }
+    if constexpr (PRE)
+      if (k > 0) load(next, 0);
+    if (l.valid) {
+      double re = 0.0, im = 0.0, n2 = 0.0, r2 = 0.0;
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        CH::norm2(wk[m], n2);
+        CH::dot(wk[m], r[m], re, im);
+        CH::norm2(r[m], r2);
+      }
+      if constexpr (P == QCD_HIP_F16) {
+        const double f = (double)nk * (double)nr;
+        re *= f;
+        im *= f;
+        n2 *= (double)nk * (double)nk;
+        r2 *= (double)nr * (double)nr;
+      }
+      own[0] = n2;
+      own[1] = r2;
+      own[2] = re;
+      own[3] = im;
+    }
+    const double t = wave_sum_scatter<4>(own);
+    if ((l.lane & 15u) == 0) sums[wid][2 * k + (l.lane >> 4)] = t;
+  }
+  for (int j0 = 0; j0 < k; j0 += J) {
+    Group g;
+    if constexpr (PRE) {
+      g = next;
+      if (j0 + J < k) load(next, j0 + J);
+    } else {
+      load(g, j0);
+    }
+    double v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = 0.0;
+    if (l.valid) {
+#pragma unroll
+      for (int i = 0; i < J; i++) {
+#pragma unroll
+        for (int m = 0; m < M; m++) CH::dot(g.a[i][m], wk[m], v[2 * i], v[2 * i + 1]);
+        if constexpr (P == QCD_HIP_F16) {
+          const double f = (double)g.nj[i] * (double)nk;
+          v[2 * i] *= f;
+          v[2 * i + 1] *= f;
+        }
+      }
+      if (j0 + J >= k) {   // the group's last vector is w_{k-1}
+        double n2 = 0.0;
+#pragma unroll
+        for (int m = 0; m < M; m++) CH::norm2(g.a[J - 1][m], n2);
+        if constexpr (P == QCD_HIP_F16) n2 *= (double)g.nj[J - 1] * (double)g.nj[J - 1];
+        last[0] = n2;
+      }
+    }
+    constexpr unsigned lanes = 64 / NV;   // lanes per value after the scatter
+    const double t = wave_sum_scatter<NV>(v);
+    const unsigned q = 2 * (unsigned)j0 + l.lane / lanes;
+    if (l.lane % lanes == 0 && q < 2 * (unsigned)k) sums[wid][q] = t;
+  }
+  {
+    const double t = wave_sum_scatter<2>(last);
+    if (l.lane == 0) sums[wid][2 * k + 4] = t;
+  }
+  __syncthreads();
+  const unsigned nv = gcr_values(k);
+  double *pr = part + blockIdx.y * rowsz + (size_t)blockIdx.x * nv;
+  for (unsigned q = threadIdx.x; q < nv; q += BLK) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) t += sums[w][q];
+    pr[q] = t;
+  }
+}
+
+// Step k's coefficients from the sums of k_gcr_dots (np workgroups), one
+// workgroup per rhs
+template <int P>
+__global__ void __launch_bounds__(1024) k_gcr_scal(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
+                                                   const int *ids) {
+  __shared__ double sums[1024];
+  __shared__ double2 cf[kN + 2];
+  sum_parts<1024>(part + blockIdx.x * rowsz, np, gcr_values(k), sums);
+  if (threadIdx.x < 64) gcr_coefficients<P>(scs + ids[blockIdx.x], sums, k, cf, true);
+}
+
+// Store M chunks of a vector of precision P given in FP64 and leave in q and
+// nrm what was stored.  FP16 takes the largest component of the site, which
+// lies in kG / M wavefronts of the workgroup (all of a site's wavefronts are in
+// one workgroup): mx holds one value per lane of the workgroup.
+template <int P, int M>
+__device__ __forceinline__ void chunk_store(const SpinorSet<P> &v, int j, const ChunkLane<P, M> &l,
+                                            const Cx<double> (&acc)[M][Chunk<P>::kC], u32x4 (&q)[M], float &nrm,
+                                            float *mx) {
+  using CH = Chunk<P>;
+  nrm = 1.0f;
+  if constexpr (P == QCD_HIP_F64) {
+#pragma unroll
+    for (int m = 0; m < M; m++) q[m] = __builtin_bit_cast(u32x4, f64x2{acc[m][0].re, acc[m][0].im});
+  } else if constexpr (P == QCD_HIP_F32) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+      q[m] = __builtin_bit_cast(u32x4, f32x4{(float)acc[m][0].re, (float)acc[m][0].im, (float)acc[m][1].re,
+                                             (float)acc[m][1].im});
+  } else {
+    float x = 0.f;
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int i = 0; i < CH::kC; i++) x = fmaxf(x, fmaxf(fabsf((float)acc[m][i].re), fabsf((float)acc[m][i].im)));
+    if constexpr (M != CH::kG) {
+      constexpr unsigned W = CH::kG / M;   // wavefronts per tile
+      const unsigned w0 = (threadIdx.x >> 6) / W * W;
+      __syncthreads();   // mx may still be read for the previous vector
+      mx[threadIdx.x] = x;
+      __syncthreads();
+#pragma unroll
+      for (unsigned i = 0; i < W; i++) x = fmaxf(x, mx[(w0 + i) * 64u + l.lane]);
+    }
+    // a site whose largest entry is below the smallest normal float is
+    // stored as zero: 1/x would overflow and 0 * inf give NaN
+    if (!(x >= FLT_MIN)) x = 0.f;
+    const float inv = x > 0.f ? 1.0f / x : 0.f;
+    nrm = x;
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int i = 0; i < CH::kC; i++)
+        q[m][i] = as_u32(__floats2half2_rn((float)acc[m][i].re * inv, (float)acc[m][i].im * inv));
+    const unsigned g0 = (l.q0 / 64u) % CH::kG;
+    if (l.valid && g0 == 0) __builtin_nontemporal_store(nrm, &v.norm[(size_t)j * v.nstride + l.site()]);
+  }
+  if (l.valid)
+#pragma unroll
+    for (int m = 0; m < M; m++) __builtin_nontemporal_store(q[m], CH::at(v, j, l.q0 + 64 * m));
+}
+
+// acc += sum of f[j] times vector j0 + j, j < cnt, J of them in flight (and
+// the next J on their way where a lane holds one chunk)
+template <int P, int M, int J>
+__device__ __forceinline__ void chunk_combine(Cx<double> (&acc)[M][Chunk<P>::kC], const SpinorSet<P> &v, int j0, int cnt,
+                                              const double2 *f, const ChunkLane<P, M> &l) {
+  using CH = Chunk<P>;
+  constexpr bool PRE = M == 1;
+  if (!l.valid) return;
+  struct Group {
+    u32x4 a[J][M];
+    float nj[J];
+  };
+  auto load = [&](Group &g, int i0) {
+#pragma unroll
+    for (int i = 0; i < J; i++) {
+      const int j = j0 + min(i0 + i, cnt - 1);
+      g.nj[i] = CH::norm(v, j, l.site());
+#pragma unroll
+      for (int m = 0; m < M; m++) g.a[i][m] = CH::load(v, j, l.q0 + 64 * m);
+    }
+  };
+  Group next;
+  if constexpr (PRE) load(next, 0);
+  for (int i0 = 0; i0 < cnt; i0 += J) {
+    Group g;
+    if constexpr (PRE) {
+      g = next;
+      if (i0 + J < cnt) load(next, i0 + J);
+    } else {
+      load(g, i0);
+    }
+#pragma unroll
+    for (int i = 0; i < J; i++) {
+      double2 c = f[min(i0 + i, cnt - 1)];
+      if (i0 + i >= cnt) c = make_double2(0.0, 0.0);
+      if constexpr (P == QCD_HIP_F16) c = make_double2(c.x * (double)g.nj[i], c.y * (double)g.nj[i]);
+#pragma unroll
+      for (int m = 0; m < M; m++) CH::axpy(acc[m], c, g.a[i][m]);
+    }
+  }
+}
+
+// w_k += sum_j coef_j w_j, then res_{k+1} = res_k + alpha w_k with the stored
+// (rounded) w_k: one pass over k + 2 vectors read and two written (k = 0: w_0
+// stays as it is).  np > 0: the step's coefficients are formed here from the
+// partial sums of np workgroups of k_gcr_dots, by every workgroup for itself in
+// the same order, and stored by the first; np = 0: k_gcr_scal has formed them.
+//
+// EXACT: w_k only, with partial sums of |w_k|^2 and <w_k, res_k> at part;
+// k_gcr_alpha and k_gcr_residual follow.  For Q in reduced precision: Q is
+// indefinite, <Q r, r> of a generic r is about |Q r| |r| / sqrt(12 V), so every
+// other step is nearly empty and the next one has |w_k|^2 of 1e-5 |Q res_k|^2
+// and less, which the difference that gcr_coefficients takes cannot give to
+// FP16 or FP32 (stagnates on 8^3x16).  D and the Schur complement have positive
+// real parts: iteration counts there equal those of the exact steps (8^3x16 and
+// 16^3x32 at kappa 0.135 and 0.139, eps 0.3, GCR(12), (32), (64)).
+template <int P, int M, int J, int BLK, bool EXACT>
+__global__ void __launch_bounds__(BLK) k_gcr_update(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, GcrScal *scs,
+                                                    const int *ids, unsigned V, double *part, size_t rowsz,
+                                                    unsigned np) {
+  using CH = Chunk<P>;
+  __shared__ double2 cf[kN + 2];
+  __shared__ double sums[BLK];
+  __shared__ float mx[P == QCD_HIP_F16 && M != CH::kG ? BLK : 1];
+  const int b = ids[blockIdx.y], k0 = b * n;
+  GcrScal *sc = scs + b;
+  if (np > 0) {
+    sum_parts<BLK>(part + blockIdx.y * rowsz, np, gcr_values(k), sums);
+    if (threadIdx.x < 64) gcr_coefficients<P>(sc, sums, k, cf, blockIdx.x == 0);
+  } else {
+    for (int j = threadIdx.x; j <= k; j += BLK) cf[j] = j < k ? sc->coef[k * kN + j] : sc->alpha[k];
+  }
+  __syncthreads();
+  double2 al = cf[k];
+  const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
+  u32x4 w[M], r[M];
+  float nw = 0.f, nr = 0.f;
+#pragma unroll
+  for (int m = 0; m < M; m++) w[m] = r[m] = u32x4{0, 0, 0, 0};
+  if (l.valid) {
+    nw = CH::norm(W, k0 + k, l.site());
+    nr = CH::norm(Rs, k0 + k, l.site());
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      w[m] = CH::load(W, k0 + k, l.q0 + 64 * m);
+      r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
+    }
+  }
+  Cx<double> acc[M][CH::kC];
+  auto start = [&](const u32x4 (&q)[M], float nq) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int i = 0; i < CH::kC; i++) {
+        const auto x = CH::get(q[m], i);
+        acc[m][i] = Cx<double>{(double)x.re, (double)x.im};
+        if constexpr (P == QCD_HIP_F16) {
+          acc[m][i].re *= (double)nq;
+          acc[m][i].im *= (double)nq;
+        }
+      }
+  };
+  if (k > 0) {
+    start(w, nw);
+    chunk_combine<P, M, J>(acc, W, k0, k, cf, l);
+    chunk_store<P, M>(W, k0 + k, l, acc, w, nw, mx);
+  }
+  if constexpr (EXACT) {
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      CH::norm2(w[m], v[0]);
+      CH::dot(w[m], r[m], v[1], v[2]);
+    }
+    if constexpr (P == QCD_HIP_F16) {
+      v[0] *= (double)nw * (double)nw;
+      v[1] *= (double)nw * (double)nr;
+      v[2] *= (double)nw * (double)nr;
+    }
+    const double t = wave_sum_scatter<4>(v);
+    __syncthreads();   // sums may still be read for the coefficients
+    if ((l.lane & 15u) == 0) sums[(threadIdx.x >> 6) * 4 + (l.lane >> 4)] = t;
+    __syncthreads();
+    if (threadIdx.x < 3) {
+      double x = 0.0;
+      for (int q = 0; q < BLK / 64; q++) x += sums[4 * q + threadIdx.x];
+      part[blockIdx.y * rowsz + (size_t)blockIdx.x * 3 + threadIdx.x] = x;
+    }
+    return;
+  }
+  start(r, nr);
+  if constexpr (P == QCD_HIP_F16) al = make_double2(al.x * (double)nw, al.y * (double)nw);
+#pragma unroll
+  for (int m = 0; m < M; m++) CH::axpy(acc[m], al, w[m]);
+  chunk_store<P, M>(Rs, k0 + k + 1, l, acc, r, nr, mx);
+}
+
+// alpha of step k from the sums of k_gcr_update<EXACT> (np workgroups)
+__global__ void __launch_bounds__(1024) k_gcr_alpha(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
+                                                    const int *ids) {
+  __shared__ double sums[1024];
+  sum_parts<1024>(part + blockIdx.x * rowsz, np, 3, sums);
+  if (threadIdx.x == 0) {
+    GcrScal *sc = scs + ids[blockIdx.x];
+    const double w = 1.0 / sums[0];
+    if (!(w == w) || isinf(w)) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
+    sc->alpha[k] = make_double2(-w * sums[1], -w * sums[2]);
+  }
+}
+
+// res_{k+1} = res_k + alpha w_k
+template <int P, int M, int BLK>
+__global__ void __launch_bounds__(BLK) k_gcr_residual(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, const GcrScal *scs,
+                                                      const int *ids, unsigned V) {
+  using CH = Chunk<P>;
+  __shared__ double2 f[2];
+  __shared__ float mx[P == QCD_HIP_F16 && M != CH::kG ? BLK : 1];
+  const int b = ids[blockIdx.y], k0 = b * n;
+  if (threadIdx.x == 0) {
+    f[0] = make_double2(1.0, 0.0);
+    f[1] = scs[b].alpha[k];
+  }
+  __syncthreads();
+  const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
+  Cx<double> acc[M][CH::kC];
+#pragma unroll
+  for (int m = 0; m < M; m++)
+#pragma unroll
+    for (int i = 0; i < CH::kC; i++) acc[m][i] = Cx<double>{0.0, 0.0};
+  chunk_combine<P, M, 1>(acc, Rs, k0 + k, 1, f, l);
+  chunk_combine<P, M, 1>(acc, W, k0 + k, 1, f + 1, l);
+  u32x4 q[M];
+  float nrm;
+  chunk_store<P, M>(Rs, k0 + k + 1, l, acc, q, nrm, mx);
+}
+
+// e_b = sum_j beta_j res_j, times |r_b| (the norm the inner source was
+// divided by) when scaled
+template <int P, int M, int J, int BLK>
+__global__ void __launch_bounds__(BLK) k_solution(SpinorSet<P> Rs, int n, const GcrScal *sc, SpinorSet<P> E,
+                                                  const int *ids, unsigned V, int scaled) {
+  using CH = Chunk<P>;
+  __shared__ double2 bt[kN];
+  __shared__ float mx[P == QCD_HIP_F16 && M != CH::kG ? BLK : 1];
+  const int b = ids[blockIdx.y];
+  const double f = scaled ? sc[b].rnorm : 1.0;
+  for (int j = threadIdx.x; j < n; j += BLK) bt[j] = make_double2(sc[b].beta[j].x * f, sc[b].beta[j].y * f);
+  __syncthreads();
+  const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
+  Cx<double> acc[M][CH::kC];
+#pragma unroll
+  for (int m = 0; m < M; m++)
+#pragma unroll
+    for (int i = 0; i < CH::kC; i++) acc[m][i] = Cx<double>{0.0, 0.0};
+  chunk_combine<P, M, J>(acc, Rs, b * n, n, bt, l);
+  u32x4 q[M];
+  float nrm;
+  chunk_store<P, M>(E, b, l, acc, q, nrm, mx);
+}
+
+// The cycle's solution sum_k (-alpha_k) p_k with p_k = res_k + sum_j coef[k][j]
+// p_j (A p_k = w_k) as sum_j beta_j res_j: beta_j = -alpha_j + sum_{k > j}
+// beta_k coef[k][j], from the last step down (lane j holds beta_j).  keep_q1
+// drops the first step's -alpha_0 as invert.c:50-53 does.
+// np > 0: the last step's coefficients are formed here first.
+template <int P>
+__global__ void __launch_bounds__(256) k_scal_beta(GcrScal *scs, int n, int keep_q1, const int *ids,
+                                                   const double *part, size_t rowsz, unsigned np) {
+  __shared__ double sums[256];
+  __shared__ double2 cf[kN + 2];
   GcrScal *sc = scs + ids[blockIdx.x];
   const int j = threadIdx.x;
-  if (j >= n) return;
+  if (np > 0) sum_parts<256>(part + blockIdx.x * rowsz, np, gcr_values(n - 1), sums);
+  if (j >= 64) return;
+  if (np > 0) gcr_coefficients<P>(sc, sums, n - 1, cf, true);
+  // (the last step's coefficients may just have been stored by other lanes)
+  auto coef = [&](int k) { return np > 0 && k == n - 1 ? cf[j] : sc->coef[k * kN + j]; };
   double2 b = make_double2(0.0, 0.0);
-  for (int k = j; k < n; k++) {
-    if (k == 0 && keep_q1) continue;
-    const double2 p = cmul2(sc->c[k], sc->a[k * n + j]);
-    b = make_double2(b.x + p.x, b.y + p.y);
+  if (j < n && !(j == 0 && keep_q1)) {
+    const double2 al = np > 0 && j == n - 1 ? cf[j] : sc->alpha[j];
+    if (!(np > 0 && j == n - 2 && cf[n].x != 0.0)) b = make_double2(-al.x, -al.y);
   }
-  sc->beta[j] = b;
+#pragma unroll 8
+  for (int k = n - 1; k > 0; k--) {
+    const double2 c = j < k ? coef(k) : make_double2(0.0, 0.0);
+    const double2 p = cmul2(make_double2(__shfl(b.x, k, 64), __shfl(b.y, k, 64)), c);
+    if (j < k) b = make_double2(b.x + p.x, b.y + p.y);
+  }
+  if (j < n) sc->beta[j] = b;
 }
 
 // outer residual norms from the Dslash partials (row x of the launch)
@@ -447,14 +864,91 @@ struct qcd_hip_solver_s {
 
 namespace {
 
+// Work split of the GCR vector kernels: M chunks per lane, J vectors in flight,
+// BLK lanes per workgroup.  Chosen by the vector length alone, so that a
+// right-hand side gets the same sums alone and in any batch.
+//   Short vectors: one chunk per lane, so that they still put a few wavefronts
+//     on every SIMD (FP16: a tile's three wavefronts share a workgroup, which
+//     finds the site norms).  Solves of 8^3x16, GCR(12), ms, Short against
+//     long: FP64 2.33 / 2.60, FP32 of 3 rhs 2.32 / 2.50, FP16 1.76 / 2.00 and
+//     of 12 rhs 2.66 / 2.62; FP64 without even-odd, GCR(32) 17.1 / 23.2.  From
+//     8000 sites up a batch of 12 FP16 rhs loses 16% with it, 3 FP32 rhs
+//     nothing, one rhs gains up to 11%.
+//   Long ones: a site (FP16, FP64) or half a site (FP32) per lane in the dots,
+//     fewer in the update, whose accumulators are FP64.  J = 2 FP16 vectors in
+//     flight in the update measured 1.5% of a 24^3x48 solve better than 4 (3
+//     wavefronts per SIMD) and 14% better than 4 held to 128 registers.  They
+//     run at 6.0-6.7 TB/s (24^3x48, 12 FP16 rhs; 16^3x32, one FP64 rhs), the
+//     rate of the fabric: running the update through the sites backwards, which
+//     would find the dots' last vectors in the last-level cache, changes nothing.
+template <int M_, int J_, int BLK_>
+struct GcrShape {
+  static constexpr int M = M_, J = J_, BLK = BLK_;
+};
+template <int P>
+struct GcrShapes;
+template <>
+struct GcrShapes<QCD_HIP_F16> {
+  using Short = GcrShape<1, 8, 192>;
+  using Dots = GcrShape<3, 4, 512>;
+  using Update = GcrShape<3, 2, 256>;
+};
+template <>
+struct GcrShapes<QCD_HIP_F32> {
+  using Short = GcrShape<1, 8, 256>;
+  using Dots = GcrShape<3, 4, 512>;
+  using Update = GcrShape<3, 4, 256>;
+};
+template <>
+struct GcrShapes<QCD_HIP_F64> {
+  using Short = GcrShape<1, 8, 256>;
+  using Dots = GcrShape<12, 1, 256>;
+  using Update = GcrShape<4, 4, 256>;
+};
+// Up to this many workgroups per rhs the update forms the coefficients from the
+// partial sums itself (8^3x16: 64 of them); past it every one of its workgroups
+// would read too many (12 FP16 rhs of 12^3x24, 324 of them: solve 9.6 ms with
+// k_gcr_scal, 10.2 without).
+constexpr unsigned kGcrParts = 128;
+template <typename SH>
+unsigned gcr_blocks(int prec, long V) {
+  const long kG = 12 * (long)spinor_comp_bytes(prec) / 16;
+  const long waves = (V + kTile - 1) / kTile * (kG / SH::M);
+  return (unsigned)((waves + SH::BLK / 64 - 1) / (SH::BLK / 64));
+}
+template <int P>
+constexpr bool gcr_short(long V) { return V <= (P == QCD_HIP_F16 ? 4096 : 8192); }
+// workgroups per rhs of the dots over vectors of V sites
+template <int P>
+unsigned gcr_parts_of(long V) {
+  using G = GcrShapes<P>;
+  return gcr_short<P>(V) ? gcr_blocks<typename G::Short>(P, V) : gcr_blocks<typename G::Dots>(P, V);
+}
+unsigned gcr_parts(int prec, long V) {
+  return prec == QCD_HIP_F64 ? gcr_parts_of<QCD_HIP_F64>(V)
+                             : prec == QCD_HIP_F32 ? gcr_parts_of<QCD_HIP_F32>(V) : gcr_parts_of<QCD_HIP_F16>(V);
+}
+// f(shape, grid) of a launch over count vectors of V sites (DOTS: the dots'
+// shape, else that of the kernels without sums)
+template <int P, bool DOTS, typename F>
+void gcr_launch(long V, int count, F f) {
+  using G = GcrShapes<P>;
+  auto call = [&](auto sh) { f(sh, dim3(gcr_blocks<decltype(sh)>(P, V), (unsigned)count)); };
+  if (gcr_short<P>(V)) call(typename G::Short{});
+  else if constexpr (DOTS) call(typename G::Dots{});
+  else call(typename G::Update{});
+}
+
 template <int P>
 int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream_t st) {
   const int n = S->prm.n_restart;
-  const unsigned V = S->Vi, nb = S->nbi;
+  const unsigned V = S->Vi;
   const int epi = S->use_q ? EPI_Q : EPI_D;
   const double m = 1.0 / (2.0 * kappa) - 4.0;
   SpinorSet<P> Rs = SpinorSet<P>::of(S->Rs), Ws = SpinorSet<P>::of(S->Ws), E = SpinorSet<P>::of(S->E);
-  const dim3 g2(nb, (unsigned)count);
+  // coefficients formed by the update kernel itself where the sums are few
+  const bool exact = P != QCD_HIP_F64 && S->use_q;
+  const unsigned np = !exact && gcr_parts(P, V) <= kGcrParts ? gcr_parts(P, V) : 0;
   for (int k = 0; k < n; k++) {
     if (S->prm.eo) {
       // w_k = D^ res_k = M res_k - H_oe (M^-1 H_eo res_k)
@@ -466,19 +960,36 @@ int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream
       QH_TRY(dslash_launch_batch(epi, false, S->Ws, k, n, S->Rs, k, n, S->gin, nullptr, 0, 0, S->ids, count, m, mu,
                                  nullptr, st, nullptr));
     }
-    if (k > 0) {
-      k_multidot<P><<<g2, kBlock, 0, st>>>(Ws, n, k, S->ids, V, S->part, S->rowsz);
-      k_scal_dots<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, nb, k, n, S->ids);
-    }
-    k_multiaxpy_norm<P><<<g2, kBlock, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V, S->part, S->rowsz);
-    k_scal_norm<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, nb, k, n, S->ids);
-    if (k + 1 < n) k_res_update<P><<<g2, kBlock, 0, st>>>(Rs, Ws, n, k, S->sc, S->ids, V);
+    gcr_launch<P, true>(V, count, [&](auto sh, dim3 grid) {
+      using SH = decltype(sh);
+      k_gcr_dots<P, SH::M, SH::J, SH::BLK><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->ids, V, S->part, S->rowsz);
+      if (!np) k_gcr_scal<P><<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
+    });
+    if (exact)
+      gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+        using SH = decltype(sh);
+        if constexpr (P != QCD_HIP_F64) {
+          k_gcr_update<P, SH::M, SH::J, SH::BLK, true><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V,
+                                                                                 S->part, S->rowsz, 0);
+          k_gcr_alpha<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
+          if (k + 1 < n) k_gcr_residual<P, SH::M, SH::BLK><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V);
+        }
+      });
+    else if (k + 1 < n)   // the last w_k and the residual after it are not used
+      gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+        using SH = decltype(sh);
+        k_gcr_update<P, SH::M, SH::J, SH::BLK, false><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V, S->part,
+                                                                                S->rowsz, np);
+      });
   }
-  k_scal_beta<<<count, kN, 0, st>>>(S->sc, n, S->prm.keep_q1, S->ids);
+  k_scal_beta<P><<<count, 256, 0, st>>>(S->sc, n, S->prm.keep_q1, S->ids, S->part, S->rowsz, np);
   // mixed even-odd solves take the correction scaled by |r^_o| (the outer
   // step adds it as it is); the others scale it where they add it
   const int scaled = S->prm.eo && S->prm.inner_prec != QCD_HIP_F64;
-  k_solution<P><<<g2, kBlock, 0, st>>>(Rs, n, S->sc, E, S->ids, V, scaled);
+  gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+    using SH = decltype(sh);
+    k_solution<P, SH::M, SH::J, SH::BLK><<<grid, SH::BLK, 0, st>>>(Rs, n, S->sc, E, S->ids, V, scaled);
+  });
   QH_CHECK(hipGetLastError());
   return 0;
 }
@@ -617,7 +1128,6 @@ int solve_batch(qcd_hip_solver_s *S, qcd_hip_field x, qcd_hip_field b, int x0, i
   QH_TRY(true_residual(S, x, x0, cnt, kappa, mu, st));
   std::vector<double> bnorm(cnt), rel(cnt);
   std::vector<int> outer(cnt, 0);
-  std::vector<GcrScal> host_sc;
   for (int i = 0; i < cnt; i++) {
     bnorm[i] = S->rn_host[i];
     rel[i] = bnorm[i] > 0.0 ? 1.0 : 0.0;
@@ -677,6 +1187,16 @@ void qcd_hip_solver_default_params(qcd_hip_solver_params *p) {
 }  // extern "C"
 
 namespace qcdhip {
+// Partial sums of one batch row: the dots of the last GCR step, or one sum per Dslash or hop workgroup (at most one per 256
+// sites, and the z-march grids).
+static size_t solver_row(qcd_hip_lattice lat, long Vi, const qcd_hip_solver_params *prm) {
+  const size_t parts = gcr_parts(prm->inner_prec, Vi);
+  // (k_gcr_update<EXACT> has three values per workgroup and at most six times
+  // the dots' workgroups)
+  const size_t dots = std::max((size_t)gcr_values(prm->n_restart - 1), (size_t)18) * parts;
+  return std::max(dots, std::max((size_t)grid_for(lat->V) + 64, (size_t)dslash_grid_bound(lat)));
+}
+
 // Device bytes qcd_hip_solver_create and qcd_hip_solver_set_gauge allocate
 // for a lattice of extents L with parameters prm: the same field shapes and
 // reduction rows, without allocating anything.
@@ -698,9 +1218,7 @@ size_t solver_device_bytes(const int L[4], const qcd_hip_solver_params *prm) {
   const bool split = prm->eo && ip == QCD_HIP_F16;                     // no r64 (split residual)
   b += (split ? 1 : 2) * field(lat.stride, QCD_HIP_F64, B);            // r64, bq
   b += sizeof(GcrScal) * B + sizeof(double) * B + sizeof(int) * B;      // sc, rn, ids
-  const size_t nb = (size_t)grid_for(V);
-  const size_t rowmax = ((size_t)2 * (n + kDotChunk) + 4) * (nb + 64);
-  b += sizeof(double) * std::max(rowmax, (size_t)dslash_grid_bound(&lat)) * B;   // partials
+  b += sizeof(double) * solver_row(&lat, Vi, prm) * B;                 // partials
   if (ip != QCD_HIP_F64) b += (size_t)36 * lat.stride * spinor_comp_bytes(ip);   // inner-precision links
   if (ip == QCD_HIP_F16) b += (size_t)8 * 36 * lat.V;                            // matrix-core hop links
   return b;
@@ -759,12 +1277,7 @@ int qcd_hip_solver_create(qcd_hip_solver *out, qcd_hip_lattice lat, const qcd_hi
   if (!rc) rc = dev_alloc((void **)&S->ids, sizeof(int) * B);
   if (!rc && hipHostMalloc((void **)&S->rn_host, sizeof(double) * B, hipHostMallocDefault) != hipSuccess) rc = 4;
   if (!rc && hipHostMalloc((void **)&S->ids_host, sizeof(int) * B, hipHostMallocDefault) != hipSuccess) rc = 4;
-  // per batch row: 2(n-1) multi-dot sums per site workgroup, or one sum per
-  // Dslash workgroup (a z-march grid never exceeds site workgroups + T*Z)
-  // (the multi-dot writes whole chunks: up to 2 (n + kDotChunk) sums)
-  const size_t rowmax = ((size_t)2 * (n + kDotChunk) + 4) * ((size_t)S->nb + 64);
-  const size_t dsl = (size_t)dslash_grid_bound(lat);
-  S->rowsz = std::max(rowmax, dsl);
+  S->rowsz = solver_row(lat, (long)S->Vi, prm);
   S->part_bytes = sizeof(double) * S->rowsz * B;
   if (!rc) rc = dev_alloc((void **)&S->part, S->part_bytes);
   if (rc) {
