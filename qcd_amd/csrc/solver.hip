@@ -245,14 +245,14 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
   double x = 0.0;
   if (p0 < g) {
     const double *a = part + q;
-    unsigned p = p0;
-    for (; p + 7 * g < np; p += 8 * g) {
+    for (unsigned p = p0; p < np; p += 8 * g) {   // eight loads in flight, the last ones too
       double y[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) y[i] = a[(size_t)(p + i * g) * nv];
+      for (int i = 0; i < 8; i++) y[i] = a[(size_t)min(p + i * g, np - 1) * nv];
+#pragma unroll
+      for (int i = 0; i < 8; i++) y[i] = p + i * g < np ? y[i] : 0.0;
       x += ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
     }
-    for (; p < np; p += g) x += a[(size_t)p * nv];
   }
   sums[t] = x;
   __syncthreads();
@@ -288,13 +288,14 @@ __host__ __device__ constexpr unsigned gcr_values(int k) { return 2 * (unsigned)
 // times the smallest before it leaves that step and the rest of the cycle out
 // (alpha = 0).
 // cf[j] = coef_j, cf[k] = alpha, cf[k + 1].x = whether step k - 1 is left out;
-// store: write the results to sc as well.
-template <int P>
+// store: write the results to sc as well.  EXACT (k_gcr_update): the coef_j
+// alone.
+template <int P, bool EXACT>
 __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, double2 *cf, bool store) {
   const int j = threadIdx.x;
   const double *own = sums + 2 * k;
   const double wl = own[4], wli = wl > 0.0 ? 1.0 / wl : 0.0, r2 = own[1];
-  const bool stop = k > 0 && (sc->stop[k - 1] || r2 > 4.0 * sc->rmin[k - 1]);
+  const bool stop = !EXACT && k > 0 && (sc->stop[k - 1] || r2 > 4.0 * sc->rmin[k - 1]);
   double e = 0.0;
   if (j < k) {
     const double w = j == k - 1 ? wli : sc->w2inv[j];
@@ -302,6 +303,10 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
     cf[j] = c;
     if (store) sc->coef[k * kN + j] = c;
     e = (d.x * d.x + d.y * d.y) * w;
+  }
+  if constexpr (EXACT) {
+    if (j == 0) sc->w2inv[k - 1] = wli;
+    return;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
@@ -329,8 +334,9 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
 // its last vector again where k is no multiple of J); PRE: the next group is
 // loaded before the present one is reduced, for launches with few wavefronts
 // per SIMD.  A wavefront adds its sums in its LDS row; the workgroup adds the
-// rows once.
-template <int P, int M, int J, int BLK>
+// rows once.  EXACT (as k_gcr_update): only the d_j and |w_{k-1}|^2 are used,
+// and res_k is not read.
+template <int P, int M, int J, int BLK, bool EXACT>
 __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, const int *ids,
                                                   unsigned V, double *part, size_t rowsz) {
   using CH = Chunk<P>;
@@ -365,16 +371,16 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
     double own[4] = {0.0, 0.0, 0.0, 0.0};
     if (l.valid) {
       nk = CH::norm(W, k0 + k, l.site());
-      nr = CH::norm(Rs, k0 + k, l.site());
+      if constexpr (!EXACT) nr = CH::norm(Rs, k0 + k, l.site());
 #pragma unroll
       for (int m = 0; m < M; m++) {
         wk[m] = CH::load(W, k0 + k, l.q0 + 64 * m);
-        r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
+        if constexpr (!EXACT) r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
       }
     }
     if constexpr (PRE)
       if (k > 0) load(next, 0);
-    if (l.valid) {
+    if (!EXACT && l.valid) {
       double re = 0.0, im = 0.0, n2 = 0.0, r2 = 0.0;
 #pragma unroll
       for (int m = 0; m < M; m++) {
@@ -394,7 +400,7 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
       own[2] = re;
       own[3] = im;
     }
-    const double t = wave_sum_scatter<4>(own);
+    const double t = EXACT ? 0.0 : wave_sum_scatter<4>(own);
     if ((l.lane & 15u) == 0) sums[wid][2 * k + (l.lane >> 4)] = t;
   }
   for (int j0 = 0; j0 < k; j0 += J) {
@@ -449,13 +455,13 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
 
 // Step k's coefficients from the sums of k_gcr_dots (np workgroups), one
 // workgroup per rhs
-template <int P>
+template <int P, bool EXACT>
 __global__ void __launch_bounds__(1024) k_gcr_scal(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
                                                    const int *ids) {
   __shared__ double sums[1024];
   __shared__ double2 cf[kN + 2];
   sum_parts<1024>(part + blockIdx.x * rowsz, np, gcr_values(k), sums);
-  if (threadIdx.x < 64) gcr_coefficients<P>(scs + ids[blockIdx.x], sums, k, cf, true);
+  if (threadIdx.x < 64) gcr_coefficients<P, EXACT>(scs + ids[blockIdx.x], sums, k, cf, true);
 }
 
 // Store M chunks of a vector of precision P given in FP64 and leave in q and
@@ -577,7 +583,7 @@ __global__ void __launch_bounds__(BLK) k_gcr_update(SpinorSet<P> W, SpinorSet<P>
   GcrScal *sc = scs + b;
   if (np > 0) {
     sum_parts<BLK>(part + blockIdx.y * rowsz, np, gcr_values(k), sums);
-    if (threadIdx.x < 64) gcr_coefficients<P>(sc, sums, k, cf, blockIdx.x == 0);
+    if (threadIdx.x < 64) gcr_coefficients<P, false>(sc, sums, k, cf, blockIdx.x == 0);
   } else {
     for (int j = threadIdx.x; j <= k; j += BLK) cf[j] = j < k ? sc->coef[k * kN + j] : sc->alpha[k];
   }
@@ -723,7 +729,7 @@ __global__ void __launch_bounds__(256) k_scal_beta(GcrScal *scs, int n, int keep
   const int j = threadIdx.x;
   if (np > 0) sum_parts<256>(part + blockIdx.x * rowsz, np, gcr_values(n - 1), sums);
   if (j >= 64) return;
-  if (np > 0) gcr_coefficients<P>(sc, sums, n - 1, cf, true);
+  if (np > 0) gcr_coefficients<P, false>(sc, sums, n - 1, cf, true);
   // (the last step's coefficients may just have been stored by other lanes)
   auto coef = [&](int k) { return np > 0 && k == n - 1 ? cf[j] : sc->coef[k * kN + j]; };
   double2 b = make_double2(0.0, 0.0);
@@ -874,13 +880,14 @@ namespace {
 //     of 12 rhs 2.66 / 2.62; FP64 without even-odd, GCR(32) 17.1 / 23.2.  From
 //     8000 sites up a batch of 12 FP16 rhs loses 16% with it, 3 FP32 rhs
 //     nothing, one rhs gains up to 11%.
-//   Long ones: a site (FP16, FP64) or half a site (FP32) per lane in the dots,
-//     fewer in the update, whose accumulators are FP64.  J = 2 FP16 vectors in
-//     flight in the update measured 1.5% of a 24^3x48 solve better than 4 (3
-//     wavefronts per SIMD) and 14% better than 4 held to 128 registers.  They
-//     run at 6.0-6.7 TB/s (24^3x48, 12 FP16 rhs; 16^3x32, one FP64 rhs), the
-//     rate of the fabric: running the update through the sites backwards, which
-//     would find the dots' last vectors in the last-level cache, changes nothing.
+//   Long ones: one site per lane and one or two vectors in flight, which leaves
+//     the most wavefronts to hide the loads: FP32 on 16^3x32, Q, GCR(32), with
+//     half a site and four vectors 124.2 ms, a site and one vector 120.8; one
+//     FP64 rhs 211.8 with a third of a site and four vectors in the update,
+//     205.9; 12 FP16 rhs on 24^3x48 with four vectors in both 135.0, 132.3.  The
+//     kernels run at 6.0-6.7 TB/s, the rate of the fabric: running the update
+//     through the sites backwards, which would find the dots' last vectors in
+//     the last-level cache, changes nothing.
 template <int M_, int J_, int BLK_>
 struct GcrShape {
   static constexpr int M = M_, J = J_, BLK = BLK_;
@@ -890,20 +897,20 @@ struct GcrShapes;
 template <>
 struct GcrShapes<QCD_HIP_F16> {
   using Short = GcrShape<1, 8, 192>;
-  using Dots = GcrShape<3, 4, 512>;
-  using Update = GcrShape<3, 2, 256>;
+  using Dots = GcrShape<3, 2, 512>;
+  using Update = GcrShape<3, 1, 256>;
 };
 template <>
 struct GcrShapes<QCD_HIP_F32> {
   using Short = GcrShape<1, 8, 256>;
-  using Dots = GcrShape<3, 4, 512>;
-  using Update = GcrShape<3, 4, 256>;
+  using Dots = GcrShape<6, 1, 512>;
+  using Update = GcrShape<6, 1, 256>;
 };
 template <>
 struct GcrShapes<QCD_HIP_F64> {
   using Short = GcrShape<1, 8, 256>;
-  using Dots = GcrShape<12, 1, 256>;
-  using Update = GcrShape<4, 4, 256>;
+  using Dots = GcrShape<12, 1, 512>;
+  using Update = GcrShape<12, 1, 256>;
 };
 // Up to this many workgroups per rhs the update forms the coefficients from the
 // partial sums itself (8^3x16: 64 of them); past it every one of its workgroups
@@ -962,8 +969,16 @@ int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream
     }
     gcr_launch<P, true>(V, count, [&](auto sh, dim3 grid) {
       using SH = decltype(sh);
-      k_gcr_dots<P, SH::M, SH::J, SH::BLK><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->ids, V, S->part, S->rowsz);
-      if (!np) k_gcr_scal<P><<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
+      auto dots = k_gcr_dots<P, SH::M, SH::J, SH::BLK, false>;
+      auto scal = k_gcr_scal<P, false>;
+      if constexpr (P != QCD_HIP_F64)
+        if (exact) {
+          if (k == 0) return;
+          dots = k_gcr_dots<P, SH::M, SH::J, SH::BLK, true>;
+          scal = k_gcr_scal<P, true>;
+        }
+      dots<<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->ids, V, S->part, S->rowsz);
+      if (!np) scal<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
     });
     if (exact)
       gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
