@@ -218,15 +218,23 @@ __global__ void __launch_bounds__(kBlock) k_gauss_gather_links(GaussArgs g, cons
   for (int k = 9; k < 36; k++) dst[gauge_index_e<E>(k, r, dstride)] = src[gauge_index_e<E>(k, s, sstride)];
 }
 
-// z steps per lane of k_gauss: four z chunks (at least 2 steps).  On a 48^3
-// slice with 12 rhs every length from 2 to 24 measured 201-226 us per
-// iteration (48: 328).  QCD_HIP_GAUSS_ZLEN overrides it.
-static unsigned gauss_zlen(unsigned Z) {
+// z steps per lane of k_gauss for a launch over `sites` (site, rhs) pairs: the
+// march saves loads but divides the wavefronts, so it is as long as leaves about
+// 4096 of them (four per SIMD).  Calls of 50 iterations with their sources, ms:
+// 24^3, 12 rhs 1.76 with 1 step, 2.14 with 6; 16^3, 12 rhs 0.77 with 1, 1.23 with
+// 4; 32^3, one rhs 0.58 with 1, 1.99 with 8; 32^3, 12 rhs 3.53 with 2, 3.60 with
+// 1 and 8; 22^3x16, 5 rhs (20 iterations) 2.84 with 3, 2.99 with 1, 3.20 with 6;
+// a 48^3 slice, 12 rhs: 201-226 us an iteration with 2 to 24.  (Lanes of one
+// spin each, without a march and with every hop's loads in flight: 5.29 ms on
+// 32^3, 2.38 on 24^3, 12 rhs; they gain on 8^3 only.)
+// QCD_HIP_GAUSS_ZLEN overrides it.
+static unsigned gauss_zlen(unsigned Z, long sites) {
   static const int env = [] {
     const char *e = std::getenv("QCD_HIP_GAUSS_ZLEN");
     return e ? std::atoi(e) : 0;
   }();
-  const unsigned r = env > 0 ? (unsigned)env : std::max(2u, (Z + 3) / 4);
+  const long per = 4096L * 64;
+  const unsigned r = env > 0 ? (unsigned)env : (unsigned)std::max(1L, std::min((sites + per / 2) / per, (long)Z));
   return r > Z ? Z : r;
 }
 
@@ -285,7 +293,7 @@ static int gauss_run(qcd_hip_field v, qcd_hip_field gauge, qcd_hip_field buf, in
   }
   const GaugeIn<P> U = GaugeIn<P>::of(links);
   const unsigned nb = (unsigned)grid_for(g.n);
-  g.zlen = gauss_zlen(g.Z);
+  g.zlen = gauss_zlen(g.Z, (long)g.n * std::min(rows, v->nrhs));
   g.ncb = (unsigned)grid_for((long)g.tn * g.X * g.Y);
   const unsigned nzc = (g.Z + g.zlen - 1) / g.zlen;
   for (int r0 = 0; r0 < v->nrhs; r0 += rows) {

@@ -60,3 +60,30 @@ def test_projection_of_ill_conditioned_links(gpu, scale):
     assert (np.abs(got - O.project_su3(m[:, 1:])).max(axis=(-1, -2)) <= tol[:, 1:]).all()
     uu = got @ got.conj().swapaxes(-1, -2)
     assert np.abs(uu - np.eye(3)).max() <= 1e-14 and np.abs(np.linalg.det(got) - 1).max() <= 1e-14
+
+
+def test_gauss_march_lengths_agree(gpu):
+    """A launch long enough to march (6 rhs: 2 planes a lane, 12 rhs: 3, the last
+    z chunk shorter) against one rhs, one plane a lane: the same bits."""
+    Q = gpu
+    L = (2, 32, 32, 34)
+    u = Q.gauge_generate(L, 0.3, 34)
+    lat = Q.Lattice(L)
+    g = Q.Gauge(lat).upload(u)
+    src = [Q.spinor_gaussian(L, 35 + r) for r in range(2)]
+    ref = []
+    for s in src:
+        f = Q.Spinor(lat).upload(s)
+        Q.gauss_smear(f, g, 4.0, -1, 3)
+        ref.append(f.download())
+    for n in (6, 12):
+        f = Q.Spinor(lat, nrhs=n)
+        for r in range(n):
+            f.upload(src[r % 2], rhs=r)
+        Q.gauss_smear(f, g, 4.0, -1, 3)
+        for r in (0, n // 2, n - 1):
+            assert np.array_equal(f.download(r), ref[r % 2])
+    v, geo = src[0], O.Geometry(L)
+    for _ in range(3):
+        v = O.gauss3d_all(geo, v, u, 4.0)
+    assert np.linalg.norm(ref[0] - v) <= 1e-13 * np.linalg.norm(v)
