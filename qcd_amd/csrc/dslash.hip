@@ -663,6 +663,9 @@ struct TuneVal {
   int map, occ;
   float ms;
   int bmap = 0, bocc = 0;   // launches over two or more rhs (0: use map, occ)
+  // D and Q without reduction take one wavefront per hop (split.hip) where that
+  // was faster: one rhs, and batches (if they were timed)
+  bool split = false, btimed = false, bsplit = false;
 };
 static std::vector<std::pair<TuneKey, TuneVal>> g_tune;
 static int g_autotune = -1;   // -1: read QCD_HIP_AUTOTUNE once
@@ -748,6 +751,30 @@ static int launch_cfg(int epi, bool red, int map, int occ, qcd_hip_field out, in
   return 1;
 }
 
+// Largest (site, rhs) count for which the tuner times one wavefront per hop.  D,
+// us, best traversal / one wavefront per hop: 8^3x16 FP64 7.7 / 4.5, FP32 6.3 /
+// 4.5, FP16 6.1 / 4.1; 12^3x24 11.5 / 10.9, 7.8 / 6.9, 6.6 / 5.7; 16^3x32 27.8 /
+// 29.0, 14.0 / 16.5, 9.7 / 11.4, over 3 rhs 61.7 / 60.9, 41.1 / 32.7, 23.4 / 26.9;
+// 20^3x40 70.1 / 69.3, 36.2 / 34.1, 21.4 / 23.8; 24^3x48 148 / 174.
+static const long kSplitSites = 1L << 20;
+// It is timed with its operands in the caches, and reads each neighbour plane
+// anew, which costs more when they are not: taken only when clearly faster, and
+// for batches of up to 4 rhs (on changing fields, us, traversal chosen without /
+// with it: FP32, 37 674 sites, 17 rhs 71.5 / 75.6; FP64, 12^3x24, 12 rhs 101 /
+// 103; FP32, 249 480 sites, 3 rhs 96.7 / 93.8).
+static const int kSplitRhs = 4;
+static const float kSplitGain = 0.92f;
+
+static DslashArgs batch_args(qcd_hip_lattice lat, double m, double tm, const Batch &bt) {
+  DslashArgs a = make_args(lat, m, tm);
+  a.ids = bt.ids;
+  a.count = (unsigned)bt.count;
+  a.in_rs = (unsigned)bt.in_rs;
+  a.out_rs = (unsigned)bt.out_rs;
+  a.b_rs = (unsigned)bt.b_rs;
+  return a;
+}
+
 // untuned default: z-march of 6 steps per lane
 static const int kDefaultMap = MAP_ZMARCH | (6 << 8);
 // Candidates: z-march lengths (1 = one site per lane), without and with the
@@ -793,6 +820,28 @@ int dslash_tune(qcd_hip_field out, qcd_hip_field in, qcd_hip_field g, int force)
                 key.L[3], key.ps, key.pg, map & 0xff, map >> 8, occ, ms * 1e3);
       if (ms < best.ms) best = TuneVal{map, occ, ms};
     }
+  }
+  // One wavefront per hop, for D and Q of few sites; map and occ stay what the
+  // other launches use.
+  auto time_split = [&](const Batch &bt, float *ms) -> int {
+    DslashArgs a = batch_args(in->lat, 0.0, 0.0, bt);
+    for (int w = 0; w < 2; w++) QH_TRY(dslash_split_launch(EPI_D, a, out, 0, in, 0, g, st));
+    QH_CHECK(hipEventRecord(e0, st));
+    for (int r = 0; r < reps; r++) QH_TRY(dslash_split_launch(EPI_D, a, out, 0, in, 0, g, st));
+    QH_CHECK(hipEventRecord(e1, st));
+    QH_CHECK(hipEventSynchronize(e1));
+    QH_CHECK(hipEventElapsedTime(ms, e0, e1));
+    *ms /= reps;
+    if (getenv("QCD_HIP_TUNE_VERBOSE"))
+      fprintf(stderr, "tune L=%dx%dx%dx%d ps=%d pg=%d %d rhs one wavefront per hop: %.2f us\n", key.L[0], key.L[1],
+              key.L[2], key.L[3], key.ps, key.pg, bt.count, *ms * 1e3);
+    return 0;
+  };
+  const bool can_split = in->prec == g->prec && in->lat->V <= kSplitSites;
+  if (can_split) {
+    float ms = 0.f;
+    QH_TRY(time_split(kOne, &ms));
+    best.split = ms < kSplitGain * best.ms;
   }
   // Batches (fields with several rhs): the best one-rhs traversal against
   // other traversals, timed over the first min(nrhs, 48) rhs (at 24^3x48 the
@@ -864,6 +913,12 @@ int dslash_tune(qcd_hip_field out, qcd_hip_field in, qcd_hip_field g, int force)
             best.bocc = occ;
           }
         }
+    best.btimed = true;
+    if (can_split && cnt <= kSplitRhs && in->lat->V * cnt <= kSplitSites) {
+      float ms = 0.f;
+      QH_TRY(time_split(bt, &ms));
+      best.bsplit = ms < kSplitGain * bbest;
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -919,6 +974,8 @@ int dslash_launch(int epi, bool red, qcd_hip_field out, int ro, qcd_hip_field in
                   qcd_hip_field b, int rb, double m, double tm, double *partials, hipStream_t stream, int *grid_out) {
   TuneVal t;
   const bool have = tune_get(key_of(in, g), &t);
+  if (have && t.split && !red && (epi == EPI_D || epi == EPI_Q))
+    return dslash_split_launch(epi, batch_args(in->lat, m, tm, kOne), out, ro, in, ri, g, stream);
   const int map = have ? t.map : kDefaultMap, occ = have ? t.occ : 0;
   return launch_cfg(epi, red, map, occ, out, ro, in, ri, g, b, rb, m, tm, partials, stream, grid_out);
 }
@@ -936,6 +993,11 @@ int dslash_launch_batch(int epi, bool red, qcd_hip_field out, int ro, int out_rs
   const bool two = have && count >= 2 && t.bmap != 0 && timed;
   const int map = two ? t.bmap : have ? t.map : kDefaultMap, occ = two ? t.bocc : have ? t.occ : 0;
   const Batch bt{ids, count, in_rs, out_rs, b_rs};
+  // (batches of a lattice tuned on one rhs: only while they are small as well)
+  const bool split = have && !red && (epi == EPI_D || epi == EPI_Q) &&
+                     (count == 1 ? t.split : t.btimed ? t.bsplit && count <= kSplitRhs
+                                                      : t.split && in->lat->V * count <= (1L << 16));
+  if (split) return dslash_split_launch(epi, batch_args(in->lat, m, tm, bt), out, ro, in, ri, g, stream);
   return launch_cfg(epi, red, map, occ, out, ro, in, ri, g, b, rb, m, tm, partials, stream, grid_out, bt);
 }
 

@@ -850,6 +850,11 @@ __device__ __forceinline__ void block_reduce_store(double v, double *partials, u
 int dslash_mma_launch(int epi, DslashArgs a, qcd_hip_field out, int ro, qcd_hip_field in, int ri, qcd_hip_field g,
                       qcd_hip_field b, int rb, hipStream_t st);
 
+// D or Q with one wavefront per hop (split.hip), for launches of few sites:
+// batch rows as in DslashArgs, the bits of the other traversals
+int dslash_split_launch(int epi, DslashArgs a, qcd_hip_field out, int ro, qcd_hip_field in, int ri,
+                        qcd_hip_field g, hipStream_t st);
+
 // launchers defined in dslash.hip
 // Batched launch over `count` right-hand sides (see DslashArgs::ids): row y
 // applies the operator to vector ri + slot*in_rs of `in`, writes vector

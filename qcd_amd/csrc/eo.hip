@@ -609,7 +609,7 @@ static int eo_launch_z(int epi, bool red, const EoArgs &e, unsigned zlen, bool t
 }
 
 // z chunks tuned per (lattice extents, spinor precision, rows per lane, rows
-// or row pairs per launch): the first launch of a shape with at least 2^17
+// or row pairs per launch; 0: one wavefront per hop): the first launch of a shape with at least 2^17
 // (row, half-site) items that may run twice (not under graph capture, out
 // aliasing neither in nor b) times chunks of 1 to 12 planes and keeps the
 // fastest; smaller launches keep one site per lane.  All give bit-identical
@@ -642,6 +642,16 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
     if ((int)e.d.count >= eo_mma_min_rhs() && !red && (epi == EO_MINV || epi == EO_SCHUR))
       return eo_mma_launch(epi, e, out, ro, in, ri, g, b, rb, st);
   }
+  // few (row, half-site) items: one wavefront per hop, unless z steps are set.
+  // Even-odd GCR(12) solves, ms, against the kernels below: 8^3x16, one rhs FP64
+  // 2.37 -> 1.85, 3 rhs FP32 2.32 -> 1.70, 12 rhs FP16 2.65 -> 2.49, FP64 4.52 ->
+  // 4.47; 12^3x24, 3 rhs FP32 3.59 -> 3.20, FP16 2.86 -> 2.71, FP64 5.20 -> 5.28;
+  // 16^3x32, one rhs (65 536 items) FP64 6.31 -> 6.25, FP32 3.68 -> 3.59, FP16
+  // 2.67 -> 2.76.
+  const double items = (double)e.d.count * e.Vh;
+  const bool may_split = !red && eo_zlen_setting().load() == 0;
+  if (may_split && items < (PS == QCD_HIP_F16 ? 65536.0 : 131072.0))
+    return eo_split_launch(epi, e, out, ro, in, ri, g, b, rb, st);
   const bool two = PS != QCD_HIP_F64 && e.d.count >= 2 && !red && (epi == EO_MINV || epi == EO_SCHUR) &&
                    eo_two_rhs();
   const unsigned rows = two ? (e.d.count + 1) / 2 : e.d.count;
@@ -656,6 +666,10 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
     if (it != eo_ztuned().end()) {
       zlen = it->second.zlen;
       et.rgroup = it->second.rgroup;
+      if (zlen == 0) {   // (a launch with reduction of the same shape keeps one site per lane)
+        if (!red) return eo_split_launch(epi, e, out, ro, in, ri, g, b, rb, st);
+        zlen = 1;
+      }
     } else {
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       QH_CHECK(hipStreamIsCapturing(st, &cs));
@@ -674,15 +688,21 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
         const bool rg_set = getenv("QCD_HIP_EO_RGROUP") != nullptr;   // a set group size is kept
         const unsigned rg4 = rg_set ? e.rgroup : std::min(4u, e.d.count);
         const unsigned rg12 = rg_set ? e.rgroup : std::min(12u, e.d.count);
-        for (unsigned z : {1u, 2u, 3u, 4u, 6u, 8u, 12u}) {
+        // z = 0: one wavefront per hop, while that is near (12 FP16 rhs of
+        // 12^3x24: 5.8 against 6.6 ms a solve; 3 FP32 rhs of 16^3x32: 8.5 against 7.5)
+        auto launch = [&](const EoArgs &ec, unsigned z) {
+          return z == 0 ? eo_split_launch(epi, ec, out, ro, in, ri, g, b, rb, st)
+                        : eo_launch_z<PS, PG>(epi, red, ec, z, two, rows, gr, si, gu, so, sb, partials, st);
+        };
+        for (unsigned z : {0u, 1u, 2u, 3u, 4u, 6u, 8u, 12u}) {
           if (z > 1 && eo_zlen_fits(e, z) != z) continue;
+          if (z == 0 && (!may_split || items > (double)(1 << 20))) continue;
           for (unsigned rg : {rg4, rg12}) {
             EoArgs ec = e;
             ec.rgroup = rg;
-            rc = eo_launch_z<PS, PG>(epi, red, ec, z, two, rows, gr, si, gu, so, sb, partials, st);
+            rc = launch(ec, z);
             if (!rc && hipEventRecord(e0, st) != hipSuccess) rc = 2;
-            for (int r = 0; r < reps && !rc; r++)
-              rc = eo_launch_z<PS, PG>(epi, red, ec, z, two, rows, gr, si, gu, so, sb, partials, st);
+            for (int r = 0; r < reps && !rc; r++) rc = launch(ec, z);
             float ms = 0.f;
             if (!rc && (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                         hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
@@ -696,7 +716,7 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
               zlen = z;
               et.rgroup = rg;
             }
-            if (rg4 == rg12) break;   // one group size
+            if (rg4 == rg12 || z == 0) break;   // one group size
           }
           if (rc) break;
         }
@@ -707,6 +727,7 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
           return rc;
         }
         eo_ztuned()[key] = EoZVal{zlen, et.rgroup};
+        if (zlen == 0) return eo_split_launch(epi, e, out, ro, in, ri, g, b, rb, st);
       }
     }
   }

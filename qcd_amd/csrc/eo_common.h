@@ -106,6 +106,10 @@ int eo_accumulate_p(qcd_hip_field x, int f0, qcd_hip_field ev, qcd_hip_field od,
 // EO_SCHUR, any rhs count
 int eo_mma_launch(int epi, const EoArgs &e, qcd_hip_field out, int ro, qcd_hip_field in, int ri, qcd_hip_field g,
                   qcd_hip_field b, int rb, hipStream_t st);
+// the hops without reduction with one wavefront per hop (split.hip), for
+// launches of few sites; the bits of k_eo_hop
+int eo_split_launch(int epi, const EoArgs &e, qcd_hip_field out, int ro, qcd_hip_field in, int ri, qcd_hip_field g,
+                    qcd_hip_field b, int rb, hipStream_t st);
 // build the matrix-core hop links of FP16 gauge field g for the phases of
 // lattice lat before a graph capture uses them (mma.hip)
 int mma_prepare(qcd_hip_field g, qcd_hip_lattice lat, hipStream_t st);
