@@ -164,7 +164,7 @@ typedef struct {
                           full D x = b; needs every extent even; op is then D */
    int    graph;       /* 1 (default): each GCR cycle is captured once as a
                           HIP graph and replayed (one launch instead of
-                          about 7 per GCR step); 0: launched kernel by kernel.
+                          about 3 per GCR step); 0: launched kernel by kernel.
                           Both run the same kernels in the same order. */
 } qcd_hip_solver_params;
 typedef struct {

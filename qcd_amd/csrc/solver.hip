@@ -7,22 +7,22 @@
 // operator A = Q = i g5 D (as invert.c) or A = D.  For A = Q the system solved
 // is Q x = i g5 b, i.e. D x = b, so the residual is ||b - D x|| either way.
 //
-// GCR iteration k (w_k = A res_k, made orthogonal to the earlier w_j and kept
-// unnormalised):
-//   k_gcr_dots:    d_j = <w_j, w_k>, j < k, |w_k|^2, <w_k, res_k>  (reads k+2
-//                  vectors)
-//   k_gcr_scal:    coef[k][j] and alpha[k] (few sums: formed by k_gcr_update)
-//   k_gcr_update:  w_k += sum_j coef[k][j] w_j, res_{k+1} = res_k + alpha[k] w_k
-//                  (reads k+2 vectors, writes 2; not needed in the last step).
-//                  Q in reduced precision: w_k, then alpha[k] from its own
-//                  sums, then res_{k+1}
-// After n iterations k_solution forms x = sum_j beta_j res_j, beta from coef and
-// alpha (the reference updates x every iteration).
+// GCR's steps are taken in blocks of S = 4 (2 and 1 for the last ones of a
+// cycle), from residual res_k: the operator S times, then
+//   k_gcr_dots:    the S new vectors with the earlier w_j, j < k, and with each
+//                  other (reads k + S + 1 vectors)
+//   k_gcr_scal:    coef and alpha of the S steps
+//   k_gcr_update:  w_k .. w_{k+S-1}, orthogonal and unnormalised, and res_{k+S}
+//                  (reads k + S + 1 vectors, writes S + 1; not needed in the
+//                  last block)
+// After n steps k_solution forms x = sum_j beta_j d_j over the directions d_j
+// that the operator was applied to, beta from coef and alpha (the reference
+// updates x every iteration).
 // All coefficients live in device memory: a cycle needs no host round trip.
 // Right-hand sides are solved in batches of prm.batch that advance in
 // lockstep: every kernel takes a second grid dimension over the batch, and
 // right-hand sides that have converged drop out of the launches.
-// Orthogonalisation is classical Gram-Schmidt in one fused pass (the
+// Orthogonalisation is block-classical Gram-Schmidt in one fused pass (the
 // reference's modified Gram-Schmidt, invert.c:68-73, is the same projection in
 // exact arithmetic); the outer FP64 residual absorbs the difference.
 #include "eo_common.h"
@@ -45,16 +45,19 @@ int eo_scale64(qcd_hip_lattice full, qcd_hip_field in, qcd_hip_field out, const 
 qcd_hip_lattice eo_half_lattice(qcd_hip_lattice full);
 
 constexpr int kN = kMaxKrylov;
+constexpr int kSteps = 4;   // most GCR steps of one block
 
-// The coefficients of one right-hand side's GCR cycle.  w_k = A res_k +
-// sum_j coef[k][j] w_j, res_{k+1} = res_k + alpha[k] w_k.
+// The coefficients of one right-hand side's GCR cycle: w_k = A d_k + sum_j
+// coef[k][j] w_j, and the residual after step k is the one before + alpha[k] w_k.
 struct GcrScal {
   double2 coef[kN * kN];   // [k][j], j < k
   double2 alpha[kN];
-  double2 beta[kN];        // the cycle's solution is sum_j beta_j res_j
+  double2 beta[kN];        // the cycle's solution is sum_j beta_j d_j
   double w2inv[kN];        // 1 / |w_k|^2 of the stored w_k
-  double rmin[kN];         // smallest |res_i|^2, i <= k
-  int stop[kN];            // the cycle's steps from k on are left out
+  double2 step[kSteps];    // what the stored residual takes of the block's w
+  double2 undo, take;      // the part of w_{k-1} that the next / this block takes out of it
+  double rmin;             // smallest |res_k|^2 so far
+  int stop;                // the rest of the cycle's steps are left out
   double rnorm;
   double rscale;
   int bad;
@@ -66,7 +69,7 @@ __device__ __forceinline__ double2 cmul2(double2 a, double2 b) {
 
 // Batched kernels: grid row y works on right-hand-side slot ids[y]; the
 // Krylov vector j of slot b is vector b*n + j of the Rs / Ws fields; row y
-// writes its partial sums at part + y*rowsz, laid out [value][workgroup].
+// writes its partial sums at part + y*rowsz.
 
 // ------------------------------------------------------------ chunks
 // A vector is an array of 16-byte chunks: tile after tile, kG groups of 64
@@ -103,15 +106,26 @@ struct Chunk {
       return to_cx<R>(as_half2(q[i]));
     }
   }
+  // product of the low half of a with the low (HI: high) half of b, exact in
+  // FP32.  Mixed-precision instructions: as a multiplication of converted values
+  // the compiler keeps every vector that is used again converted, in twice the
+  // registers.
+  template <bool HI>
+  static __device__ __forceinline__ float half_product(unsigned a, unsigned b) {
+    float r;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b));
+    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
   // sum over the chunk of conj(a) b, of stored values
   static __device__ __forceinline__ void dot(u32x4 a, u32x4 b, double &re, double &im) {
 #pragma unroll
     for (int i = 0; i < kC; i++) {
       const auto x = get(a, i), y = get(b, i);
       if constexpr (P == QCD_HIP_F16) {
-        // a product of two half values is exact in FP32; one rounding per sum
-        re += (double)fmaf(x.im, y.im, x.re * y.re);
-        im += (double)fmaf(-x.im, y.re, x.re * y.im);
+        // one rounding per sum
+        re += (double)fmaf(x.im, y.im, half_product<false>(a[i], b[i]));
+        im += (double)fmaf(-x.im, y.re, half_product<true>(a[i], b[i]));
       } else {
         re = fma((double)x.re, (double)y.re, fma((double)x.im, (double)y.im, re));
         im = fma((double)x.re, (double)y.im, fma(-(double)x.im, (double)y.re, im));
@@ -211,6 +225,21 @@ __device__ __forceinline__ double wave_sum_scatter(double (&v)[NV]) {
   return v[0];
 }
 
+// out[i] = x[i] summed over the wavefront, i < min(NX, used), NP at a time
+template <int NP, int NX>
+__device__ __forceinline__ void wave_reduce(const double (&x)[NX], double *out, int used) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < NX; i += NP) {
+    double y[NP];
+#pragma unroll
+    for (int q = 0; q < NP; q++) y[q] = i + q < NX ? x[i + q < NX ? i + q : 0] : 0.0;
+    const double t = wave_sum_scatter<NP>(y);
+    const int q = i + lane / (64 / NP);
+    if (lane % (64 / NP) == 0 && q < (NX < used ? NX : used)) out[q] = t;
+  }
+}
+
 // Sum a [nv][nb] partial array (one wave per value, an order fixed by nb)
 // into sums.  Each lane keeps four running sums over partials 256 apart, so
 // its loads do not wait on one chain of additions (rows of 20 000 partials
@@ -235,23 +264,28 @@ __device__ void wave_sums(const double *part, int nv, unsigned nb, double *sums)
   }
 }
 
-// sums[q] = sum over p < np of part[p nv + q], q < nv <= BLK, in an order fixed
-// by np and BLK: BLK / nv lanes per value, each over every (BLK / nv)th p, then
-// a tree over LDS.  The whole workgroup calls it; sums holds BLK values.
+// sums[q] = sum over p < np of part[p nv + q], q < nv, in an order fixed by np,
+// nv and BLK: BLK / nv lanes per value, each over every (BLK / nv)th p, then a
+// tree over LDS.  The whole workgroup calls it; sums holds BLK values, nv <= BLK.
 template <int BLK>
 __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsigned nv, double *sums) {
+  constexpr unsigned NL = 8;
   unsigned g = BLK / nv;
   const unsigned t = threadIdx.x, p0 = t / nv, q = t - p0 * nv;
   double x = 0.0;
   if (p0 < g) {
     const double *a = part + q;
-    for (unsigned p = p0; p < np; p += 8 * g) {   // eight loads in flight, the last ones too
-      double y[8];
+    for (unsigned p = p0; p < np; p += NL * g) {   // NL loads in flight, the last ones too (16: no faster)
+      double y[NL];
 #pragma unroll
-      for (int i = 0; i < 8; i++) y[i] = a[(size_t)min(p + i * g, np - 1) * nv];
+      for (unsigned i = 0; i < NL; i++) y[i] = a[(size_t)min(p + i * g, np - 1) * nv];
 #pragma unroll
-      for (int i = 0; i < 8; i++) y[i] = p + i * g < np ? y[i] : 0.0;
-      x += ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+      for (unsigned i = 0; i < NL; i++) y[i] = p + i * g < np ? y[i] : 0.0;
+#pragma unroll
+      for (unsigned h = NL / 2; h > 0; h /= 2)
+#pragma unroll
+        for (unsigned i = 0; i < h; i++) y[i] += y[i + h];
+      x += y[0];
     }
   }
   sums[t] = x;
@@ -264,85 +298,190 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
   }
 }
 
-// Smallest |w_k|^2 / |A res_k|^2 that the difference below can tell from
-// rounding of the stored vectors
+// ------------------------------------------------------- blocks of GCR steps
+// Directions of a block of S steps at k: d_0 = res_k, d_{a+1} = (A - theta) d_a,
+// so v_a = A d_a = d_{a+1} + theta d_a.  w_k .. w_{k+S-1} span what S single steps
+// would add, so the residual and the solution after the block are those of
+// GCR(n).  The S vectors are projected against the
+// w_j, j < k, in one pass over them and formed in a second one, where single
+// steps take 2 S passes, and these passes are what a cycle spends its time on
+// (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2
+// and 4, ms: one FP64 rhs, Q, GCR(32) on 16^3x32 204, 126, 87; 12 FP16 rhs,
+// GCR(12) on 24^3x48 132, 107, 98, on 16^3x32 21.0, 16.9, 15.5.
+//
+// theta is the local term m + 4 of D and of the Schur complement (0 for Q): the
+// d_a are then, but for factors, the residuals of Richardson's iteration, about
+// as independent of each other as the residuals of single steps, and a long FP16
+// cycle reaches the same residual: GCR(32) on 8^3x16, kappa 0.125, 4.0e-4 of the
+// one before, single steps 4.9e-4 (d_1 without theta 8.1e-4).  The outer step
+// counts are those of single
+// steps for FP64, FP32 and FP16, Q and D, GCR(4) to GCR(64), kappa 0.12 to
+// 0.139, random and point sources (FP16 with 64 steps: one cycle more or less).
+
+// Smallest |w_{k+a}|^2 / |v_a|^2 that is told from rounding of the stored vectors:
+// a v_a with less to itself is left out of the cycle
 template <int P>
-constexpr double gcr_floor() { return P == QCD_HIP_F64 ? 1e-13 : P == QCD_HIP_F32 ? 1e-6 : 1e-4; }
+constexpr double gcr_floor() { return P == QCD_HIP_F64 ? 1e-13 : P == QCD_HIP_F32 ? 1e-12 : 1e-6; }
 
-// sums of step k: d_j = <w_j, A res_k> for j < k (re, im), |A res_k|^2,
-// |res_k|^2, <A res_k, res_k> (re, im), |w_{k-1}|^2
-__host__ __device__ constexpr unsigned gcr_values(int k) { return 2 * (unsigned)k + 5; }
+// sums of a block of S steps at k: <w_j, d_{a+1}>, a < S, at 2 S j + 2 a (re,
+// im) for j < k; then at 2 S k: <d_b, d_a> for b < a <= S at a a + 2 b (re,
+// im), |d_a|^2 at a a + 2 a; then |w_{k-1-i}|^2, i < kSteps
+template <int S>
+constexpr unsigned gcr_own = (S + 1) * (S + 1);
+template <int S>
+__host__ __device__ constexpr unsigned gcr_values(int k) {
+  return 2 * S * (unsigned)k + gcr_own<S> + kSteps;
+}
 
-// Coefficients of step k from its sums (first wavefront of a workgroup).  The
-// w_j are orthogonal to each other and to res_k, so with
-//   coef_j = -d_j / |w_j|^2,  w_k = A res_k + sum_j coef_j w_j
-// |w_k|^2 = |A res_k|^2 - sum_j |d_j|^2 / |w_j|^2 and <w_k, res_k> =
-// <A res_k, res_k>: the step length alpha = -<w_k, res_k> / |w_k|^2 is known
-// before w_k is formed, and w_k and res_{k+1} come out of one pass.  The
-// solution is formed from the same coef and alpha, so it matches res_{k+1}
-// whatever alpha is; rounding in alpha only makes the step a little shorter or
-// longer than the best one.  Where the difference cancels (A res_k in the span
-// of the w_j) it is bounded below, which shortens the step.  In reduced
-// precision the w_j of a long cycle lose their orthogonality and a step can
-// come out far too long (FP16, 64 steps on 270 sites): |res_k|^2 above four
-// times the smallest before it leaves that step and the rest of the cycle out
-// (alpha = 0).
-// cf[j] = coef_j, cf[k] = alpha, cf[k + 1].x = whether step k - 1 is left out;
-// store: write the results to sc as well.  EXACT (k_gcr_update): the coef_j
-// alone.
-template <int P, bool EXACT>
-__device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, double2 *cf, bool store) {
+__device__ __forceinline__ double2 cadd2(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 conj2(double2 a) { return make_double2(a.x, -a.y); }
+__device__ __forceinline__ double2 scale2(double f, double2 a) { return make_double2(f * a.x, f * a.y); }
+__device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.y; }
+
+// Coefficients of a block of S steps from its sums (one wavefront, lane j takes
+// w_j).  The w_j are orthogonal to each other and to res_k, so with
+//   <w_{k+b}, v_a>, |w_{k+a}|^2, <w_{k+a}, res_k>
+// from the Gram matrix of the v_a less its part along the w_j (an L D L^H
+// factorisation) every step length is known before the w_{k+a} are formed, and
+// w_k .. w_{k+S-1} and res_{k+S} come out of one pass.  The solution is formed
+// from the same coef and alpha, so it matches the residual whatever alpha is;
+// rounding in alpha only makes a step a little shorter or longer than the best
+// one.  A v_a in the span of the others (gcr_floor: exhausted spaces) gets alpha =
+// 0 and w2inv = 0, so nothing refers to it.  In reduced precision the w_j of a
+// long cycle lose their orthogonality and a step can come out far too long
+// (FP16, 64 steps on 270 sites): |res_k|^2 above four times the smallest before
+// it leaves the last block and the rest of the cycle out (alpha = 0).  prev:
+// steps of the block before.
+//
+// The next block starts from res_{k+S}, which has to hold something of
+// w_{k+S-1} for its vectors to be new.  Q is indefinite and leaves every other
+// step nearly empty (point sources: empty): then the stored residual takes
+// kKeep |res_{k+S}| of w_{k+S-1} in place of the step alpha, the solution alpha
+// itself, and the next block takes the difference (undo) out again.
+constexpr double kKeep = 0.5;
+template <int P, int S>
+__device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, int prev, double theta) {
   const int j = threadIdx.x;
-  const double *own = sums + 2 * k;
-  const double wl = own[4], wli = wl > 0.0 ? 1.0 / wl : 0.0, r2 = own[1];
-  const bool stop = !EXACT && k > 0 && (sc->stop[k - 1] || r2 > 4.0 * sc->rmin[k - 1]);
-  double e = 0.0;
+  const double *own = sums + 2 * S * k, *wn = own + gcr_own<S>;
+  const double r2 = own[0] - (k > 0 ? norm2(sc->undo) * wn[0] : 0.0);
+  const bool stop = k > 0 && (sc->stop || r2 > 4.0 * sc->rmin);
+  constexpr int NV = S * S > 1 ? S * S : 2;
+  double e[NV] = {};   // what the w_j take of the v_a's Gram matrix
+  double2 d[S] = {};
   if (j < k) {
-    const double w = j == k - 1 ? wli : sc->w2inv[j];
-    const double2 d = make_double2(sums[2 * j], sums[2 * j + 1]), c = make_double2(-w * d.x, -w * d.y);
-    cf[j] = c;
-    if (store) sc->coef[k * kN + j] = c;
-    e = (d.x * d.x + d.y * d.y) * w;
-  }
-  if constexpr (EXACT) {
-    if (j == 0) sc->w2inv[k - 1] = wli;
-    return;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
-  if (j == 0) {
-    const double n = own[0], t = fmax(n - e, gcr_floor<P>() * n), w = 1.0 / t;
-    const double2 al = stop ? make_double2(0.0, 0.0) : make_double2(-w * own[2], -w * own[3]);
-    cf[k] = al;
-    cf[k + 1] = make_double2(stop ? 1.0 : 0.0, 0.0);
-    if (store) {
-      // Krylov space is sick (invert.c:75-79)
-      if (!stop && (!(w == w) || isinf(w) || !(e == e))) sc->bad = 1;
-      if (k > 0) sc->w2inv[k - 1] = wli;
-      if (stop) sc->alpha[k - 1] = make_double2(0.0, 0.0);
-      sc->rmin[k] = k > 0 ? fmin(sc->rmin[k - 1], r2) : r2;
-      sc->stop[k] = stop;
-      sc->alpha[k] = al;
+    double w;
+    w = sc->w2inv[j];
+    if (j >= k - prev && w > 0.0) {   // as stored
+      const double x = wn[k - 1 - j];
+      w = x > 0.0 ? 1.0 / x : 0.0;
+      sc->w2inv[j] = w;
     }
+#pragma unroll
+    for (int a = S - 1; a >= 0; a--) {
+      const double *x = sums + 2 * (S * j + a);
+      d[a] = make_double2(x[0], x[1]);
+      if (a > 0) d[a] = cadd2(d[a], make_double2(theta * x[-2], theta * x[-1]));
+      else if (j == k - 1) d[0] = cadd2(d[0], scale2(-theta * wn[0], sc->undo));   // <w_j, res_k> = 0
+    }
+#pragma unroll
+    for (int a = 0; a < S; a++) {
+      sc->coef[(k + a) * kN + j] = scale2(-w, d[a]);
+#pragma unroll
+      for (int b = 0; b < a; b++) {
+        const double2 x = cmul2(conj2(d[b]), d[a]);
+        e[a * a + 2 * b] = w * x.x;
+        e[a * a + 2 * b + 1] = w * x.y;
+      }
+      e[a * a + 2 * a] = w * norm2(d[a]);
+    }
+  }
+  const double t = wave_sum_scatter<NV>(e);
+  // <d_b, d_a>
+  auto dd = [&](int b, int a) {
+    if (a == b) return make_double2(own[a * a + 2 * a], 0.0);
+    const double *x = b < a ? own + a * a + 2 * b : own + b * b + 2 * a;
+    return make_double2(x[0], b < a ? x[1] : -x[1]);
+  };
+  // <v_b, v_a>, v_a = d_{a+1} + theta d_a
+  auto vv = [&](int b, int a) {
+    return cadd2(cadd2(dd(b + 1, a + 1), scale2(theta, cadd2(dd(b + 1, a), dd(b, a + 1)))),
+                 scale2(theta * theta, dd(b, a)));
+  };
+  double2 L[S][S], g[S][S], R[S];
+  double wi[S], rest = r2;
+  bool bad = false;
+#pragma unroll
+  for (int a = 0; a < S; a++) {
+    const double n = vv(a, a).x;
+    double N = n - __shfl(t, (a * a + 2 * a) * (64 / NV), 64);
+    R[a] = cadd2(dd(a + 1, 0), scale2(theta, dd(a, 0)));
+    if (k > 0)   // res_k = d_0 + undo w_{k-1}
+      R[a] = cadd2(R[a], cmul2(sc->undo, make_double2(__shfl(d[a].x, k - 1, 64), -__shfl(d[a].y, k - 1, 64))));
+#pragma unroll
+    for (int b = 0; b < a; b++) {
+      const double2 x = vv(b, a);
+      L[a][b] = make_double2(x.x - __shfl(t, (a * a + 2 * b) * (64 / NV), 64),
+                             x.y - __shfl(t, (a * a + 2 * b + 1) * (64 / NV), 64));   // <w_{k+b}, v_a>
+#pragma unroll
+      for (int c = 0; c < b; c++) L[a][b] = cadd2(L[a][b], cmul2(conj2(g[b][c]), L[a][c]));
+      g[a][b] = scale2(-wi[b], L[a][b]);
+      N -= wi[b] * norm2(L[a][b]);
+      R[a] = cadd2(R[a], cmul2(conj2(g[a][b]), R[b]));
+      if (j == 0) sc->coef[(k + a) * kN + k + b] = g[a][b];
+    }
+    wi[a] = N > gcr_floor<P>() * n ? 1.0 / N : 0.0;
+    bad = bad || !(N == N) || isinf(N) || (a == 0 && !(n > 0.0));
+    rest -= wi[a] * norm2(R[a]);
+    if (j == 0) {
+      sc->w2inv[k + a] = wi[a];
+      sc->alpha[k + a] = sc->step[a] = stop ? make_double2(0.0, 0.0) : scale2(-wi[a], R[a]);
+    }
+  }
+  if (j == 0) {
+    if (!stop && bad) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
+    if (stop)
+      for (int i = 1; i <= prev; i++) sc->alpha[k - i] = make_double2(0.0, 0.0);
+    sc->rmin = k > 0 ? fmin(sc->rmin, r2) : r2;
+    sc->stop = stop;
+    // res_k as stored less the last block's undo
+    sc->take = k > 0 ? sc->undo : make_double2(0.0, 0.0);
+    const double2 al = scale2(-wi[S - 1], R[S - 1]);
+    const double least = kKeep * kKeep * fmax(rest, 0.0) * wi[S - 1], len = norm2(al);
+    double2 undo = make_double2(0.0, 0.0);
+    if (!stop && len < least) {   // (w2inv = 0: never)
+      const double f = sqrt(least);
+      const double2 x = len > 0.0 ? scale2(f / sqrt(len), al) : make_double2(f, 0.0);
+      sc->step[S - 1] = x;
+      undo = make_double2(al.x - x.x, al.y - x.y);
+    }
+    sc->undo = undo;
   }
 }
 
-// Step k's sums (gcr_values) with the unorthogonalised w_k = A res_k, one partial
-// per value and workgroup, a workgroup's side by side.
+// vector d_a of a block of S steps at k: the last one where the last w goes,
+// the others among the search directions
+template <int P, int S>
+struct GcrD {
+  const SpinorSet<P> &set;
+  int slot;
+  __device__ __forceinline__ GcrD(const SpinorSet<P> &W, const SpinorSet<P> &Rs, int k, int a)
+      : set(a == S ? W : Rs), slot(k + (a == S ? S - 1 : a)) {}
+};
+
+// The sums (gcr_values) of a block of S steps at k, one partial per value and
+// workgroup, a workgroup's side by side.
 //
-// Streams k + 2 vectors, J of them in flight at a time (the last group reads
-// its last vector again where k is no multiple of J); PRE: the next group is
-// loaded before the present one is reduced, for launches with few wavefronts
-// per SIMD.  A wavefront adds its sums in its LDS row; the workgroup adds the
-// rows once.  EXACT (as k_gcr_update): only the d_j and |w_{k-1}|^2 are used,
-// and res_k is not read.
-template <int P, int M, int J, int BLK, bool EXACT>
-__global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, const int *ids,
-                                                  unsigned V, double *part, size_t rowsz) {
+// Streams k + S + 1 vectors, J of the w_j in flight at a time (the last group
+// reads its last vector again where k is no multiple of J); PRE: the next
+// group is loaded before the present one is reduced, for launches with few
+// wavefronts per SIMD.  A wavefront adds its sums in its LDS row; the workgroup
+// adds the rows once.
+template <int P, int S, int M, int J, int BLK, bool PRE>
+__global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, int prev,
+                                                  const int *ids, unsigned V, double *part, size_t rowsz) {
   using CH = Chunk<P>;
-  constexpr int NW = BLK / 64, NV = 2 * J;
-  constexpr bool PRE = M == 1;
-  __shared__ double sums[NW][2 * kN + 8];
+  constexpr int NW = BLK / 64, D = S + 1, NV = 2 * S * J, NP = NV <= 4 ? 4 : NV <= 8 ? 8 : 16;
+  __shared__ double sums[NW][gcr_values<S>(kN - S)];
   const int b = ids[blockIdx.y];
   const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
   const unsigned wid = threadIdx.x >> 6;
@@ -361,47 +500,39 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
       for (int m = 0; m < M; m++) g.a[i][m] = CH::load(W, j, l.q0 + 64 * m);
     }
   };
-  u32x4 wk[M];
-  float nk = 0.f;
-  double last[2] = {0.0, 0.0};
+  u32x4 d[D][M];
+  float nd[D] = {};
   Group next;
+  double *own = sums[wid] + 2 * S * k;
+  if (l.lane < kSteps) own[gcr_own<S> + l.lane] = 0.0;
   {
-    u32x4 r[M];
-    float nr = 0.f;
-    double own[4] = {0.0, 0.0, 0.0, 0.0};
-    if (l.valid) {
-      nk = CH::norm(W, k0 + k, l.site());
-      if constexpr (!EXACT) nr = CH::norm(Rs, k0 + k, l.site());
+    double x[gcr_own<S>] = {};
+    if (l.valid)
 #pragma unroll
-      for (int m = 0; m < M; m++) {
-        wk[m] = CH::load(W, k0 + k, l.q0 + 64 * m);
-        if constexpr (!EXACT) r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
+      for (int a = 0; a < D; a++) {
+        const GcrD<P, S> v(W, Rs, k0 + k, a);
+        nd[a] = CH::norm(v.set, v.slot, l.site());
+#pragma unroll
+        for (int m = 0; m < M; m++) d[a][m] = CH::load(v.set, v.slot, l.q0 + 64 * m);
       }
-    }
     if constexpr (PRE)
       if (k > 0) load(next, 0);
-    if (!EXACT && l.valid) {
-      double re = 0.0, im = 0.0, n2 = 0.0, r2 = 0.0;
+    if (l.valid)
 #pragma unroll
-      for (int m = 0; m < M; m++) {
-        CH::norm2(wk[m], n2);
-        CH::dot(wk[m], r[m], re, im);
-        CH::norm2(r[m], r2);
+      for (int a = 0; a < D; a++) {
+        double *y = x + a * a;
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+#pragma unroll
+          for (int c = 0; c < a; c++) CH::dot(d[c][m], d[a][m], y[2 * c], y[2 * c + 1]);
+          CH::norm2(d[a][m], y[2 * a]);
+        }
+        if constexpr (P == QCD_HIP_F16) {
+#pragma unroll
+          for (int c = 0; c <= 2 * a; c++) y[c] *= (double)nd[a] * (double)nd[c / 2];
+        }
       }
-      if constexpr (P == QCD_HIP_F16) {
-        const double f = (double)nk * (double)nr;
-        re *= f;
-        im *= f;
-        n2 *= (double)nk * (double)nk;
-        r2 *= (double)nr * (double)nr;
-      }
-      own[0] = n2;
-      own[1] = r2;
-      own[2] = re;
-      own[3] = im;
-    }
-    const double t = EXACT ? 0.0 : wave_sum_scatter<4>(own);
-    if ((l.lane & 15u) == 0) sums[wid][2 * k + (l.lane >> 4)] = t;
+    wave_reduce<NP>(x, own, gcr_own<S>);
   }
   for (int j0 = 0; j0 < k; j0 += J) {
     Group g;
@@ -411,39 +542,38 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
     } else {
       load(g, j0);
     }
-    double v[NV];
+    double x[NV] = {};
+    if (l.valid)
 #pragma unroll
-    for (int i = 0; i < NV; i++) v[i] = 0.0;
-    if (l.valid) {
+      for (int i = 0; i < J; i++)
 #pragma unroll
-      for (int i = 0; i < J; i++) {
+        for (int a = 0; a < S; a++) {
+          double *y = x + 2 * (S * i + a);
 #pragma unroll
-        for (int m = 0; m < M; m++) CH::dot(g.a[i][m], wk[m], v[2 * i], v[2 * i + 1]);
-        if constexpr (P == QCD_HIP_F16) {
-          const double f = (double)g.nj[i] * (double)nk;
-          v[2 * i] *= f;
-          v[2 * i + 1] *= f;
+          for (int m = 0; m < M; m++) CH::dot(g.a[i][m], d[a + 1][m], y[0], y[1]);
+          if constexpr (P == QCD_HIP_F16) {
+            const double f = (double)g.nj[i] * (double)nd[a + 1];
+            y[0] *= f;
+            y[1] *= f;
+          }
         }
-      }
-      if (j0 + J >= k) {   // the group's last vector is w_{k-1}
-        double n2 = 0.0;
+    wave_reduce<NP>(x, sums[wid] + 2 * S * j0, 2 * S * (k - j0));
+    if (j0 + J > k - prev)   // the block before: |w_j|^2 as stored
 #pragma unroll
-        for (int m = 0; m < M; m++) CH::norm2(g.a[J - 1][m], n2);
-        if constexpr (P == QCD_HIP_F16) n2 *= (double)g.nj[J - 1] * (double)g.nj[J - 1];
-        last[0] = n2;
-      }
-    }
-    constexpr unsigned lanes = 64 / NV;   // lanes per value after the scatter
-    const double t = wave_sum_scatter<NV>(v);
-    const unsigned q = 2 * (unsigned)j0 + l.lane / lanes;
-    if (l.lane % lanes == 0 && q < 2 * (unsigned)k) sums[wid][q] = t;
-  }
-  {
-    const double t = wave_sum_scatter<2>(last);
-    if (l.lane == 0) sums[wid][2 * k + 4] = t;
+      for (int i = 0; i < J; i++)
+        if (j0 + i >= k - prev && j0 + i < k) {
+          double y[2] = {0.0, 0.0};
+          if (l.valid) {
+#pragma unroll
+            for (int m = 0; m < M; m++) CH::norm2(g.a[i][m], y[0]);
+            if constexpr (P == QCD_HIP_F16) y[0] *= (double)g.nj[i] * (double)g.nj[i];
+          }
+          const double t = wave_sum_scatter<2>(y);
+          if (l.lane == 0) own[gcr_own<S> + (k - 1 - (j0 + i))] = t;
+        }
   }
   __syncthreads();
-  const unsigned nv = gcr_values(k);
+  const unsigned nv = gcr_values<S>(k);
   double *pr = part + blockIdx.y * rowsz + (size_t)blockIdx.x * nv;
   for (unsigned q = threadIdx.x; q < nv; q += BLK) {
     double t = 0.0;
@@ -453,15 +583,30 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
   }
 }
 
-// Step k's coefficients from the sums of k_gcr_dots (np workgroups), one
+// The coefficients of a block from the sums of k_gcr_dots (np workgroups), one
 // workgroup per rhs
-template <int P, bool EXACT>
+template <int P, int S>
 __global__ void __launch_bounds__(1024) k_gcr_scal(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
-                                                   const int *ids) {
+                                                   int prev, double theta, const int *ids) {
   __shared__ double sums[1024];
-  __shared__ double2 cf[kN + 2];
-  sum_parts<1024>(part + blockIdx.x * rowsz, np, gcr_values(k), sums);
-  if (threadIdx.x < 64) gcr_coefficients<P, EXACT>(scs + ids[blockIdx.x], sums, k, cf, true);
+  static_assert(gcr_values<S>(kN - S) <= 1024, "one value per lane");
+  sum_parts<1024>(part + blockIdx.x * rowsz, np, gcr_values<S>(k), sums);
+  if (threadIdx.x < 64) gcr_coefficients<P, S>(scs + ids[blockIdx.x], sums, k, prev, theta);
+}
+
+// The sums of c workgroups of k_gcr_dots each, added up behind the partial sums
+// of all np: the one workgroup of k_gcr_scal reads 0.1 TB/s.  Solves of one rhs
+// on 16^3x32, Q, GCR(32), without and with it, ms: FP64 (512 workgroups, up to
+// 253 values) 90.2, 89.1; FP32 (1024) 22.3, 20.8.
+__global__ void __launch_bounds__(256) k_gcr_sum(double *part, size_t rowsz, unsigned np, unsigned nv, unsigned c) {
+  double *row = part + blockIdx.y * rowsz;
+  const unsigned p0 = blockIdx.x * c, p1 = min(p0 + c, np);
+  for (unsigned q = threadIdx.x; q < nv; q += 256) {
+    double t = 0.0;
+#pragma unroll 8
+    for (unsigned p = p0; p < p1; p++) t += row[(size_t)p * nv + q];
+    row[(size_t)(np + blockIdx.x) * nv + q] = t;
+  }
 }
 
 // Store M chunks of a vector of precision P given in FP64 and leave in q and
@@ -515,13 +660,12 @@ __device__ __forceinline__ void chunk_store(const SpinorSet<P> &v, int j, const 
     for (int m = 0; m < M; m++) __builtin_nontemporal_store(q[m], CH::at(v, j, l.q0 + 64 * m));
 }
 
-// acc += sum of f[j] times vector j0 + j, j < cnt, J of them in flight (and
-// the next J on their way where a lane holds one chunk)
-template <int P, int M, int J>
-__device__ __forceinline__ void chunk_combine(Cx<double> (&acc)[M][Chunk<P>::kC], const SpinorSet<P> &v, int j0, int cnt,
-                                              const double2 *f, const ChunkLane<P, M> &l) {
+// acc[a] += sum of f[a kN + j] times vector j0 + j, j < cnt, J of them in flight
+// (and the next J on their way where a lane holds one chunk)
+template <int P, int S, int M, int J, bool PRE>
+__device__ __forceinline__ void chunk_combine(Cx<double> (&acc)[S][M][Chunk<P>::kC], const SpinorSet<P> &v, int j0,
+                                              int cnt, const double2 *f, const ChunkLane<P, M> &l) {
   using CH = Chunk<P>;
-  constexpr bool PRE = M == 1;
   if (!l.valid) return;
   struct Group {
     u32x4 a[J][M];
@@ -547,153 +691,101 @@ __device__ __forceinline__ void chunk_combine(Cx<double> (&acc)[M][Chunk<P>::kC]
       load(g, i0);
     }
 #pragma unroll
-    for (int i = 0; i < J; i++) {
-      double2 c = f[min(i0 + i, cnt - 1)];
-      if (i0 + i >= cnt) c = make_double2(0.0, 0.0);
-      if constexpr (P == QCD_HIP_F16) c = make_double2(c.x * (double)g.nj[i], c.y * (double)g.nj[i]);
+    for (int i = 0; i < J; i++)
 #pragma unroll
-      for (int m = 0; m < M; m++) CH::axpy(acc[m], c, g.a[i][m]);
-    }
+      for (int a = 0; a < S; a++) {
+        double2 c = f[a * kN + min(i0 + i, cnt - 1)];
+        if (i0 + i >= cnt) c = make_double2(0.0, 0.0);
+        if constexpr (P == QCD_HIP_F16) c = make_double2(c.x * (double)g.nj[i], c.y * (double)g.nj[i]);
+#pragma unroll
+        for (int m = 0; m < M; m++) CH::axpy(acc[a][m], c, g.a[i][m]);
+      }
   }
 }
 
-// w_k += sum_j coef_j w_j, then res_{k+1} = res_k + alpha w_k with the stored
-// (rounded) w_k: one pass over k + 2 vectors read and two written (k = 0: w_0
-// stays as it is).  np > 0: the step's coefficients are formed here from the
-// partial sums of np workgroups of k_gcr_dots, by every workgroup for itself in
-// the same order, and stored by the first; np = 0: k_gcr_scal has formed them.
-//
-// EXACT: w_k only, with partial sums of |w_k|^2 and <w_k, res_k> at part;
-// k_gcr_alpha and k_gcr_residual follow.  For Q in reduced precision: Q is
-// indefinite, <Q r, r> of a generic r is about |Q r| |r| / sqrt(12 V), so every
-// other step is nearly empty and the next one has |w_k|^2 of 1e-5 |Q res_k|^2
-// and less, which the difference that gcr_coefficients takes cannot give to
-// FP16 or FP32 (stagnates on 8^3x16).  D and the Schur complement have positive
-// real parts: iteration counts there equal those of the exact steps (8^3x16 and
-// 16^3x32 at kappa 0.135 and 0.139, eps 0.3, GCR(12), (32), (64)).
-template <int P, int M, int J, int BLK, bool EXACT>
-__global__ void __launch_bounds__(BLK) k_gcr_update(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, GcrScal *scs,
-                                                    const int *ids, unsigned V, double *part, size_t rowsz,
-                                                    unsigned np) {
+// w_{k+a} = v_a + sum_j coef_aj w_j, j < k + a, then res_{k+S} = res_k + sum_a
+// step_a w_{k+a} with the stored (rounded) w: one pass over k + S + 1 vectors
+// read and S + 1 written.
+template <int P, int S, int M, int J, int BLK, bool PRE>
+__global__ void __launch_bounds__(BLK) k_gcr_update(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, double theta,
+                                                    const GcrScal *scs, const int *ids, unsigned V) {
   using CH = Chunk<P>;
-  __shared__ double2 cf[kN + 2];
-  __shared__ double sums[BLK];
+  __shared__ double2 cf[S * kN], st[S + 1];
   __shared__ float mx[P == QCD_HIP_F16 && M != CH::kG ? BLK : 1];
   const int b = ids[blockIdx.y], k0 = b * n;
-  GcrScal *sc = scs + b;
-  if (np > 0) {
-    sum_parts<BLK>(part + blockIdx.y * rowsz, np, gcr_values(k), sums);
-    if (threadIdx.x < 64) gcr_coefficients<P, false>(sc, sums, k, cf, blockIdx.x == 0);
-  } else {
-    for (int j = threadIdx.x; j <= k; j += BLK) cf[j] = j < k ? sc->coef[k * kN + j] : sc->alpha[k];
-  }
+  const GcrScal *sc = scs + b;
+  for (int i = threadIdx.x; i < S * kN; i += BLK) cf[i] = sc->coef[k * kN + i];
+  if (threadIdx.x <= S) st[threadIdx.x] = threadIdx.x < S ? sc->step[threadIdx.x] : sc->take;
   __syncthreads();
-  double2 al = cf[k];
   const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
-  u32x4 w[M], r[M];
-  float nw = 0.f, nr = 0.f;
+  auto coef = [](double2 f, float nrm) {
+    return P == QCD_HIP_F16 ? scale2((double)nrm, f) : f;
+  };
+  auto load = [&](u32x4 (&c)[M], float &nrm, const SpinorSet<P> &v, int slot) {
+    nrm = l.valid ? CH::norm(v, slot, l.site()) : 0.f;
 #pragma unroll
-  for (int m = 0; m < M; m++) w[m] = r[m] = u32x4{0, 0, 0, 0};
-  if (l.valid) {
-    nw = CH::norm(W, k0 + k, l.site());
-    nr = CH::norm(Rs, k0 + k, l.site());
-#pragma unroll
-    for (int m = 0; m < M; m++) {
-      w[m] = CH::load(W, k0 + k, l.q0 + 64 * m);
-      r[m] = CH::load(Rs, k0 + k, l.q0 + 64 * m);
-    }
-  }
-  Cx<double> acc[M][CH::kC];
-  auto start = [&](const u32x4 (&q)[M], float nq) {
+    for (int m = 0; m < M; m++) c[m] = l.valid ? CH::load(v, slot, l.q0 + 64 * m) : u32x4{0, 0, 0, 0};
+  };
+  auto set = [&](Cx<double> (&x)[M][CH::kC], const u32x4 (&c)[M], float nrm) {
 #pragma unroll
     for (int m = 0; m < M; m++)
 #pragma unroll
       for (int i = 0; i < CH::kC; i++) {
-        const auto x = CH::get(q[m], i);
-        acc[m][i] = Cx<double>{(double)x.re, (double)x.im};
+        const auto y = CH::get(c[m], i);
+        x[m][i] = Cx<double>{(double)y.re, (double)y.im};
         if constexpr (P == QCD_HIP_F16) {
-          acc[m][i].re *= (double)nq;
-          acc[m][i].im *= (double)nq;
+          x[m][i].re *= (double)nrm;
+          x[m][i].im *= (double)nrm;
         }
       }
   };
-  if (k > 0) {
-    start(w, nw);
-    chunk_combine<P, M, J>(acc, W, k0, k, cf, l);
-    chunk_store<P, M>(W, k0 + k, l, acc, w, nw, mx);
-  }
-  if constexpr (EXACT) {
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
+  Cx<double> acc[S][M][CH::kC];
+  u32x4 r[M], q[S][M];
+  float nr, nq[S];
+  load(r, nr, Rs, k0 + k);
+  {
+    u32x4 c[S][M];
+    float nc[S];
 #pragma unroll
-    for (int m = 0; m < M; m++) {
-      CH::norm2(w[m], v[0]);
-      CH::dot(w[m], r[m], v[1], v[2]);
+    for (int a = 0; a < S; a++) {
+      const GcrD<P, S> v(W, Rs, k0 + k, a + 1);
+      load(c[a], nc[a], v.set, v.slot);
     }
-    if constexpr (P == QCD_HIP_F16) {
-      v[0] *= (double)nw * (double)nw;
-      v[1] *= (double)nw * (double)nr;
-      v[2] *= (double)nw * (double)nr;
-    }
-    const double t = wave_sum_scatter<4>(v);
-    __syncthreads();   // sums may still be read for the coefficients
-    if ((l.lane & 15u) == 0) sums[(threadIdx.x >> 6) * 4 + (l.lane >> 4)] = t;
-    __syncthreads();
-    if (threadIdx.x < 3) {
-      double x = 0.0;
-      for (int q = 0; q < BLK / 64; q++) x += sums[4 * q + threadIdx.x];
-      part[blockIdx.y * rowsz + (size_t)blockIdx.x * 3 + threadIdx.x] = x;
-    }
-    return;
-  }
-  start(r, nr);
-  if constexpr (P == QCD_HIP_F16) al = make_double2(al.x * (double)nw, al.y * (double)nw);
 #pragma unroll
-  for (int m = 0; m < M; m++) CH::axpy(acc[m], al, w[m]);
-  chunk_store<P, M>(Rs, k0 + k + 1, l, acc, r, nr, mx);
+    for (int a = 0; a < S; a++) {
+      set(acc[a], c[a], nc[a]);
+#pragma unroll
+      for (int m = 0; m < M; m++)
+        CH::axpy(acc[a][m], coef(make_double2(theta, 0.0), a > 0 ? nc[a - 1] : nr), a > 0 ? c[a - 1][m] : r[m]);
+    }
+  }
+  if (k > 0) chunk_combine<P, S, M, J, PRE>(acc, W, k0, k, cf, l);
+  Cx<double> res[M][CH::kC];
+  set(res, r, nr);
+  if (st[S].x != 0.0 || st[S].y != 0.0) {
+    load(r, nr, W, k0 + k - 1);
+#pragma unroll
+    for (int m = 0; m < M; m++) CH::axpy(res[m], coef(st[S], nr), r[m]);
+  }
+#pragma unroll
+  for (int a = 0; a < S; a++) {
+#pragma unroll
+    for (int c = 0; c < a; c++) {
+      const double2 f = coef(cf[a * kN + k + c], nq[c]);
+#pragma unroll
+      for (int m = 0; m < M; m++) CH::axpy(acc[a][m], f, q[c][m]);
+    }
+    chunk_store<P, M>(W, k0 + k + a, l, acc[a], q[a], nq[a], mx);
+    const double2 f = coef(st[a], nq[a]);
+#pragma unroll
+    for (int m = 0; m < M; m++) CH::axpy(res[m], f, q[a][m]);
+  }
+  chunk_store<P, M>(Rs, k0 + k + S, l, res, r, nr, mx);
 }
 
-// alpha of step k from the sums of k_gcr_update<EXACT> (np workgroups)
-__global__ void __launch_bounds__(1024) k_gcr_alpha(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
-                                                    const int *ids) {
-  __shared__ double sums[1024];
-  sum_parts<1024>(part + blockIdx.x * rowsz, np, 3, sums);
-  if (threadIdx.x == 0) {
-    GcrScal *sc = scs + ids[blockIdx.x];
-    const double w = 1.0 / sums[0];
-    if (!(w == w) || isinf(w)) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
-    sc->alpha[k] = make_double2(-w * sums[1], -w * sums[2]);
-  }
-}
-
-// res_{k+1} = res_k + alpha w_k
-template <int P, int M, int BLK>
-__global__ void __launch_bounds__(BLK) k_gcr_residual(SpinorSet<P> W, SpinorSet<P> Rs, int n, int k, const GcrScal *scs,
-                                                      const int *ids, unsigned V) {
-  using CH = Chunk<P>;
-  __shared__ double2 f[2];
-  __shared__ float mx[P == QCD_HIP_F16 && M != CH::kG ? BLK : 1];
-  const int b = ids[blockIdx.y], k0 = b * n;
-  if (threadIdx.x == 0) {
-    f[0] = make_double2(1.0, 0.0);
-    f[1] = scs[b].alpha[k];
-  }
-  __syncthreads();
-  const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
-  Cx<double> acc[M][CH::kC];
-#pragma unroll
-  for (int m = 0; m < M; m++)
-#pragma unroll
-    for (int i = 0; i < CH::kC; i++) acc[m][i] = Cx<double>{0.0, 0.0};
-  chunk_combine<P, M, 1>(acc, Rs, k0 + k, 1, f, l);
-  chunk_combine<P, M, 1>(acc, W, k0 + k, 1, f + 1, l);
-  u32x4 q[M];
-  float nrm;
-  chunk_store<P, M>(Rs, k0 + k + 1, l, acc, q, nrm, mx);
-}
-
-// e_b = sum_j beta_j res_j, times |r_b| (the norm the inner source was
+// e_b = sum_j beta_j d_j, times |r_b| (the norm the inner source was
 // divided by) when scaled
-template <int P, int M, int J, int BLK>
+template <int P, int M, int J, int BLK, bool PRE>
 __global__ void __launch_bounds__(BLK) k_solution(SpinorSet<P> Rs, int n, const GcrScal *sc, SpinorSet<P> E,
                                                   const int *ids, unsigned V, int scaled) {
   using CH = Chunk<P>;
@@ -704,42 +796,29 @@ __global__ void __launch_bounds__(BLK) k_solution(SpinorSet<P> Rs, int n, const 
   for (int j = threadIdx.x; j < n; j += BLK) bt[j] = make_double2(sc[b].beta[j].x * f, sc[b].beta[j].y * f);
   __syncthreads();
   const ChunkLane<P, M> l = ChunkLane<P, M>::of(V);
-  Cx<double> acc[M][CH::kC];
+  Cx<double> acc[1][M][CH::kC];
 #pragma unroll
   for (int m = 0; m < M; m++)
 #pragma unroll
-    for (int i = 0; i < CH::kC; i++) acc[m][i] = Cx<double>{0.0, 0.0};
-  chunk_combine<P, M, J>(acc, Rs, b * n, n, bt, l);
+    for (int i = 0; i < CH::kC; i++) acc[0][m][i] = Cx<double>{0.0, 0.0};
+  chunk_combine<P, 1, M, J, PRE>(acc, Rs, b * n, n, bt, l);
   u32x4 q[M];
   float nrm;
-  chunk_store<P, M>(E, b, l, acc, q, nrm, mx);
+  chunk_store<P, M>(E, b, l, acc[0], q, nrm, mx);
 }
 
-// The cycle's solution sum_k (-alpha_k) p_k with p_k = res_k + sum_j coef[k][j]
-// p_j (A p_k = w_k) as sum_j beta_j res_j: beta_j = -alpha_j + sum_{k > j}
-// beta_k coef[k][j], from the last step down (lane j holds beta_j).  keep_q1
-// drops the first step's -alpha_0 as invert.c:50-53 does.
-// np > 0: the last step's coefficients are formed here first.
-template <int P>
-__global__ void __launch_bounds__(256) k_scal_beta(GcrScal *scs, int n, int keep_q1, const int *ids,
-                                                   const double *part, size_t rowsz, unsigned np) {
-  __shared__ double sums[256];
-  __shared__ double2 cf[kN + 2];
+// The cycle's solution sum_k (-alpha_k) p_k with p_k = d_k + sum_j coef[k][j]
+// p_j (A p_k = w_k) as sum_j beta_j d_j: beta_j = -alpha_j + sum_{k > j} beta_k
+// coef[k][j], from the last step down (lane j holds beta_j).  keep_q1 drops the
+// first step's -alpha_0 as invert.c:50-53 does.
+__global__ void __launch_bounds__(64) k_scal_beta(GcrScal *scs, int n, int keep_q1, const int *ids) {
   GcrScal *sc = scs + ids[blockIdx.x];
   const int j = threadIdx.x;
-  if (np > 0) sum_parts<256>(part + blockIdx.x * rowsz, np, gcr_values(n - 1), sums);
-  if (j >= 64) return;
-  if (np > 0) gcr_coefficients<P, false>(sc, sums, n - 1, cf, true);
-  // (the last step's coefficients may just have been stored by other lanes)
-  auto coef = [&](int k) { return np > 0 && k == n - 1 ? cf[j] : sc->coef[k * kN + j]; };
   double2 b = make_double2(0.0, 0.0);
-  if (j < n && !(j == 0 && keep_q1)) {
-    const double2 al = np > 0 && j == n - 1 ? cf[j] : sc->alpha[j];
-    if (!(np > 0 && j == n - 2 && cf[n].x != 0.0)) b = make_double2(-al.x, -al.y);
-  }
+  if (j < n && !(j == 0 && keep_q1)) b = make_double2(-sc->alpha[j].x, -sc->alpha[j].y);
 #pragma unroll 8
   for (int k = n - 1; k > 0; k--) {
-    const double2 c = j < k ? coef(k) : make_double2(0.0, 0.0);
+    const double2 c = j < k ? sc->coef[k * kN + j] : make_double2(0.0, 0.0);
     const double2 p = cmul2(make_double2(__shfl(b.x, k, 64), __shfl(b.y, k, 64)), c);
     if (j < k) b = make_double2(b.x + p.x, b.y + p.y);
   }
@@ -829,8 +908,8 @@ struct qcd_hip_solver_s {
   hipStream_t stream = nullptr;     // the solver's own stream
   qcd_hip_field g64 = nullptr;      // caller's FP64 gauge field (not owned)
   qcd_hip_field gin = nullptr;      // inner-precision copy (owned unless F64)
-  qcd_hip_field Rs = nullptr;       // n*B search directions res_j (inner precision)
-  qcd_hip_field Ws = nullptr;       // n*B vectors w_j = A res_j (inner precision)
+  qcd_hip_field Rs = nullptr;       // n*B directions d_j (inner precision)
+  qcd_hip_field Ws = nullptr;       // n*B orthogonal vectors w_j (inner precision)
   qcd_hip_field E = nullptr;        // B inner corrections (inner precision)
   qcd_hip_field r64 = nullptr;      // B FP64 residuals (not allocated with split_res)
   // FP16-inner even-odd: the true residual is stored straight into the FP16
@@ -870,53 +949,51 @@ struct qcd_hip_solver_s {
 
 namespace {
 
-// Work split of the GCR vector kernels: M chunks per lane, J vectors in flight,
-// BLK lanes per workgroup.  Chosen by the vector length alone, so that a
-// right-hand side gets the same sums alone and in any batch.
+// Work split of the GCR vector kernels: M chunks per lane, J vectors in flight
+// (PRE: and the next J on their way), BLK lanes per workgroup.  Chosen by the
+// vector length alone, so that a right-hand side gets the same sums alone and in
+// any batch.
 //   Short vectors: one chunk per lane, so that they still put a few wavefronts
 //     on every SIMD (FP16: a tile's three wavefronts share a workgroup, which
-//     finds the site norms).  Solves of 8^3x16, GCR(12), ms, Short against
-//     long: FP64 2.33 / 2.60, FP32 of 3 rhs 2.32 / 2.50, FP16 1.76 / 2.00 and
-//     of 12 rhs 2.66 / 2.62; FP64 without even-odd, GCR(32) 17.1 / 23.2.  From
-//     8000 sites up a batch of 12 FP16 rhs loses 16% with it, 3 FP32 rhs
-//     nothing, one rhs gains up to 11%.
-//   Long ones: one site per lane and one or two vectors in flight, which leaves
-//     the most wavefronts to hide the loads: FP32 on 16^3x32, Q, GCR(32), with
-//     half a site and four vectors 124.2 ms, a site and one vector 120.8; one
-//     FP64 rhs 211.8 with a third of a site and four vectors in the update,
-//     205.9; 12 FP16 rhs on 24^3x48 with four vectors in both 135.0, 132.3.  The
-//     kernels run at 6.0-6.7 TB/s, the rate of the fabric: running the update
-//     through the sites backwards, which would find the dots' last vectors in
-//     the last-level cache, changes nothing.
-template <int M_, int J_, int BLK_>
+//     finds the site norms).  Solves, ms, Short against long: 8^3x16 even-odd,
+//     one FP64 rhs, GCR(32) 1.31 / 1.70, three FP32, GCR(16) 0.98 / 1.05, one
+//     FP16, GCR(12) 1.13 / 1.21, twelve, GCR(32) 3.84 / 3.88.  9216 sites: FP64
+//     1.55 / 1.81, FP32 1.28 / 1.30, FP16 1.22 / 1.30 but twelve 5.83 / 5.60;
+//     16 128 sites: FP64 and FP32 2% slower.
+//   Long ones: what measured best, us per launch (12 FP16 rhs, GCR(12), 24^3x48;
+//     one FP64 rhs, GCR(32), 16^3x32; three FP32, GCR(16), 16^3x24, even-odd).
+//     FP16 dots: (3, 1, 256, PRE) 396, two vectors in flight 424 to 513, 512
+//     lanes 515, a third of a site 529; they are bound by the FP64 additions of
+//     the products.  FP16 update: a third of a site, 192 lanes 480, 384 lanes
+//     594, two vectors in flight 519, a whole site (its four FP64 accumulators
+//     leave one wavefront per SIMD) 746.  FP64 dots: half a site 71, a whole one
+//     115; update 96 and 97 to 100.  FP32 dots: half a site, one vector, 256
+//     lanes 29.4, two vectors 32.9, 512 lanes 37.6; update 37.2 to 38.9.
+template <int M_, int J_, int BLK_, bool PRE_>
 struct GcrShape {
   static constexpr int M = M_, J = J_, BLK = BLK_;
+  static constexpr bool PRE = PRE_;
 };
 template <int P>
 struct GcrShapes;
 template <>
 struct GcrShapes<QCD_HIP_F16> {
-  using Short = GcrShape<1, 8, 192>;
-  using Dots = GcrShape<3, 2, 512>;
-  using Update = GcrShape<3, 1, 256>;
+  using Short = GcrShape<1, 2, 192, true>;
+  using Dots = GcrShape<3, 1, 256, true>;
+  using Update = GcrShape<1, 1, 192, true>;
 };
 template <>
 struct GcrShapes<QCD_HIP_F32> {
-  using Short = GcrShape<1, 8, 256>;
-  using Dots = GcrShape<6, 1, 512>;
-  using Update = GcrShape<6, 1, 256>;
+  using Short = GcrShape<1, 4, 256, true>;
+  using Dots = GcrShape<3, 1, 256, false>;
+  using Update = GcrShape<3, 1, 256, false>;
 };
 template <>
 struct GcrShapes<QCD_HIP_F64> {
-  using Short = GcrShape<1, 8, 256>;
-  using Dots = GcrShape<12, 1, 512>;
-  using Update = GcrShape<12, 1, 256>;
+  using Short = GcrShape<1, 4, 256, true>;
+  using Dots = GcrShape<6, 1, 512, false>;
+  using Update = GcrShape<6, 1, 256, false>;
 };
-// Up to this many workgroups per rhs the update forms the coefficients from the
-// partial sums itself (8^3x16: 64 of them); past it every one of its workgroups
-// would read too many (12 FP16 rhs of 12^3x24, 324 of them: solve 9.6 ms with
-// k_gcr_scal, 10.2 without).
-constexpr unsigned kGcrParts = 128;
 template <typename SH>
 unsigned gcr_blocks(int prec, long V) {
   const long kG = 12 * (long)spinor_comp_bytes(prec) / 16;
@@ -924,7 +1001,7 @@ unsigned gcr_blocks(int prec, long V) {
   return (unsigned)((waves + SH::BLK / 64 - 1) / (SH::BLK / 64));
 }
 template <int P>
-constexpr bool gcr_short(long V) { return V <= (P == QCD_HIP_F16 ? 4096 : 8192); }
+constexpr bool gcr_short(long V) { return V <= (P == QCD_HIP_F16 ? 4096 : 12288); }
 // workgroups per rhs of the dots over vectors of V sites
 template <int P>
 unsigned gcr_parts_of(long V) {
@@ -946,64 +1023,77 @@ void gcr_launch(long V, int count, F f) {
   else call(typename G::Update{});
 }
 
+// More partial sums than kGcrParts are added up in up to kGcrSums groups first.
+constexpr unsigned kGcrParts = 256, kGcrSums = 64;
+
+// Steps k .. k + ST - 1 of the cycle (prev: of the block before), the hops of
+// matvec(out, out slot, in slot) included
+template <int P, int ST, typename F>
+int gcr_block(qcd_hip_solver_s *S, int count, int k, int prev, double theta, hipStream_t st, F matvec) {
+  const int n = S->prm.n_restart;
+  const unsigned V = S->Vi;
+  SpinorSet<P> Rs = SpinorSet<P>::of(S->Rs), Ws = SpinorSet<P>::of(S->Ws);
+  for (int a = 0; a < ST; a++) {
+    const bool last = a == ST - 1;
+    QH_TRY(matvec(last ? S->Ws : S->Rs, last ? k + a : k + a + 1, k + a));
+  }
+  gcr_launch<P, true>(V, count, [&](auto sh, dim3 grid) {
+    using SH = decltype(sh);
+    k_gcr_dots<P, ST, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, prev, S->ids, V, S->part,
+                                                                       S->rowsz);
+    unsigned np = grid.x;
+    const double *part = S->part;
+    if (np > kGcrParts) {
+      const unsigned nv = gcr_values<ST>(k), c = std::max(32u, (np + kGcrSums - 1) / kGcrSums), g = (np + c - 1) / c;
+      k_gcr_sum<<<dim3(g, (unsigned)count), 256, 0, st>>>(S->part, S->rowsz, np, nv, c);
+      part += (size_t)np * nv;
+      np = g;
+    }
+    k_gcr_scal<P, ST><<<count, 1024, 0, st>>>(S->sc, part, S->rowsz, np, k, prev, theta, S->ids);
+  });
+  if (k + ST < n)   // the last w and the residual after them are not used
+    gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+      using SH = decltype(sh);
+      k_gcr_update<P, ST, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, theta, S->sc, S->ids, V);
+    });
+  return 0;
+}
+
 template <int P>
 int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream_t st) {
   const int n = S->prm.n_restart;
   const unsigned V = S->Vi;
   const int epi = S->use_q ? EPI_Q : EPI_D;
   const double m = 1.0 / (2.0 * kappa) - 4.0;
-  SpinorSet<P> Rs = SpinorSet<P>::of(S->Rs), Ws = SpinorSet<P>::of(S->Ws), E = SpinorSet<P>::of(S->E);
-  // coefficients formed by the update kernel itself where the sums are few
-  const bool exact = P != QCD_HIP_F64 && S->use_q;
-  const unsigned np = !exact && gcr_parts(P, V) <= kGcrParts ? gcr_parts(P, V) : 0;
-  for (int k = 0; k < n; k++) {
+  SpinorSet<P> Rs = SpinorSet<P>::of(S->Rs), E = SpinorSet<P>::of(S->E);
+  // Q, and the local term left out of D and of the Schur complement
+  const double theta = S->use_q ? 0.0 : m + 4.0;
+  // out = (A - theta) Rs[slot ri]
+  auto matvec = [&](qcd_hip_field out, int ro, int ri) -> int {
     if (S->prm.eo) {
-      // w_k = D^ res_k = M res_k - H_oe (M^-1 H_eo res_k)
-      QH_TRY(eo_launch(EO_MINV, false, S->te, 0, 1, S->Rs, k, n, S->gin, nullptr, 0, 0, S->ids, count, m, mu, 0,
+      // D^ r = M r - H_oe (M^-1 H_eo r)
+      QH_TRY(eo_launch(EO_MINV, false, S->te, 0, 1, S->Rs, ri, n, S->gin, nullptr, 0, 0, S->ids, count, m, mu, 0,
                        nullptr, st, nullptr));
-      QH_TRY(eo_launch(EO_SCHUR, false, S->Ws, k, n, S->te, 0, 1, S->gin, S->Rs, k, n, S->ids, count, m, mu, 1,
-                       nullptr, st, nullptr));
-    } else {
-      QH_TRY(dslash_launch_batch(epi, false, S->Ws, k, n, S->Rs, k, n, S->gin, nullptr, 0, 0, S->ids, count, m, mu,
-                                 nullptr, st, nullptr));
+      return eo_launch(EO_SCHUR, false, out, ro, n, S->te, 0, 1, S->gin, S->Rs, ri, n, S->ids, count, m - theta, mu, 1,
+                       nullptr, st, nullptr);
     }
-    gcr_launch<P, true>(V, count, [&](auto sh, dim3 grid) {
-      using SH = decltype(sh);
-      auto dots = k_gcr_dots<P, SH::M, SH::J, SH::BLK, false>;
-      auto scal = k_gcr_scal<P, false>;
-      if constexpr (P != QCD_HIP_F64)
-        if (exact) {
-          if (k == 0) return;
-          dots = k_gcr_dots<P, SH::M, SH::J, SH::BLK, true>;
-          scal = k_gcr_scal<P, true>;
-        }
-      dots<<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->ids, V, S->part, S->rowsz);
-      if (!np) scal<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
-    });
-    if (exact)
-      gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
-        using SH = decltype(sh);
-        if constexpr (P != QCD_HIP_F64) {
-          k_gcr_update<P, SH::M, SH::J, SH::BLK, true><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V,
-                                                                                 S->part, S->rowsz, 0);
-          k_gcr_alpha<<<count, 1024, 0, st>>>(S->sc, S->part, S->rowsz, grid.x, k, S->ids);
-          if (k + 1 < n) k_gcr_residual<P, SH::M, SH::BLK><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V);
-        }
-      });
-    else if (k + 1 < n)   // the last w_k and the residual after it are not used
-      gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
-        using SH = decltype(sh);
-        k_gcr_update<P, SH::M, SH::J, SH::BLK, false><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, S->sc, S->ids, V, S->part,
-                                                                                S->rowsz, np);
-      });
+    return dslash_launch_batch(epi, false, out, ro, n, S->Rs, ri, n, S->gin, nullptr, 0, 0, S->ids, count, m - theta,
+                               mu, nullptr, st, nullptr);
+  };
+  for (int k = 0, prev = 0; k < n; k += prev) {
+    const int left = n - k;
+    if (left >= 4) QH_TRY((gcr_block<P, 4>(S, count, k, prev, theta, st, matvec)));
+    else if (left >= 2) QH_TRY((gcr_block<P, 2>(S, count, k, prev, theta, st, matvec)));
+    else QH_TRY((gcr_block<P, 1>(S, count, k, prev, theta, st, matvec)));
+    prev = left >= 4 ? 4 : left >= 2 ? 2 : 1;
   }
-  k_scal_beta<P><<<count, 256, 0, st>>>(S->sc, n, S->prm.keep_q1, S->ids, S->part, S->rowsz, np);
+  k_scal_beta<<<count, 64, 0, st>>>(S->sc, n, S->prm.keep_q1, S->ids);
   // mixed even-odd solves take the correction scaled by |r^_o| (the outer
   // step adds it as it is); the others scale it where they add it
   const int scaled = S->prm.eo && S->prm.inner_prec != QCD_HIP_F64;
   gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
     using SH = decltype(sh);
-    k_solution<P, SH::M, SH::J, SH::BLK><<<grid, SH::BLK, 0, st>>>(Rs, n, S->sc, E, S->ids, V, scaled);
+    k_solution<P, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Rs, n, S->sc, E, S->ids, V, scaled);
   });
   QH_CHECK(hipGetLastError());
   return 0;
@@ -1206,9 +1296,10 @@ namespace qcdhip {
 // sites, and the z-march grids).
 static size_t solver_row(qcd_hip_lattice lat, long Vi, const qcd_hip_solver_params *prm) {
   const size_t parts = gcr_parts(prm->inner_prec, Vi);
-  // (k_gcr_update<EXACT> has three values per workgroup and at most six times
-  // the dots' workgroups)
-  const size_t dots = std::max((size_t)gcr_values(prm->n_restart - 1), (size_t)18) * parts;
+  const int n = prm->n_restart;
+  const size_t nv = std::max({gcr_values<4>(std::max(n - 4, 0)), gcr_values<2>(std::max(n - 2, 0)),
+                              gcr_values<1>(n - 1)});
+  const size_t dots = (parts + kGcrSums) * nv;
   return std::max(dots, std::max((size_t)grid_for(lat->V) + 64, (size_t)dslash_grid_bound(lat)));
 }
 
