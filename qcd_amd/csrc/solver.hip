@@ -756,12 +756,14 @@ __global__ void __launch_bounds__(BLK) k_gcr_update(SpinorSet<P> W, SpinorSet<P>
       set(acc[a], c[a], nc[a]);
 #pragma unroll
       for (int m = 0; m < M; m++)
-        CH::axpy(acc[a][m], coef(make_double2(theta, 0.0), a > 0 ? nc[a - 1] : nr), a > 0 ? c[a - 1][m] : r[m]);
+        if (a > 0) CH::axpy(acc[a][m], coef(make_double2(theta, 0.0), nc[a - 1]), c[a - 1][m]);
     }
   }
   if (k > 0) chunk_combine<P, S, M, J, PRE>(acc, W, k0, k, cf, l);
   Cx<double> res[M][CH::kC];
   set(res, r, nr);
+#pragma unroll
+  for (int m = 0; m < M; m++) CH::axpy(acc[0][m], coef(make_double2(theta, 0.0), nr), r[m]);
   if (st[S].x != 0.0 || st[S].y != 0.0) {
     load(r, nr, W, k0 + k - 1);
 #pragma unroll
@@ -964,11 +966,12 @@ namespace {
 //     one FP64 rhs, GCR(32), 16^3x32; three FP32, GCR(16), 16^3x24, even-odd).
 //     FP16 dots: (3, 1, 256, PRE) 396, two vectors in flight 424 to 513, 512
 //     lanes 515, a third of a site 529; they are bound by the FP64 additions of
-//     the products.  FP16 update: a third of a site, 192 lanes 480, 384 lanes
-//     594, two vectors in flight 519, a whole site (its four FP64 accumulators
-//     leave one wavefront per SIMD) 746.  FP64 dots: half a site 71, a whole one
-//     115; update 96 and 97 to 100.  FP32 dots: half a site, one vector, 256
-//     lanes 29.4, two vectors 32.9, 512 lanes 37.6; update 37.2 to 38.9.
+//     the products.  FP16 update: a third of a site, 192 lanes 501 (four
+//     wavefronts per SIMD; with six registers more, three, 652), 384 lanes 594,
+//     two vectors in flight 519, a whole site (its four FP64 accumulators leave
+//     one wavefront per SIMD) 746.  FP64 dots: half a site 71, a whole one 115;
+//     update 96 and 97 to 100.  FP32 dots: half a site, one vector, 256 lanes
+//     29.4, two vectors 32.9, 512 lanes 37.6; update 37.2 to 38.9.
 template <int M_, int J_, int BLK_, bool PRE_>
 struct GcrShape {
   static constexpr int M = M_, J = J_, BLK = BLK_;
