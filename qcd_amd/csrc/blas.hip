@@ -240,7 +240,7 @@ static int propagator_copy(qcd_hip_field f, int r0, double *prop, bool up) {
   hipStream_t st = ctx()->stream;
   const dim3 grid((unsigned)grid_for(V), 12);
   int rc = 0;
-  if (up && hipMemcpyAsync(buf, prop, bytes, hipMemcpyHostToDevice, st) != hipSuccess) rc = 2;
+  if (up && host_copy(buf, prop, bytes, true, st) != hipSuccess) rc = 2;
   if (!rc) {
     switch (f->prec) {
       case QCD_HIP_F64:
@@ -258,7 +258,7 @@ static int propagator_copy(qcd_hip_field f, int r0, double *prop, bool up) {
     }
     if (hipGetLastError() != hipSuccess) rc = 2;
   }
-  if (!rc && !up && hipMemcpyAsync(prop, buf, bytes, hipMemcpyDeviceToHost, st) != hipSuccess) rc = 2;
+  if (!rc && !up && host_copy(buf, prop, bytes, false, st) != hipSuccess) rc = 2;
   if (hipStreamSynchronize(st) != hipSuccess) rc = 2;
   dev_free(buf, bytes);
   if (rc) set_error("propagator %s: device error", up ? "upload" : "download");

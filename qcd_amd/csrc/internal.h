@@ -68,6 +68,8 @@ Context *ctx();                       // current context (initialised on first u
 // fields, tuning table) when several host threads drive separate streams.
 std::recursive_mutex &state_mutex();
 int ensure_init();
+// copy between device and pageable host memory (up: to the device), on st
+hipError_t host_copy(void *dev, void *host, size_t bytes, bool up, hipStream_t st);
 int dev_alloc(void **p, size_t bytes);
 void dev_free(void *p, size_t bytes);
 int gauge_create_unfilled(qcd_hip_field *f, qcd_hip_lattice lat);
