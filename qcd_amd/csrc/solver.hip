@@ -7,8 +7,8 @@
 // operator A = Q = i g5 D (as invert.c) or A = D.  For A = Q the system solved
 // is Q x = i g5 b, i.e. D x = b, so the residual is ||b - D x|| either way.
 //
-// GCR's steps are taken in blocks of S = 4 (2 and 1 for the last ones of a
-// cycle), from residual res_k: the operator S times, then
+// GCR's steps are taken in blocks of S = 8 (FP16: 4; then 4, 2 and 1 for the last
+// ones of a cycle), from residual res_k: the operator S times, then
 //   k_gcr_dots:    the S new vectors with the earlier w_j, j < k, and with each
 //                  other (reads k + S + 1 vectors)
 //   k_gcr_scal:    coef and alpha of the S steps
@@ -45,7 +45,7 @@ int eo_scale64(qcd_hip_lattice full, qcd_hip_field in, qcd_hip_field out, const 
 qcd_hip_lattice eo_half_lattice(qcd_hip_lattice full);
 
 constexpr int kN = kMaxKrylov;
-constexpr int kSteps = 4;   // most GCR steps of one block
+constexpr int kSteps = 8;   // most GCR steps of one block
 
 // The coefficients of one right-hand side's GCR cycle: w_k = A d_k + sum_j
 // coef[k][j] w_j, and the residual after step k is the one before + alpha[k] w_k.
@@ -226,8 +226,9 @@ __device__ __forceinline__ double wave_sum_scatter(double (&v)[NV]) {
 }
 
 // out[i] = x[i] summed over the wavefront, i < min(NX, used), NP at a time
-template <int NP, int NX>
+template <int NP_, int NX>
 __device__ __forceinline__ void wave_reduce(const double (&x)[NX], double *out, int used) {
+  constexpr int NP = NP_ < 16 ? NP_ : 16;
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < NX; i += NP) {
@@ -305,9 +306,12 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
 // GCR(n).  The S vectors are projected against the
 // w_j, j < k, in one pass over them and formed in a second one, where single
 // steps take 2 S passes, and these passes are what a cycle spends its time on
-// (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2
-// and 4, ms: one FP64 rhs, Q, GCR(32) on 16^3x32 204, 126, 87; 12 FP16 rhs,
-// GCR(12) on 24^3x48 132, 107, 98, on 16^3x32 21.0, 16.9, 15.5.
+// (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2, 4
+// and 8, ms: one FP64 rhs, Q, GCR(32) on 16^3x32 204, 126, 87, 69; one FP32 rhs
+// 4: 20.8, 8: 17.3; 12 FP16 rhs, GCR(12) on 24^3x48 132, 107, 96, 97, on 16^3x32
+// 21.0, 16.9, 15.0, 16.0.  FP16 stays at 4: its dots are bound by arithmetic, which
+// blocks do not save, and eight steps carry up to twice the rounding of single
+// ones into long cycles.
 //
 // theta is the local term m + 4 of D and of the Schur complement (0 for Q): the
 // d_a are then, but for factors, the residuals of Richardson's iteration, about
@@ -360,101 +364,108 @@ __device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.
 // itself, and the next block takes the difference (undo) out again.
 constexpr double kKeep = 0.5;
 template <int P, int S>
-__device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, int prev, double theta) {
-  const int j = threadIdx.x;
+__device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, int prev, double theta,
+                                                 double *tot) {
+  const int l = threadIdx.x;
   const double *own = sums + 2 * S * k, *wn = own + gcr_own<S>;
-  const double r2 = own[0] - (k > 0 ? norm2(sc->undo) * wn[0] : 0.0);
+  const double2 undo = k > 0 ? sc->undo : make_double2(0.0, 0.0);
+  const double r2 = own[0] - (k > 0 ? norm2(undo) * wn[0] : 0.0);
   const bool stop = k > 0 && (sc->stop || r2 > 4.0 * sc->rmin);
-  constexpr int NV = S * S > 1 ? S * S : 2;
-  double e[NV] = {};   // what the w_j take of the v_a's Gram matrix
-  double2 d[S] = {};
-  if (j < k) {
-    double w;
-    w = sc->w2inv[j];
-    if (j >= k - prev && w > 0.0) {   // as stored
-      const double x = wn[k - 1 - j];
-      w = x > 0.0 ? 1.0 / x : 0.0;
-      sc->w2inv[j] = w;
-    }
+  // <w_j, v_a>
+  auto wv = [&](int j, int a) {
+    const double *x = sums + 2 * (S * j + a);
+    double2 d = make_double2(x[0], x[1]);
+    if (a > 0) d = cadd2(d, make_double2(theta * x[-2], theta * x[-1]));
+    else if (j == k - 1) d = cadd2(d, scale2(-theta * wn[0], undo));   // <w_j, res_k> = 0
+    return d;
+  };
+  // what the w_j take of the v_a's Gram matrix: tot, indexed as the sums are
+  {
+    double w = 0.0;
+    double2 d[S] = {};
+    if (l < k) {
+      w = sc->w2inv[l];
+      if (l >= k - prev && w > 0.0) {   // as stored
+        const double x = wn[k - 1 - l];
+        w = x > 0.0 ? 1.0 / x : 0.0;
+        sc->w2inv[l] = w;
+      }
 #pragma unroll
-    for (int a = S - 1; a >= 0; a--) {
-      const double *x = sums + 2 * (S * j + a);
-      d[a] = make_double2(x[0], x[1]);
-      if (a > 0) d[a] = cadd2(d[a], make_double2(theta * x[-2], theta * x[-1]));
-      else if (j == k - 1) d[0] = cadd2(d[0], scale2(-theta * wn[0], sc->undo));   // <w_j, res_k> = 0
+      for (int a = 0; a < S; a++) {
+        d[a] = wv(l, a);
+        sc->coef[(k + a) * kN + l] = scale2(-w, d[a]);
+      }
     }
 #pragma unroll
     for (int a = 0; a < S; a++) {
-      sc->coef[(k + a) * kN + j] = scale2(-w, d[a]);
+      double e[2 * S] = {};
 #pragma unroll
-      for (int b = 0; b < a; b++) {
-        const double2 x = cmul2(conj2(d[b]), d[a]);
-        e[a * a + 2 * b] = w * x.x;
-        e[a * a + 2 * b + 1] = w * x.y;
+      for (int c = 0; c < a; c++) {
+        const double2 x = cmul2(conj2(d[c]), d[a]);
+        e[2 * c] = w * x.x;
+        e[2 * c + 1] = w * x.y;
       }
-      e[a * a + 2 * a] = w * norm2(d[a]);
+      e[2 * a] = w * norm2(d[a]);
+      wave_reduce<2 * S>(e, tot + a * a, 2 * a + 1);
     }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
-  const double t = wave_sum_scatter<NV>(e);
-  // <d_b, d_a>
-  auto dd = [&](int b, int a) {
-    if (a == b) return make_double2(own[a * a + 2 * a], 0.0);
-    const double *x = b < a ? own + a * a + 2 * b : own + b * b + 2 * a;
-    return make_double2(x[0], b < a ? x[1] : -x[1]);
+  // <x_b, x_a> from a table of the lower triangle
+  auto entry = [](const double *x, int b, int a) {
+    if (a == b) return make_double2(x[a * a + 2 * a], 0.0);
+    return b < a ? make_double2(x[a * a + 2 * b], x[a * a + 2 * b + 1])
+                 : make_double2(x[b * b + 2 * a], -x[b * b + 2 * a + 1]);
   };
-  // <v_b, v_a>, v_a = d_{a+1} + theta d_a
-  auto vv = [&](int b, int a) {
-    return cadd2(cadd2(dd(b + 1, a + 1), scale2(theta, cadd2(dd(b + 1, a), dd(b, a + 1)))),
-                 scale2(theta * theta, dd(b, a)));
-  };
-  double2 L[S][S], g[S][S], R[S];
-  double wi[S], rest = r2;
+  // lane l < S S holds G = <v_i, v_j>, and R = <v_j, res_k>
+  const int i = l / S % S, j = l % S;
+  const double2 full = cadd2(cadd2(entry(own, i + 1, j + 1),
+                                   scale2(theta, cadd2(entry(own, i + 1, j), entry(own, i, j + 1)))),
+                             scale2(theta * theta, entry(own, i, j)));
+  const double2 x = entry(tot, i, j);
+  double2 G = make_double2(full.x - x.x, full.y - x.y);
+  double2 R = cadd2(entry(own, j + 1, 0), scale2(theta, entry(own, j, 0)));
+  if (k > 0) R = cadd2(R, cmul2(undo, conj2(wv(k - 1, j))));   // res_k = d_0 + undo w_{k-1}
+  double rest = r2, w = 0.0;
+  double2 al = make_double2(0.0, 0.0);
   bool bad = false;
 #pragma unroll
   for (int a = 0; a < S; a++) {
-    const double n = vv(a, a).x;
-    double N = n - __shfl(t, (a * a + 2 * a) * (64 / NV), 64);
-    R[a] = cadd2(dd(a + 1, 0), scale2(theta, dd(a, 0)));
-    if (k > 0)   // res_k = d_0 + undo w_{k-1}
-      R[a] = cadd2(R[a], cmul2(sc->undo, make_double2(__shfl(d[a].x, k - 1, 64), -__shfl(d[a].y, k - 1, 64))));
-#pragma unroll
-    for (int b = 0; b < a; b++) {
-      const double2 x = vv(b, a);
-      L[a][b] = make_double2(x.x - __shfl(t, (a * a + 2 * b) * (64 / NV), 64),
-                             x.y - __shfl(t, (a * a + 2 * b + 1) * (64 / NV), 64));   // <w_{k+b}, v_a>
-#pragma unroll
-      for (int c = 0; c < b; c++) L[a][b] = cadd2(L[a][b], cmul2(conj2(g[b][c]), L[a][c]));
-      g[a][b] = scale2(-wi[b], L[a][b]);
-      N -= wi[b] * norm2(L[a][b]);
-      R[a] = cadd2(R[a], cmul2(conj2(g[a][b]), R[b]));
-      if (j == 0) sc->coef[(k + a) * kN + k + b] = g[a][b];
-    }
-    wi[a] = N > gcr_floor<P>() * n ? 1.0 / N : 0.0;
+    const int o = a * S;   // lanes of row a: <w_{k+a}, v_j>
+    const double N = __shfl(G.x, o + a, 64), n = __shfl(full.x, o + a, 64);
+    const double2 Gj = make_double2(__shfl(G.x, o + j, 64), __shfl(G.y, o + j, 64));
+    const double2 Gi = make_double2(__shfl(G.x, o + i, 64), __shfl(G.y, o + i, 64));
+    const double2 Ra = make_double2(__shfl(R.x, a, 64), __shfl(R.y, a, 64));
+    w = N > gcr_floor<P>() * n ? 1.0 / N : 0.0;
     bad = bad || !(N == N) || isinf(N) || (a == 0 && !(n > 0.0));
-    rest -= wi[a] * norm2(R[a]);
-    if (j == 0) {
-      sc->w2inv[k + a] = wi[a];
-      sc->alpha[k + a] = sc->step[a] = stop ? make_double2(0.0, 0.0) : scale2(-wi[a], R[a]);
+    rest -= w * norm2(Ra);
+    al = scale2(-w, Ra);
+    if (l == 0) {
+      sc->w2inv[k + a] = w;
+      sc->alpha[k + a] = sc->step[a] = stop ? make_double2(0.0, 0.0) : al;
+    }
+    if (j > a) {
+      if (l < S) sc->coef[(k + j) * kN + k + a] = scale2(-w, Gj);
+      R = cadd2(R, scale2(-w, cmul2(conj2(Gj), Ra)));
+      if (i > a) G = cadd2(G, scale2(-w, cmul2(conj2(Gi), Gj)));
     }
   }
-  if (j == 0) {
+  if (l == 0) {
     if (!stop && bad) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
     if (stop)
-      for (int i = 1; i <= prev; i++) sc->alpha[k - i] = make_double2(0.0, 0.0);
+      for (int q = 1; q <= prev; q++) sc->alpha[k - q] = make_double2(0.0, 0.0);
     sc->rmin = k > 0 ? fmin(sc->rmin, r2) : r2;
     sc->stop = stop;
-    // res_k as stored less the last block's undo
-    sc->take = k > 0 ? sc->undo : make_double2(0.0, 0.0);
-    const double2 al = scale2(-wi[S - 1], R[S - 1]);
-    const double least = kKeep * kKeep * fmax(rest, 0.0) * wi[S - 1], len = norm2(al);
-    double2 undo = make_double2(0.0, 0.0);
-    if (!stop && len < least) {   // (w2inv = 0: never)
+    sc->take = undo;
+    const double least = kKeep * kKeep * fmax(rest, 0.0) * w, len = norm2(al);
+    double2 un = make_double2(0.0, 0.0);
+    if (!stop && len < least) {   // (w = 0: never)
       const double f = sqrt(least);
-      const double2 x = len > 0.0 ? scale2(f / sqrt(len), al) : make_double2(f, 0.0);
-      sc->step[S - 1] = x;
-      undo = make_double2(al.x - x.x, al.y - x.y);
+      const double2 y = len > 0.0 ? scale2(f / sqrt(len), al) : make_double2(f, 0.0);
+      sc->step[S - 1] = y;
+      un = make_double2(al.x - y.x, al.y - y.y);
     }
-    sc->undo = undo;
+    sc->undo = un;
   }
 }
 
@@ -506,7 +517,6 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
   double *own = sums[wid] + 2 * S * k;
   if (l.lane < kSteps) own[gcr_own<S> + l.lane] = 0.0;
   {
-    double x[gcr_own<S>] = {};
     if (l.valid)
 #pragma unroll
       for (int a = 0; a < D; a++) {
@@ -517,22 +527,29 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
       }
     if constexpr (PRE)
       if (k > 0) load(next, 0);
-    if (l.valid)
+    // the Gram matrix, kRows rows at a time (nine vectors have 81 sums)
+    constexpr int kRows = D > 5 ? 1 : D;
 #pragma unroll
-      for (int a = 0; a < D; a++) {
-        double *y = x + a * a;
+    for (int a0 = 0; a0 < D; a0 += kRows) {
+      constexpr int NX = D > 5 ? 2 * D - 1 : gcr_own<S>;
+      double x[NX] = {};
+      if (l.valid)
 #pragma unroll
-        for (int m = 0; m < M; m++) {
+        for (int a = a0; a < a0 + kRows; a++) {
+          double *y = x + a * a - a0 * a0;
 #pragma unroll
-          for (int c = 0; c < a; c++) CH::dot(d[c][m], d[a][m], y[2 * c], y[2 * c + 1]);
-          CH::norm2(d[a][m], y[2 * a]);
+          for (int m = 0; m < M; m++) {
+#pragma unroll
+            for (int c = 0; c < a; c++) CH::dot(d[c][m], d[a][m], y[2 * c], y[2 * c + 1]);
+            CH::norm2(d[a][m], y[2 * a]);
+          }
+          if constexpr (P == QCD_HIP_F16) {
+#pragma unroll
+            for (int c = 0; c <= 2 * a; c++) y[c] *= (double)nd[a] * (double)nd[c / 2];
+          }
         }
-        if constexpr (P == QCD_HIP_F16) {
-#pragma unroll
-          for (int c = 0; c <= 2 * a; c++) y[c] *= (double)nd[a] * (double)nd[c / 2];
-        }
-      }
-    wave_reduce<NP>(x, own, gcr_own<S>);
+      wave_reduce<NP>(x, own + a0 * a0, D > 5 ? 2 * a0 + 1 : NX);
+    }
   }
   for (int j0 = 0; j0 < k; j0 += J) {
     Group g;
@@ -588,16 +605,16 @@ __global__ void __launch_bounds__(BLK) k_gcr_dots(SpinorSet<P> W, SpinorSet<P> R
 template <int P, int S>
 __global__ void __launch_bounds__(1024) k_gcr_scal(GcrScal *scs, const double *part, size_t rowsz, unsigned np, int k,
                                                    int prev, double theta, const int *ids) {
-  __shared__ double sums[1024];
+  __shared__ double sums[1024], tot[S * S];
   static_assert(gcr_values<S>(kN - S) <= 1024, "one value per lane");
   sum_parts<1024>(part + blockIdx.x * rowsz, np, gcr_values<S>(k), sums);
-  if (threadIdx.x < 64) gcr_coefficients<P, S>(scs + ids[blockIdx.x], sums, k, prev, theta);
+  if (threadIdx.x < 64) gcr_coefficients<P, S>(scs + ids[blockIdx.x], sums, k, prev, theta, tot);
 }
 
 // The sums of c workgroups of k_gcr_dots each, added up behind the partial sums
 // of all np: the one workgroup of k_gcr_scal reads 0.1 TB/s.  Solves of one rhs
 // on 16^3x32, Q, GCR(32), without and with it, ms: FP64 (512 workgroups, up to
-// 253 values) 90.2, 89.1; FP32 (1024) 22.3, 20.8.
+// 253 values) 90.2, 89.1; FP32 (1024) 22.3, 20.8 (in blocks of 4).
 __global__ void __launch_bounds__(256) k_gcr_sum(double *part, size_t rowsz, unsigned np, unsigned nv, unsigned c) {
   double *row = part + blockIdx.y * rowsz;
   const unsigned p0 = blockIdx.x * c, p1 = min(p0 + c, np);
@@ -972,6 +989,11 @@ namespace {
 //     one wavefront per SIMD) 746.  FP64 dots: half a site 71, a whole one 115;
 //     update 96 and 97 to 100.  FP32 dots: half a site, one vector, 256 lanes
 //     29.4, two vectors 32.9, 512 lanes 37.6; update 37.2 to 38.9.
+//   Blocks of 8 hold twice the vectors and accumulators.  FP64 (as above) dots: a
+//     quarter of a site, 256 lanes 86, 512 lanes 101, a third of a site 90, a
+//     sixth 96; update: a quarter 119.5, a third 119.4, a sixth 125 to 127.  FP32
+//     on 16^3x32, Q, GCR(32), dots: a third of a site, PRE 64, without 73, half a
+//     site 86, a sixth 83; update: a sixth 66, a third 68, half a site 78.
 template <int M_, int J_, int BLK_, bool PRE_>
 struct GcrShape {
   static constexpr int M = M_, J = J_, BLK = BLK_;
@@ -981,21 +1003,33 @@ template <int P>
 struct GcrShapes;
 template <>
 struct GcrShapes<QCD_HIP_F16> {
+  static constexpr int S = 4;   // steps of a block
   using Short = GcrShape<1, 2, 192, true>;
   using Dots = GcrShape<3, 1, 256, true>;
   using Update = GcrShape<1, 1, 192, true>;
+  using Short8 = Short;   // (not used)
+  using Dots8 = Dots;
+  using Update8 = Update;
 };
 template <>
 struct GcrShapes<QCD_HIP_F32> {
+  static constexpr int S = 8;
   using Short = GcrShape<1, 4, 256, true>;
   using Dots = GcrShape<3, 1, 256, false>;
   using Update = GcrShape<3, 1, 256, false>;
+  using Short8 = GcrShape<1, 2, 256, true>;
+  using Dots8 = GcrShape<2, 1, 256, true>;
+  using Update8 = GcrShape<1, 2, 256, true>;
 };
 template <>
 struct GcrShapes<QCD_HIP_F64> {
+  static constexpr int S = 8;
   using Short = GcrShape<1, 4, 256, true>;
   using Dots = GcrShape<6, 1, 512, false>;
   using Update = GcrShape<6, 1, 256, false>;
+  using Short8 = GcrShape<1, 2, 256, true>;
+  using Dots8 = GcrShape<3, 1, 256, false>;
+  using Update8 = GcrShape<3, 1, 256, false>;
 };
 template <typename SH>
 unsigned gcr_blocks(int prec, long V) {
@@ -1005,27 +1039,27 @@ unsigned gcr_blocks(int prec, long V) {
 }
 template <int P>
 constexpr bool gcr_short(long V) { return V <= (P == QCD_HIP_F16 ? 4096 : 12288); }
-// workgroups per rhs of the dots over vectors of V sites
-template <int P>
-unsigned gcr_parts_of(long V) {
-  using G = GcrShapes<P>;
-  return gcr_short<P>(V) ? gcr_blocks<typename G::Short>(P, V) : gcr_blocks<typename G::Dots>(P, V);
-}
-unsigned gcr_parts(int prec, long V) {
-  return prec == QCD_HIP_F64 ? gcr_parts_of<QCD_HIP_F64>(V)
-                             : prec == QCD_HIP_F32 ? gcr_parts_of<QCD_HIP_F32>(V) : gcr_parts_of<QCD_HIP_F16>(V);
-}
 // f(shape, grid) of a launch over count vectors of V sites (DOTS: the dots'
-// shape, else that of the kernels without sums)
-template <int P, bool DOTS, typename F>
+// shape, else that of the kernels without sums) in a block of ST steps
+template <int P, int ST, bool DOTS, typename F>
 void gcr_launch(long V, int count, F f) {
   using G = GcrShapes<P>;
   auto call = [&](auto sh) { f(sh, dim3(gcr_blocks<decltype(sh)>(P, V), (unsigned)count)); };
-  if (gcr_short<P>(V)) call(typename G::Short{});
-  else if constexpr (DOTS) call(typename G::Dots{});
-  else call(typename G::Update{});
+  constexpr bool B8 = ST == 8;
+  if (gcr_short<P>(V)) call(std::conditional_t<B8, typename G::Short8, typename G::Short>{});
+  else if constexpr (DOTS) call(std::conditional_t<B8, typename G::Dots8, typename G::Dots>{});
+  else call(std::conditional_t<B8, typename G::Update8, typename G::Update>{});
 }
-
+// f(block size constant) for the next block of a cycle with left steps to go
+template <int P, typename F>
+int gcr_next(int left, F f) {
+  constexpr int S = GcrShapes<P>::S;
+  if constexpr (S >= 8)
+    if (left >= 8) return f(std::integral_constant<int, 8>{});
+  if (left >= 4) return f(std::integral_constant<int, 4>{});
+  if (left >= 2) return f(std::integral_constant<int, 2>{});
+  return f(std::integral_constant<int, 1>{});
+}
 // More partial sums than kGcrParts are added up in up to kGcrSums groups first.
 constexpr unsigned kGcrParts = 256, kGcrSums = 64;
 
@@ -1040,7 +1074,7 @@ int gcr_block(qcd_hip_solver_s *S, int count, int k, int prev, double theta, hip
     const bool last = a == ST - 1;
     QH_TRY(matvec(last ? S->Ws : S->Rs, last ? k + a : k + a + 1, k + a));
   }
-  gcr_launch<P, true>(V, count, [&](auto sh, dim3 grid) {
+  gcr_launch<P, ST, true>(V, count, [&](auto sh, dim3 grid) {
     using SH = decltype(sh);
     k_gcr_dots<P, ST, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, prev, S->ids, V, S->part,
                                                                        S->rowsz);
@@ -1055,7 +1089,7 @@ int gcr_block(qcd_hip_solver_s *S, int count, int k, int prev, double theta, hip
     k_gcr_scal<P, ST><<<count, 1024, 0, st>>>(S->sc, part, S->rowsz, np, k, prev, theta, S->ids);
   });
   if (k + ST < n)   // the last w and the residual after them are not used
-    gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+    gcr_launch<P, ST, false>(V, count, [&](auto sh, dim3 grid) {
       using SH = decltype(sh);
       k_gcr_update<P, ST, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Ws, Rs, n, k, theta, S->sc, S->ids, V);
     });
@@ -1083,18 +1117,18 @@ int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream
     return dslash_launch_batch(epi, false, out, ro, n, S->Rs, ri, n, S->gin, nullptr, 0, 0, S->ids, count, m - theta,
                                mu, nullptr, st, nullptr);
   };
-  for (int k = 0, prev = 0; k < n; k += prev) {
-    const int left = n - k;
-    if (left >= 4) QH_TRY((gcr_block<P, 4>(S, count, k, prev, theta, st, matvec)));
-    else if (left >= 2) QH_TRY((gcr_block<P, 2>(S, count, k, prev, theta, st, matvec)));
-    else QH_TRY((gcr_block<P, 1>(S, count, k, prev, theta, st, matvec)));
-    prev = left >= 4 ? 4 : left >= 2 ? 2 : 1;
-  }
+  for (int k = 0, prev = 0; k < n; k += prev)
+    QH_TRY(gcr_next<P>(n - k, [&](auto st_c) -> int {
+      constexpr int ST = decltype(st_c)::value;
+      QH_TRY((gcr_block<P, ST>(S, count, k, prev, theta, st, matvec)));
+      prev = ST;
+      return 0;
+    }));
   k_scal_beta<<<count, 64, 0, st>>>(S->sc, n, S->prm.keep_q1, S->ids);
   // mixed even-odd solves take the correction scaled by |r^_o| (the outer
   // step adds it as it is); the others scale it where they add it
   const int scaled = S->prm.eo && S->prm.inner_prec != QCD_HIP_F64;
-  gcr_launch<P, false>(V, count, [&](auto sh, dim3 grid) {
+  gcr_launch<P, 1, false>(V, count, [&](auto sh, dim3 grid) {
     using SH = decltype(sh);
     k_solution<P, SH::M, SH::J, SH::BLK, SH::PRE><<<grid, SH::BLK, 0, st>>>(Rs, n, S->sc, E, S->ids, V, scaled);
   });
@@ -1298,11 +1332,22 @@ namespace qcdhip {
 // Partial sums of one batch row: the dots of the last GCR step, or one sum per Dslash or hop workgroup (at most one per 256
 // sites, and the z-march grids).
 static size_t solver_row(qcd_hip_lattice lat, long Vi, const qcd_hip_solver_params *prm) {
-  const size_t parts = gcr_parts(prm->inner_prec, Vi);
   const int n = prm->n_restart;
-  const size_t nv = std::max({gcr_values<4>(std::max(n - 4, 0)), gcr_values<2>(std::max(n - 2, 0)),
-                              gcr_values<1>(n - 1)});
-  const size_t dots = (parts + kGcrSums) * nv;
+  size_t dots = 0;
+  auto blocks = [&](auto p) {
+    constexpr int P = decltype(p)::value;
+    for (int k = 0; k < n;)
+      k += gcr_next<P>(n - k, [&](auto st) -> int {
+        constexpr int ST = decltype(st)::value;
+        gcr_launch<P, ST, true>(Vi, 1, [&](auto, dim3 grid) {
+          dots = std::max(dots, (size_t)(grid.x + kGcrSums) * gcr_values<ST>(k));
+        });
+        return ST;
+      });
+  };
+  if (prm->inner_prec == QCD_HIP_F64) blocks(std::integral_constant<int, QCD_HIP_F64>{});
+  else if (prm->inner_prec == QCD_HIP_F32) blocks(std::integral_constant<int, QCD_HIP_F32>{});
+  else blocks(std::integral_constant<int, QCD_HIP_F16>{});
   return std::max(dots, std::max((size_t)grid_for(lat->V) + 64, (size_t)dslash_grid_bound(lat)));
 }
 

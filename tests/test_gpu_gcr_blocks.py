@@ -47,3 +47,17 @@ def test_cycles_of_every_remainder(gpu, op, eo, mu, n, point):
 def test_sums_in_two_stages(gpu, L, prec):
     Q = gpu
     _solve(Q, L, Q.spinor_gaussian(L, 73), prec, 11, "D", 0, 0.0)
+
+
+@pytest.mark.parametrize("op,eo,mu", [("D", 0, 0.04), ("D", 1, 0.0), ("Q", 0, 0.0), ("Q", 0, 0.04)])
+@pytest.mark.parametrize("n", [8, 9, 15, 16, 27, 31, 64])
+@pytest.mark.parametrize("point", [0, 1])
+def test_blocks_of_eight(gpu, op, eo, mu, n, point):
+    """Cycles with blocks of eight and every shorter one behind them: the FP32
+    and FP64 cycle counts agree (a cycle that FP32 storage, 6e-8, ends early
+    leaves the next one as much to do)."""
+    Q = gpu
+    L = (8, 6, 4, 6)
+    src = Q.point_source(L, (1, 2, 3, 0), 2, 1) if point else Q.spinor_gaussian(L, 74)
+    ref = _solve(Q, L, src, "f64", n, op, eo, mu)
+    assert abs(_solve(Q, L, src, "f32", n, op, eo, mu) - ref) <= max(1, ref // 8)
