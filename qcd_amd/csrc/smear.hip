@@ -184,6 +184,126 @@ __global__ void __launch_bounds__(kBlock) k_gauss(GaussArgs g, SpinorIn<P> in, G
   }
 }
 
+// k_gauss for large launches: the same steps with the same arithmetic in the same
+// order (bit-identical), but the workgroup's centres lie in LDS, where its lanes
+// read their x and y neighbours (those outside its 128 columns come from memory),
+// and each link is loaded while the hop before it is multiplied: k_gauss waits
+// for five hops' loads one after the other.  128 columns rather than 256: finer
+// rounds (two wavefronts per SIMD in FP64).  Calls of 50 iterations with their
+// sources, ms, k_gauss / here: 32^3, 12 rhs FP64 2.55 / 2.23 (43.7 -> 37.5 us an
+// iteration; 256 columns 2.33), FP32 1.66 / 1.52, FP16 1.54 / 1.45; 24^3, 12 rhs
+// 1.51 / 1.39, 1.19 / 1.08, 1.21 / 1.09; 48^3, 12 rhs 11.2 / 9.0, 5.9 / 5.2, 4.34 /
+// 4.00.
+constexpr int kGaussBlock = 128;
+template <int P, bool OUT_FIELD>
+__global__ void __launch_bounds__(kGaussBlock) k_gauss_tile(GaussArgs g, SpinorIn<P> in, GaugeIn<P> U, SpinorOut<P> out,
+                                                  double alpha, double nrm) {
+  using R = typename Prec<P>::R;
+  __shared__ Cx<R> ctr[12][kGaussBlock];   // psi(z) of the workgroup's columns
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const unsigned row = lb % g.count, rest = lb / g.count;
+  const unsigned zc = rest / g.ncb, c0 = (rest - zc * g.ncb) * kGaussBlock;
+  const unsigned PC = g.tn * g.X * g.Y;   // columns per plane
+  const unsigned z0 = zc * g.zlen;
+  if (c0 >= PC || z0 >= g.Z) return;   // whole workgroups
+  const unsigned z1 = min(z0 + g.zlen, g.Z), l = threadIdx.x;
+  const bool valid = c0 + l < PC;
+  const unsigned col = valid ? c0 + l : PC - 1;
+  const unsigned rxy = col / g.tn, tt = col - rxy * g.tn, y = rxy / g.X, x = rxy - y * g.X;
+  const unsigned sx = g.tn, sy = g.tn * g.X;
+  const unsigned xp = x == g.X - 1 ? col - x * sx : col + sx, xm = x == 0 ? col + (g.X - 1) * sx : col - sx;
+  const unsigned yp = y == g.Y - 1 ? col - y * sy : col + sy, ym = y == 0 ? col + (g.Y - 1) * sy : col - sy;
+  const SpinorIn<P> src = in.advanced(row);
+  const SpinorOut<P> dst = out.advanced(row);
+  const R ia = (R)(1.0 / alpha), f = (R)(alpha * nrm);
+  auto pin = [&](Cx<R> v[12]) {
+#pragma unroll
+    for (int k = 0; k < 12; k++) asm volatile("" : "+v"(v[k].re), "+v"(v[k].im));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add = [&](Cx<R> acc[12], const Cx<R> (&ps)[12], const Cx<R> (&u)[9], auto dag) {
+#pragma unroll
+    for (int sp = 0; sp < 4; sp++) {
+      Cx<R> w[3];
+      su3_mul<decltype(dag)::value>(w, u, &ps[3 * sp]);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        acc[3 * sp + k].re += w[k].re;
+        acc[3 * sp + k].im += w[k].im;
+      }
+    }
+  };
+  // psi of column n at plane offset p: this workgroup's centre or from memory
+  auto psi = [&](Cx<R> (&ps)[12], unsigned n, unsigned p) {
+    const unsigned i = n - c0;
+    if (i < kGaussBlock) {
+#pragma unroll
+      for (int k = 0; k < 12; k++) ps[k] = ctr[k][i];
+    } else {
+      src.load(n + p, ps);
+    }
+  };
+  auto keep = [&](const Cx<R> (&v)[12]) {
+#pragma unroll
+    for (int k = 0; k < 12; k++) ctr[k][l] = v[k];
+  };
+  const std::false_type fwd;
+  const std::true_type bwd;
+  Cx<R> bz[12];
+  {
+    const unsigned zm = PC * (z0 == 0 ? g.Z - 1 : z0 - 1);
+    Cx<R> ps[12], u[9];
+#pragma unroll
+    for (int k = 0; k < 12; k++) bz[k] = Cx<R>{R(0), R(0)};
+    src.load(col + zm, ps);
+    U.load(3, col + zm, u);
+    add(bz, ps, u, bwd);
+    pin(bz);
+    src.load(col + PC * z0, ps);
+    keep(ps);
+  }
+  for (unsigned z = z0; z < z1; z++) {
+    const unsigned p = PC * z, c = col + p;
+    Cx<R> acc[12], ps[12], u[9], un[9];
+    U.load(1, c, u);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 12; k++) acc[k] = Cx<R>{ctr[k][l].re * ia + bz[k].re, ctr[k][l].im * ia + bz[k].im};
+    U.load(1, xm + p, un);
+    psi(ps, xp, p);
+    add(acc, ps, u, fwd);
+    pin(acc);
+    U.load(2, c, u);
+    psi(ps, xm, p);
+    add(acc, ps, un, bwd);
+    pin(acc);
+    U.load(2, ym + p, un);
+    psi(ps, yp, p);
+    add(acc, ps, u, fwd);
+    pin(acc);
+    U.load(3, c, u);
+    psi(ps, ym, p);
+    add(acc, ps, un, bwd);
+    pin(acc);
+    // last, the z direction: the next step's backward hop from this centre and
+    // U_z here, then the forward hop, whose spinor is the next step's centre
+    src.load(z == g.Z - 1 ? col : c + PC, ps);
+#pragma unroll
+    for (int sp = 0; sp < 4; sp++) {
+      Cx<R> w[3], q[3] = {ctr[3 * sp][l], ctr[3 * sp + 1][l], ctr[3 * sp + 2][l]};
+      su3_mul<true>(w, u, q);
+#pragma unroll
+      for (int k = 0; k < 3; k++) bz[3 * sp + k] = w[k];
+    }
+    add(acc, ps, u, fwd);
+#pragma unroll
+    for (int k = 0; k < 12; k++) acc[k] = Cx<R>{acc[k].re * f, acc[k].im * f};
+    if (valid) dst.store(OUT_FIELD ? (g.tn > 1 ? tt : g.t0) + g.T * (rxy + g.X * g.Y * z) : c, acc);
+    __syncthreads();   // the neighbours have read this plane
+    keep(ps);
+  }
+}
+
 // Stored values (and FP16 norms) of the slice's sites: field -> compact buffer.
 // src and dst point at right-hand side 0; rows lie 12 sstride / 12 dstride
 // elements apart.
@@ -220,14 +340,11 @@ __global__ void __launch_bounds__(kBlock) k_gauss_gather_links(GaussArgs g, cons
 
 // z steps per lane of k_gauss for a launch over `sites` (site, rhs) pairs: the
 // march saves loads but divides the wavefronts, so it is as long as leaves about
-// 4096 of them (four per SIMD).  Calls of 50 iterations with their sources, ms:
-// 24^3, 12 rhs 1.76 with 1 step, 2.14 with 6; 16^3, 12 rhs 0.77 with 1, 1.23 with
-// 4; 32^3, one rhs 0.58 with 1, 1.99 with 8; 32^3, 12 rhs 3.53 with 2, 3.60 with
-// 1 and 8; 22^3x16, 5 rhs (20 iterations) 2.84 with 3, 2.99 with 1, 3.20 with 6;
-// a 48^3 slice, 12 rhs: 201-226 us an iteration with 2 to 24.  (Lanes of one
-// spin each, without a march and with every hop's loads in flight: 5.29 ms on
-// 32^3, 2.38 on 24^3, 12 rhs; they gain on 8^3 only.)
-// QCD_HIP_GAUSS_ZLEN overrides it.
+// 4096 of them (four per SIMD): one step below kGaussTile, a few for whole FP16
+// fields.  Calls of 50 iterations with their sources, ms: 16^3, 12 FP64 rhs 0.77
+// with 1 step, 1.23 with 4; 32^3, one rhs 0.58 with 1, 1.99 with 8.  (Lanes of one
+// spin each, without a march and with every hop's loads in flight, gain on 8^3
+// only.)  QCD_HIP_GAUSS_ZLEN overrides it, for launches of every size.
 static unsigned gauss_zlen(unsigned Z, long sites) {
   static const int env = [] {
     const char *e = std::getenv("QCD_HIP_GAUSS_ZLEN");
@@ -236,6 +353,34 @@ static unsigned gauss_zlen(unsigned Z, long sites) {
   const long per = 4096L * 64;
   const unsigned r = env > 0 ? (unsigned)env : (unsigned)std::max(1L, std::min((sites + per / 2) / per, (long)Z));
   return r > Z ? Z : r;
+}
+
+// From this many (site, rhs) pairs a launch takes k_gauss_tile: calls of 50
+// iterations, ms, k_gauss / k_gauss_tile: 16^3, 12 rhs FP64 0.71 / 0.77, FP32 0.69 /
+// 0.71, FP16 0.65 / 0.76; 17 x 19 x 28, 5 rhs 0.62 / 0.69; 20^3, 12 rhs 0.98 / 0.97,
+// 0.83 / 0.85, 0.84 / 0.85; 32^3, 3 rhs 0.97 / 0.88, 0.68 / 0.62, 0.68 / 0.66.  Whole
+// FP16 fields stay with k_gauss (22^3x16, 5 rhs, 20 iterations 1.10 / 1.12).
+constexpr long kGaussTile = 96 * 1024;
+
+// z steps per lane of k_gauss_tile: a round of workgroups takes a time of z
+// steps and about one more to start, so the z that makes ceil(workgroups /
+// slots) (z + 1.2) smallest.  32^3, 12 rhs FP64 (1024 slots), z = 1, 2, 3, 4, 6, 8:
+// 2.57, 2.44, 2.65 (1056 workgroups), 2.23 (768), 2.65, 2.98 ms; 24^3 1.47, 1.39 (720),
+// 1.55, 1.82; FP32 on 24^3 1.08 (1440 of 1536 slots), 1.14.  FP16 loses from three
+// steps up.
+static unsigned gauss_tile_zlen(int prec, unsigned Z, long blocks) {
+  const long slots = prec == QCD_HIP_F64 ? 1024 : 1536;
+  unsigned best = 1;
+  double cost = 0.0;
+  for (unsigned z = 1; z <= Z && z <= (prec == QCD_HIP_F16 ? 2u : 8u); z++) {
+    const long n = blocks * ((Z + z - 1) / z);
+    const double c = (double)((n + slots - 1) / slots) * (z + 1.2);
+    if (z == 1 || c < cost) {
+      best = z;
+      cost = c;
+    }
+  }
+  return best;
 }
 
 // Rows of one pass: two compact buffers of `rows` right-hand sides each stay
@@ -293,8 +438,11 @@ static int gauss_run(qcd_hip_field v, qcd_hip_field gauge, qcd_hip_field buf, in
   }
   const GaugeIn<P> U = GaugeIn<P>::of(links);
   const unsigned nb = (unsigned)grid_for(g.n);
-  g.zlen = gauss_zlen(g.Z, (long)g.n * std::min(rows, v->nrhs));
-  g.ncb = (unsigned)grid_for((long)g.tn * g.X * g.Y);
+  const long pairs = (long)g.n * std::min(rows, v->nrhs), columns = (long)g.tn * g.X * g.Y;
+  const bool tile = pairs >= kGaussTile && !(P == QCD_HIP_F16 && g.tn > 1) && !std::getenv("QCD_HIP_GAUSS_ZLEN");
+  const int block = tile ? kGaussBlock : kBlock;
+  g.ncb = (unsigned)grid_for(columns, block);
+  g.zlen = tile ? gauss_tile_zlen(P, g.Z, (long)g.ncb * std::min(rows, v->nrhs)) : gauss_zlen(g.Z, pairs);
   const unsigned nzc = (g.Z + g.zlen - 1) / g.zlen;
   for (int r0 = 0; r0 < v->nrhs; r0 += rows) {
     g.count = (unsigned)std::min(rows, v->nrhs - r0);
@@ -309,8 +457,10 @@ static int gauss_run(qcd_hip_field v, qcd_hip_field gauge, qcd_hip_field buf, in
     for (int it = 0; it < niter; it++) {
       const bool from_a = (it % 2) == 0;
       const SpinorIn<P> &src = from_a ? ain : bin;
-      if (it == niter - 1) k_gauss<P, true><<<zgrid, kBlock, 0, st>>>(g, src, U, vout, alpha, nrm);
-      else k_gauss<P, false><<<zgrid, kBlock, 0, st>>>(g, src, U, from_a ? bout : aout, alpha, nrm);
+      const bool last = it == niter - 1;
+      auto k = tile ? (last ? k_gauss_tile<P, true> : k_gauss_tile<P, false>)
+                    : (last ? k_gauss<P, true> : k_gauss<P, false>);
+      k<<<zgrid, block, 0, st>>>(g, src, U, last ? vout : from_a ? bout : aout, alpha, nrm);
       QH_CHECK(hipGetLastError());
     }
   }

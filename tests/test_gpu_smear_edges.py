@@ -87,3 +87,26 @@ def test_gauss_march_lengths_agree(gpu):
     for _ in range(3):
         v = O.gauss3d_all(geo, v, u, 4.0)
     assert np.linalg.norm(ref[0] - v) <= 1e-13 * np.linalg.norm(v)
+
+
+# 128 columns per workgroup: partial last one, rows longer than it, planes
+# shorter than it; chunks of 1 to 8 planes with a shorter last one
+@pytest.mark.parametrize("L,slice_,nrhs", [((4, 34, 29, 31), 1, 12), ((2, 150, 9, 40), 0, 3), ((4, 6, 5, 350), 3, 12),
+                                           ((8, 18, 14, 22), -1, 7), ((2, 48, 40, 50), 0, 12)])
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+def test_gauss_tiles_match_columns(gpu, prec, L, slice_, nrhs):
+    """Large launches take another kernel than one rhs alone: same bits."""
+    Q = gpu
+    lat = Q.Lattice(L)
+    g64, g = Q.Gauge(lat), Q.Gauge(lat, Q.PREC[prec])
+    Q.gauge_generate_device(g64, 0.3, 41)
+    Q.convert(g, g64)
+    v = Q.Spinor(lat, Q.PREC[prec], nrhs)
+    src = [Q.spinor_gaussian(L, 42 + r) for r in (0, 1)]
+    for r in range(nrhs):
+        v.upload(src[r % 2], rhs=r)
+    Q.gauss_smear(v, g, 0.6, slice_, 3)
+    for r in (0, nrhs - 1):
+        one = Q.Spinor(lat, Q.PREC[prec]).upload(src[r % 2])
+        Q.gauss_smear(one, g, 0.6, slice_, 3)
+        assert np.array_equal(one.download(), v.download(r))
