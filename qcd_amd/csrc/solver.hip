@@ -303,10 +303,9 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
 // Directions of a block of S steps at k: d_0 = res_k, d_{a+1} = (A - theta) d_a,
 // so v_a = A d_a = d_{a+1} + theta d_a.  w_k .. w_{k+S-1} span what S single steps
 // would add, so the residual and the solution after the block are those of
-// GCR(n).  The S vectors are projected against the
-// w_j, j < k, in one pass over them and formed in a second one, where single
-// steps take 2 S passes, and these passes are what a cycle spends its time on
-// (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2, 4
+// GCR(n).  The S vectors are projected against the w_j, j < k, in one pass over
+// them and formed in a second one, where single steps take 2 S passes, and these
+// passes are what a cycle spends its time on (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2, 4
 // and 8, ms: one FP64 rhs, Q, GCR(32) on 16^3x32 204, 126, 87, 69; one FP32 rhs
 // 4: 20.8, 8: 17.3; 12 FP16 rhs, GCR(12) on 24^3x48 132, 107, 96, 97, on 16^3x32
 // 21.0, 16.9, 15.0, 16.0.  FP16 stays at 4: its dots are bound by arithmetic, which
@@ -318,9 +317,9 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
 // as independent of each other as the residuals of single steps, and a long FP16
 // cycle reaches the same residual: GCR(32) on 8^3x16, kappa 0.125, 4.0e-4 of the
 // one before, single steps 4.9e-4 (d_1 without theta 8.1e-4).  The outer step
-// counts are those of single
-// steps for FP64, FP32 and FP16, Q and D, GCR(4) to GCR(64), kappa 0.12 to
-// 0.139, random and point sources (FP16 with 64 steps: one cycle more or less).
+// counts are those of single steps for FP64, FP32 and FP16, Q and D, GCR(4) to
+// GCR(64), kappa 0.1 to 0.139, random and point sources, where single steps
+// converge (FP16 with 64 steps: one cycle more or less).
 
 // Smallest |w_{k+a}|^2 / |v_a|^2 that is told from rounding of the stored vectors:
 // a v_a with less to itself is left out of the cycle

@@ -61,3 +61,18 @@ def test_blocks_of_eight(gpu, op, eo, mu, n, point):
     src = Q.point_source(L, (1, 2, 3, 0), 2, 1) if point else Q.spinor_gaussian(L, 74)
     ref = _solve(Q, L, src, "f64", n, op, eo, mu)
     assert abs(_solve(Q, L, src, "f32", n, op, eo, mu) - ref) <= max(1, ref // 8)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("op,eo,mu", [("D", 0, 0.0), ("D", 1, 0.0), ("Q", 0, 0.0), ("D", 1, 5.0)])
+@pytest.mark.parametrize("n", [12, 24])
+def test_heavy_masses(gpu, prec, op, eo, mu, n):
+    """kappa 0.005: a few steps reach the rounding of the stored vectors, the
+    rest of the cycle works in their noise and has to leave the solution alone."""
+    Q = gpu
+    L = (8, 6, 4, 6)
+    src, u, lat = Q.spinor_gaussian(L, 75), Q.gauge_generate(L, 0.2, 71), Q.Lattice(L)
+    fb, fx = Q.Spinor(lat).upload(src), Q.Spinor(lat)
+    S = Q.Solver(lat, Q.Gauge(lat).upload(u), n_restart=n, tol=TOL, inner_prec=prec, op=op, eo=eo, max_outer=30)
+    S.solve(fx, fb, 0.005, mu)
+    assert O.b_minus_Dx(O.Geometry(L), fx.download(), src, u, 0.005, mu) <= TOL
