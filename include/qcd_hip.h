@@ -38,7 +38,8 @@ int    qcd_hip_device_name(char *buf, int len);
 int    qcd_hip_synchronize(void);
 size_t qcd_hip_bytes_in_use(void);
 /* Device blocks freed by the library are cached for reuse (hipFree would
- * synchronise the device); this hands the cache back to the runtime. */
+ * synchronise the device), and large host transfers keep 16 MB of pinned
+ * memory; this hands both back to the runtime. */
 void   qcd_hip_release_cache(void);
 
 /* ------------------------------------------------------------ lattice
