@@ -353,8 +353,14 @@ __device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.
 // 0 and w2inv = 0, so nothing refers to it.  In reduced precision the w_j of a
 // long cycle lose their orthogonality and a step can come out far too long
 // (FP16, 64 steps on 270 sites): |res_k|^2 above four times the smallest before
-// it leaves the last block and the rest of the cycle out (alpha = 0).  prev:
-// steps of the block before.
+// it leaves the last block and the rest of the cycle out (alpha = 0).  That is
+// seen one block late, and never for a cycle's last one.  But the steps of a
+// block cannot take more off |res_k|^2 than there is (Bessel): sums that claim so
+// by more than kExcess of it come from vectors that are not orthogonal, and leave
+// their own block and the rest out.  (FP16, Q, mu = 0.04, point source, 8x6x4x6,
+// one cycle of 40 steps: 0.36 of the residual without this, 0.016 with it; a
+// block that is too long without claiming too much can still double |res|.)
+// prev: steps of the block before.
 //
 // The next block starts from res_{k+S}, which has to hold something of
 // w_{k+S-1} for its vectors to be new.  Q is indefinite and leaves every other
@@ -362,6 +368,7 @@ __device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.
 // kKeep |res_{k+S}| of w_{k+S-1} in place of the step alpha, the solution alpha
 // itself, and the next block takes the difference (undo) out again.
 constexpr double kKeep = 0.5;
+constexpr double kExcess = 0.01;   // above the rounding of the sums, of single and half precision vectors too
 template <int P, int S>
 __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums, int k, int prev, double theta,
                                                  double *tot) {
@@ -427,7 +434,7 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
   if (k > 0) R = cadd2(R, cmul2(undo, conj2(wv(k - 1, j))));   // res_k = d_0 + undo w_{k-1}
   double rest = r2, w = 0.0;
   double2 al = make_double2(0.0, 0.0);
-  bool bad = false;
+  bool bad = false, cut = false;
 #pragma unroll
   for (int a = 0; a < S; a++) {
     const int o = a * S;   // lanes of row a: <w_{k+a}, v_j>
@@ -438,6 +445,7 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
     w = N > gcr_floor<P>() * n ? 1.0 / N : 0.0;
     bad = bad || !(N == N) || isinf(N) || (a == 0 && !(n > 0.0));
     rest -= w * norm2(Ra);
+    cut = cut || rest < -kExcess * r2;
     al = scale2(-w, Ra);
     if (l == 0) {
       sc->w2inv[k + a] = w;
@@ -453,12 +461,14 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
     if (!stop && bad) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
     if (stop)
       for (int q = 1; q <= prev; q++) sc->alpha[k - q] = make_double2(0.0, 0.0);
+    if (cut)
+      for (int a = 0; a < S; a++) sc->alpha[k + a] = sc->step[a] = make_double2(0.0, 0.0);
     sc->rmin = k > 0 ? fmin(sc->rmin, r2) : r2;
-    sc->stop = stop;
+    sc->stop = stop || cut;
     sc->take = undo;
     const double least = kKeep * kKeep * fmax(rest, 0.0) * w, len = norm2(al);
     double2 un = make_double2(0.0, 0.0);
-    if (!stop && len < least) {   // (w = 0: never)
+    if (!stop && !cut && len < least) {   // (w = 0: never)
       const double f = sqrt(least);
       const double2 y = len > 0.0 ? scale2(f / sqrt(len), al) : make_double2(f, 0.0);
       sc->step[S - 1] = y;

@@ -1,0 +1,39 @@
+"""What one GCR cycle (max_outer = 1) leaves of the residual."""
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+EPS = 0.3
+
+
+def _source(L, point):
+    return O.point_source(L, (1, 0, 1, 1), 1, 2) if point else O.spinor_gaussian(L, 62)
+
+
+def _one_cycle(Q, L, b, kappa, mu, op, eo, prec, n, seed=61):
+    lat = Q.Lattice(L)
+    g = Q.Gauge(lat).upload(O.gauge_generate(L, EPS, seed))
+    fb, fx = Q.Spinor(lat).upload(b), Q.Spinor(lat)
+    S = Q.Solver(lat, g, n_restart=n, tol=1e-15, inner_prec=prec, op=op, eo=eo, max_outer=1)
+    r = S.solve(fx, fb, kappa, mu, check=False)
+    S.close()
+    assert r["rc"] in (0, 6) and r["outer"] == 1
+    return r["relres"]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("op", ["Q", "D"])
+@pytest.mark.parametrize("L", [(6, 3, 5, 3), (8, 6, 4, 6), (16, 8, 8, 8)])
+@pytest.mark.parametrize("kappa,mu", [(0.12, 0.0), (0.12, 0.04), (0.139, 0.0)])
+def test_longer_cycles_reach_no_less(gpu, prec, op, L, kappa, mu):
+    """A block of steps that is too long is left out, the last one of a cycle
+    too: |res| stays within twice the smallest of any shorter cycle."""
+    Q = gpu
+    b = _source(L, True)
+    least = 1.0
+    for n in (8, 16, 24, 28, 32, 36, 40, 44, 48, 56, 64):
+        r = _one_cycle(Q, L, b, kappa, mu, op, 0, prec, n)
+        assert r <= 2.0 * least
+        least = min(least, r)
