@@ -359,8 +359,9 @@ __device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.
 // by more than kExcess of it come from vectors that are not orthogonal, and leave
 // their own block and the rest out.  (FP16, Q, mu = 0.04, point source, 8x6x4x6,
 // one cycle of 40 steps: 0.36 of the residual without this, 0.016 with it; a
-// block that is too long without claiming too much can still double |res|.)
-// prev: steps of the block before.
+// block that is too long without claiming too much can still double |res|.)  A
+// residual of exactly 0 (heavy quarks: FP16 vectors of a few steps) ends the
+// cycle as well.  prev: steps of the block before.
 //
 // The next block starts from res_{k+S}, which has to hold something of
 // w_{k+S-1} for its vectors to be new.  Q is indefinite and leaves every other
@@ -377,6 +378,7 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
   const double2 undo = k > 0 ? sc->undo : make_double2(0.0, 0.0);
   const double r2 = own[0] - (k > 0 ? norm2(undo) * wn[0] : 0.0);
   const bool stop = k > 0 && (sc->stop || r2 > 4.0 * sc->rmin);
+  const bool done = r2 <= 0.0;   // (also where an even-odd source has nothing on the odd sites)
   // <w_j, v_a>
   auto wv = [&](int j, int a) {
     const double *x = sums + 2 * (S * j + a);
@@ -449,7 +451,7 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
     al = scale2(-w, Ra);
     if (l == 0) {
       sc->w2inv[k + a] = w;
-      sc->alpha[k + a] = sc->step[a] = stop ? make_double2(0.0, 0.0) : al;
+      sc->alpha[k + a] = sc->step[a] = stop || done ? make_double2(0.0, 0.0) : al;
     }
     if (j > a) {
       if (l < S) sc->coef[(k + j) * kN + k + a] = scale2(-w, Gj);
@@ -458,17 +460,17 @@ __device__ __forceinline__ void gcr_coefficients(GcrScal *sc, const double *sums
     }
   }
   if (l == 0) {
-    if (!stop && bad) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
+    if (!stop && !done && bad) sc->bad = 1;   // Krylov space is sick (invert.c:75-79)
     if (stop)
       for (int q = 1; q <= prev; q++) sc->alpha[k - q] = make_double2(0.0, 0.0);
     if (cut)
       for (int a = 0; a < S; a++) sc->alpha[k + a] = sc->step[a] = make_double2(0.0, 0.0);
     sc->rmin = k > 0 ? fmin(sc->rmin, r2) : r2;
-    sc->stop = stop || cut;
+    sc->stop = stop || cut || done;
     sc->take = undo;
     const double least = kKeep * kKeep * fmax(rest, 0.0) * w, len = norm2(al);
     double2 un = make_double2(0.0, 0.0);
-    if (!stop && !cut && len < least) {   // (w = 0: never)
+    if (!sc->stop && len < least) {   // (w = 0: never)
       const double f = sqrt(least);
       const double2 y = len > 0.0 ? scale2(f / sqrt(len), al) : make_double2(f, 0.0);
       sc->step[S - 1] = y;

@@ -37,3 +37,21 @@ def test_longer_cycles_reach_no_less(gpu, prec, op, L, kappa, mu):
         r = _one_cycle(Q, L, b, kappa, mu, op, 0, prec, n)
         assert r <= 2.0 * least
         least = min(least, r)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("links,kappa", [(1.0, 1e-5), (1e-8, 0.12), (0.0, 0.12)])
+@pytest.mark.parametrize("point", [0, 1])
+def test_residual_of_zero_ends_the_cycle(gpu, prec, links, kappa, point):
+    """Local operators, but for little: a few steps, or none for an even point
+    source, leave a residual that is stored as exactly 0."""
+    Q = gpu
+    L = (8, 6, 4, 6)
+    lat, u = Q.Lattice(L), links * O.gauge_generate(L, EPS, 61)
+    b = O.point_source(L, (0, 0, 0, 0), 1, 2) if point else _source(L, 0)
+    for eo in (0, 1):
+        for n in (4, 12, 32):
+            fb, fx = Q.Spinor(lat).upload(b), Q.Spinor(lat)
+            S = Q.Solver(lat, Q.Gauge(lat).upload(u), n_restart=n, tol=1e-10, inner_prec=prec, op="D", eo=eo, max_outer=20)
+            S.solve(fx, fb, kappa)
+            assert O.b_minus_Dx(O.Geometry(L), fx.download(), b, u, kappa) <= 1e-10
