@@ -964,6 +964,7 @@ struct qcd_hip_solver_s {
   // M^-1 temporaries, the odd correction; FP64 for an FP64 inner solve, the
   // inner precision otherwise
   qcd_hip_field reh = nullptr, roh = nullptr, th = nullptr, eoh = nullptr;
+  bool single = false;               // GCR steps one by one (solve_rhs)
   // the captured GCR cycle (prm.graph) and the launch arguments it was
   // captured with; every buffer it touches belongs to the solver
   hipGraphExec_t cycle = nullptr;
@@ -1063,8 +1064,9 @@ void gcr_launch(long V, int count, F f) {
 }
 // f(block size constant) for the next block of a cycle with left steps to go
 template <int P, typename F>
-int gcr_next(int left, F f) {
+int gcr_next(int left, bool single, F f) {
   constexpr int S = GcrShapes<P>::S;
+  if (single) return f(std::integral_constant<int, 1>{});
   if constexpr (S >= 8)
     if (left >= 8) return f(std::integral_constant<int, 8>{});
   if (left >= 4) return f(std::integral_constant<int, 4>{});
@@ -1129,7 +1131,7 @@ int gcr_cycle(qcd_hip_solver_s *S, int count, double kappa, double mu, hipStream
                                mu, nullptr, st, nullptr);
   };
   for (int k = 0, prev = 0; k < n; k += prev)
-    QH_TRY(gcr_next<P>(n - k, [&](auto st_c) -> int {
+    QH_TRY(gcr_next<P>(n - k, S->single, [&](auto st_c) -> int {
       constexpr int ST = decltype(st_c)::value;
       QH_TRY((gcr_block<P, ST>(S, count, k, prev, theta, st, matvec)));
       prev = ST;
@@ -1267,9 +1269,9 @@ int upload_ids(qcd_hip_solver_s *S, const std::vector<int> &ids, hipStream_t st)
   return 0;
 }
 
-// Solve rhs [x0, x0 + cnt) of b into x.
+// Solve rhs [x0, x0 + cnt) of b into x; *broke: a breakdown ended it.
 int solve_batch(qcd_hip_solver_s *S, qcd_hip_field x, qcd_hip_field b, int x0, int cnt, double kappa, double mu,
-                hipStream_t st, qcd_hip_solver_stats *tot, int *worst) {
+                hipStream_t st, qcd_hip_solver_stats *tot, int *worst, bool *broke) {
   const unsigned V = (unsigned)S->lat->V;
   k_start<<<dim3(S->nb, (unsigned)cnt), kBlock, 0, st>>>(SpinorSet<QCD_HIP_F64>::of(b), SpinorSet<QCD_HIP_F64>::of(x),
                                                          x0, SpinorSet<QCD_HIP_F64>::of(S->bq), S->use_q, V);
@@ -1316,7 +1318,31 @@ int solve_batch(qcd_hip_solver_s *S, qcd_hip_field x, qcd_hip_field b, int x0, i
     tot->relres = std::max(tot->relres, rel[i]);
     if (!bad && rel[i] > S->prm.tol) *worst = std::max(*worst, 6);
   }
-  if (bad) *worst = 5;
+  *broke = bad;
+  return 0;
+}
+
+// solve_batch, and after a breakdown once more with single GCR steps.  A block
+// applies the operator up to eight times without a normalisation: eight powers
+// of a norm of 6e4 (kappa 1e-5, Q) or single ones of links far from SU(3) leave
+// the range of FP32, which a step at a time stays in.
+int solve_rhs(qcd_hip_solver_s *S, qcd_hip_field x, qcd_hip_field b, int x0, int cnt, double kappa, double mu,
+              hipStream_t st, qcd_hip_solver_stats *tot, int *worst) {
+  const qcd_hip_solver_stats before = *tot;
+  const int worst0 = *worst;
+  bool broke = false;
+  QH_TRY(solve_batch(S, x, b, x0, cnt, kappa, mu, st, tot, worst, &broke));
+  if (broke) {
+    *tot = before;
+    *worst = worst0;
+    S->drop_cycle();
+    S->single = true;
+    const int rc = solve_batch(S, x, b, x0, cnt, kappa, mu, st, tot, worst, &broke);
+    S->drop_cycle();
+    S->single = false;
+    QH_TRY(rc);
+  }
+  if (broke) *worst = 5;
   return 0;
 }
 
@@ -1347,14 +1373,15 @@ static size_t solver_row(qcd_hip_lattice lat, long Vi, const qcd_hip_solver_para
   size_t dots = 0;
   auto blocks = [&](auto p) {
     constexpr int P = decltype(p)::value;
-    for (int k = 0; k < n;)
-      k += gcr_next<P>(n - k, [&](auto st) -> int {
-        constexpr int ST = decltype(st)::value;
-        gcr_launch<P, ST, true>(Vi, 1, [&](auto, dim3 grid) {
-          dots = std::max(dots, (size_t)(grid.x + kGcrSums) * gcr_values<ST>(k));
+    for (bool single : {false, true})
+      for (int k = 0; k < n;)
+        k += gcr_next<P>(n - k, single, [&](auto st) -> int {
+          constexpr int ST = decltype(st)::value;
+          gcr_launch<P, ST, true>(Vi, 1, [&](auto, dim3 grid) {
+            dots = std::max(dots, (size_t)(grid.x + kGcrSums) * gcr_values<ST>(k));
+          });
+          return ST;
         });
-        return ST;
-      });
   };
   if (prm->inner_prec == QCD_HIP_F64) blocks(std::integral_constant<int, QCD_HIP_F64>{});
   else if (prm->inner_prec == QCD_HIP_F32) blocks(std::integral_constant<int, QCD_HIP_F32>{});
@@ -1536,7 +1563,7 @@ int qcd_hip_solver_solve(qcd_hip_solver S, qcd_hip_field x, qcd_hip_field b, dou
   int worst = 0;
   for (int r0 = 0; r0 < b->nrhs && worst != 5; r0 += S->B) {
     const int cnt = std::min(S->B, b->nrhs - r0);
-    QH_TRY(solve_batch(S, x, b, r0, cnt, kappa, mu, st, &tot, &worst));
+    QH_TRY(solve_rhs(S, x, b, r0, cnt, kappa, mu, st, &tot, &worst));
   }
   tot.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   if (stats) *stats = tot;

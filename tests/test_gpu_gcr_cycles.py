@@ -1,4 +1,5 @@
 """What one GCR cycle (max_outer = 1) leaves of the residual."""
+import numpy as np
 import pytest
 
 import oracle as O
@@ -55,3 +56,28 @@ def test_residual_of_zero_ends_the_cycle(gpu, prec, links, kappa, point):
             S = Q.Solver(lat, Q.Gauge(lat).upload(u), n_restart=n, tol=1e-10, inner_prec=prec, op="D", eo=eo, max_outer=20)
             S.solve(fx, fb, kappa)
             assert O.b_minus_Dx(O.Geometry(L), fx.download(), b, u, kappa) <= 1e-10
+
+
+@pytest.mark.parametrize("prec", ["f32", "f16"])
+@pytest.mark.parametrize("op,eo,kappa,mu,links,n", [("Q", 0, 1e-12, 0.0, 1.0, 4), ("D", 0, 0.12, 1e10, 1.0, 4),
+                                                    ("D", 1, 0.12, 1e10, 1.0, 4), ("Q", 0, 0.12, 0.0, 1e6, 32)])
+@pytest.mark.parametrize("graph", [0, 1])
+def test_operators_of_large_norm(gpu, prec, op, eo, kappa, mu, links, n, graph):
+    """Powers of the operator leave the range of FP32: solved in single steps.
+    The solver then does an ordinary solve as a new one does."""
+    Q = gpu
+    if prec == "f16" and links > 6e4:
+        pytest.skip("FP16 links end at 65504")
+    L = (8, 6, 4, 6)
+    lat, u, b = Q.Lattice(L), O.gauge_generate(L, EPS, 61), _source(L, 0)
+    fb, fx, fy = Q.Spinor(lat).upload(b), Q.Spinor(lat), Q.Spinor(lat)
+    kw = dict(n_restart=n, tol=1e-10, inner_prec=prec, op=op, eo=eo, max_outer=100, graph=graph)
+    g, big = Q.Gauge(lat).upload(u), Q.Gauge(lat).upload(links * u)
+    S = Q.Solver(lat, big, **kw)
+    for _ in range(2):
+        S.solve(fx, fb, kappa, mu)
+        assert O.b_minus_Dx(O.Geometry(L), fx.download(), b, links * u, kappa, mu) <= 1e-10
+    S.set_gauge(g)
+    r = S.solve(fx, fb, 0.05, 0.03)
+    assert r == {**Q.Solver(lat, g, **kw).solve(fy, fb, 0.05, 0.03), "seconds": r["seconds"]}
+    assert np.array_equal(fx.download(), fy.download())
