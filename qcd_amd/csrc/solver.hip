@@ -106,30 +106,15 @@ struct Chunk {
       return to_cx<R>(as_half2(q[i]));
     }
   }
-  // product of the low half of a with the low (HI: high) half of b, exact in
-  // FP32.  Mixed-precision instructions: as a multiplication of converted values
-  // the compiler keeps every vector that is used again converted, in twice the
-  // registers.
-  template <bool HI>
-  static __device__ __forceinline__ float half_product(unsigned a, unsigned b) {
-    float r;
-    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b));
-    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-  }
-  // sum over the chunk of conj(a) b, of stored values
+  // sum over the chunk of conj(a) b, of stored values, in FP64 from the product on
+  // (FP16 with each pair of products added in FP32: 12 rhs on 24^3x48, 406 against
+  // 496 us a launch, 96.1 against 98.5 ms a solve)
   static __device__ __forceinline__ void dot(u32x4 a, u32x4 b, double &re, double &im) {
 #pragma unroll
     for (int i = 0; i < kC; i++) {
       const auto x = get(a, i), y = get(b, i);
-      if constexpr (P == QCD_HIP_F16) {
-        // one rounding per sum
-        re += (double)fmaf(x.im, y.im, half_product<false>(a[i], b[i]));
-        im += (double)fmaf(-x.im, y.re, half_product<true>(a[i], b[i]));
-      } else {
-        re = fma((double)x.re, (double)y.re, fma((double)x.im, (double)y.im, re));
-        im = fma((double)x.re, (double)y.im, fma(-(double)x.im, (double)y.re, im));
-      }
+      re = fma((double)x.re, (double)y.re, fma((double)x.im, (double)y.im, re));
+      im = fma((double)x.re, (double)y.im, fma(-(double)x.im, (double)y.re, im));
     }
   }
   // |a|^2 of stored values
@@ -137,8 +122,7 @@ struct Chunk {
 #pragma unroll
     for (int i = 0; i < kC; i++) {
       const auto x = get(a, i);
-      if constexpr (P == QCD_HIP_F16) re += (double)fmaf(x.im, x.im, x.re * x.re);
-      else re = fma((double)x.re, (double)x.re, fma((double)x.im, (double)x.im, re));
+      re = fma((double)x.re, (double)x.re, fma((double)x.im, (double)x.im, re));
     }
   }
   // acc += c a (FP16: c includes the site norm)
@@ -993,9 +977,9 @@ namespace {
 //     16 128 sites: FP64 and FP32 2% slower.
 //   Long ones: what measured best, us per launch (12 FP16 rhs, GCR(12), 24^3x48;
 //     one FP64 rhs, GCR(32), 16^3x32; three FP32, GCR(16), 16^3x24, even-odd).
-//     FP16 dots: (3, 1, 256, PRE) 396, two vectors in flight 424 to 513, 512
-//     lanes 515, a third of a site 529; they are bound by the FP64 additions of
-//     the products.  FP16 update: a third of a site, 192 lanes 501 (four
+//     FP16 dots: a third of a site, two vectors 496, one 508, three 618, a whole
+//     site 542 (its vectors in FP64 take all registers); they are bound by the FP64
+//     arithmetic.  FP16 update: a third of a site, 192 lanes 501 (four
 //     wavefronts per SIMD; with six registers more, three, 652), 384 lanes 594,
 //     two vectors in flight 519, a whole site (its four FP64 accumulators leave
 //     one wavefront per SIMD) 746.  FP64 dots: half a site 71, a whole one 115;
@@ -1017,7 +1001,7 @@ template <>
 struct GcrShapes<QCD_HIP_F16> {
   static constexpr int S = 4;   // steps of a block
   using Short = GcrShape<1, 2, 192, true>;
-  using Dots = GcrShape<3, 1, 256, true>;
+  using Dots = Short;
   using Update = GcrShape<1, 1, 192, true>;
   using Short8 = Short;   // (not used)
   using Dots8 = Dots;
