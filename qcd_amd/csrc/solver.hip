@@ -968,13 +968,13 @@ namespace {
 // (PRE: and the next J on their way), BLK lanes per workgroup.  Chosen by the
 // vector length alone, so that a right-hand side gets the same sums alone and in
 // any batch.
-//   Short vectors: one chunk per lane, so that they still put a few wavefronts
-//     on every SIMD (FP16: a tile's three wavefronts share a workgroup, which
-//     finds the site norms).  Solves, ms, Short against long: 8^3x16 even-odd,
-//     one FP64 rhs, GCR(32) 1.31 / 1.70, three FP32, GCR(16) 0.98 / 1.05, one
-//     FP16, GCR(12) 1.13 / 1.21, twelve, GCR(32) 3.84 / 3.88.  9216 sites: FP64
-//     1.55 / 1.81, FP32 1.28 / 1.30, FP16 1.22 / 1.30 but twelve 5.83 / 5.60;
-//     16 128 sites: FP64 and FP32 2% slower.
+//   Short FP64 and FP32 vectors: one chunk per lane, so that they still put a few
+//     wavefronts on every SIMD.  Solves, ms, Short against long: 8^3x16 even-odd,
+//     one FP64 rhs, GCR(32) 1.31 / 1.70, three FP32, GCR(16) 0.98 / 1.05.  9216
+//     sites: FP64 1.55 / 1.81, FP32 1.28 / 1.30; 16 128 sites: both 2% slower.
+//   FP16 vectors: one chunk per lane at every length; a tile's three wavefronts
+//     share a workgroup, which finds the site norms.  (One vector in flight in the
+//     update against two: 0.1 to 1% slower up to 8^3x16, as much faster from 12^3x24.)
 //   Long ones: what measured best, us per launch (12 FP16 rhs, GCR(12), 24^3x48;
 //     one FP64 rhs, GCR(32), 16^3x32; three FP32, GCR(16), 16^3x24, even-odd).
 //     FP16 dots: a third of a site, two vectors 496, one 508, three 618, a whole
@@ -1000,12 +1000,8 @@ struct GcrShapes;
 template <>
 struct GcrShapes<QCD_HIP_F16> {
   static constexpr int S = 4;   // steps of a block
-  using Short = GcrShape<1, 2, 192, true>;
-  using Dots = Short;
+  using Dots = GcrShape<1, 2, 192, true>;
   using Update = GcrShape<1, 1, 192, true>;
-  using Short8 = Short;   // (not used)
-  using Dots8 = Dots;
-  using Update8 = Update;
 };
 template <>
 struct GcrShapes<QCD_HIP_F32> {
@@ -1033,18 +1029,21 @@ unsigned gcr_blocks(int prec, long V) {
   const long waves = (V + kTile - 1) / kTile * (kG / SH::M);
   return (unsigned)((waves + SH::BLK / 64 - 1) / (SH::BLK / 64));
 }
-template <int P>
-constexpr bool gcr_short(long V) { return V <= (P == QCD_HIP_F16 ? 4096 : 12288); }
 // f(shape, grid) of a launch over count vectors of V sites (DOTS: the dots'
 // shape, else that of the kernels without sums) in a block of ST steps
 template <int P, int ST, bool DOTS, typename F>
 void gcr_launch(long V, int count, F f) {
   using G = GcrShapes<P>;
   auto call = [&](auto sh) { f(sh, dim3(gcr_blocks<decltype(sh)>(P, V), (unsigned)count)); };
-  constexpr bool B8 = ST == 8;
-  if (gcr_short<P>(V)) call(std::conditional_t<B8, typename G::Short8, typename G::Short>{});
-  else if constexpr (DOTS) call(std::conditional_t<B8, typename G::Dots8, typename G::Dots>{});
-  else call(std::conditional_t<B8, typename G::Update8, typename G::Update>{});
+  constexpr long kShort = 12288;
+  if constexpr (P == QCD_HIP_F16) call(std::conditional_t<DOTS, typename G::Dots, typename G::Update>{});
+  else if constexpr (ST == 8) {
+    if (V <= kShort) call(typename G::Short8{});
+    else call(std::conditional_t<DOTS, typename G::Dots8, typename G::Update8>{});
+  } else {
+    if (V <= kShort) call(typename G::Short{});
+    else call(std::conditional_t<DOTS, typename G::Dots, typename G::Update>{});
+  }
 }
 // f(block size constant) for the next block of a cycle with left steps to go
 template <int P, typename F>
