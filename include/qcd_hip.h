@@ -108,13 +108,17 @@ int qcd_hip_dslash_time(qcd_hip_field out, qcd_hip_field in, qcd_hip_field gauge
  * next step's centre, 5 | (n << 8) = traversal 2 with two rhs per lane for
  * FP32/FP16 batches with the D or Q epilogue, 6 = FP16 batches on the
  * matrix cores: MFMA applies each link to the spin-projected neighbour
- * spinors of 4 rhs per wavefront of 16 sites) and occupancy variant (0 = compiler default, 2 or 3 =
+ * spinors of 4 rhs per wavefront of 16 sites, 7 = one wavefront per hop for
+ * launches of few sites) and occupancy variant (0 = compiler default, 2 or 3 =
  * at least that many waves per SIMD, 16 = scheduling fences between hop
  * directions) on these fields and keep the fastest for their (lattice
  * extents, precisions).  Runs by itself on first use unless the environment
  * sets QCD_HIP_AUTOTUNE=0.  All candidates give bit-identical results. */
 int qcd_hip_dslash_tune(qcd_hip_field out, qcd_hip_field in, qcd_hip_field gauge, int tuned[2], double *ms);
 int qcd_hip_dslash_set_config(qcd_hip_field in, qcd_hip_field gauge, int map, int occ);
+/* The traversal that qcd_hip_dslash takes now for count rhs of these fields,
+ * -1 before they are tuned. */
+int qcd_hip_dslash_chosen(qcd_hip_field in, qcd_hip_field gauge, int count);
 /* The traversal candidates (map values above) the autotuner times: fills up
  * to max entries of maps and returns how many there are. */
 int qcd_hip_dslash_candidates(int *maps, int max);

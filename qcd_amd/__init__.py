@@ -129,6 +129,7 @@ def lib():
         "qcd_hip_dslash_time": (i, [_vp, _vp, _vp, d, d, i, i, i, _dp]),
         "qcd_hip_dslash_tune": (i, [_vp, _vp, _vp, ctypes.POINTER(ctypes.c_int), _dp]),
         "qcd_hip_dslash_set_config": (i, [_vp, _vp, i, i]),
+        "qcd_hip_dslash_chosen": (i, [_vp, _vp, i]),
         "qcd_hip_dslash_candidates": (i, [ctypes.POINTER(ctypes.c_int), i]),
         "qcd_hip_gauss_smear": (i, [_vp, _vp, d, i, i]),
         "qcd_hip_norm2": (i, [_vp, i, _dp]),
@@ -427,6 +428,11 @@ def dslash_candidates():
     buf = (ctypes.c_int * n)()
     lib().qcd_hip_dslash_candidates(buf, n)
     return list(buf)
+
+
+def dslash_chosen(inp, gauge, count=1):
+    """The traversal that D and Q over count rhs take now (7: one wavefront per hop), -1 before tuning."""
+    return int(lib().qcd_hip_dslash_chosen(inp.h, gauge.h, int(count)))
 
 
 def dslash_set_config(inp, gauge, map_, occ):

@@ -666,6 +666,7 @@ struct TuneVal {
   // D and Q without reduction take one wavefront per hop (split.hip) where that
   // was faster: one rhs, and batches (if they were timed)
   bool split = false, btimed = false, bsplit = false;
+  bool forced = false;   // set by qcd_hip_dslash_set_config: batches of any count too
 };
 static std::vector<std::pair<TuneKey, TuneVal>> g_tune;
 static int g_autotune = -1;   // -1: read QCD_HIP_AUTOTUNE once
@@ -764,6 +765,15 @@ static const long kSplitSites = 1L << 20;
 // 103; FP32, 249 480 sites, 3 rhs 96.7 / 93.8).
 static const int kSplitRhs = 4;
 static const float kSplitGain = 0.92f;
+
+// whether D or Q without reduction of count rhs takes one wavefront per hop.
+// Batches that were not timed (a lattice tuned on one rhs) take it while they are
+// small, and within the same count.
+static bool takes_split(const TuneVal &t, long V, int count) {
+  if (t.forced) return V * count <= kSplitSites;
+  if (count == 1) return t.split;
+  return count <= kSplitRhs && (t.btimed ? t.bsplit : t.split && V * count <= (1L << 16));
+}
 
 static DslashArgs batch_args(qcd_hip_lattice lat, double m, double tm, const Batch &bt) {
   DslashArgs a = make_args(lat, m, tm);
@@ -988,7 +998,7 @@ int dslash_launch(int epi, bool red, qcd_hip_field out, int ro, qcd_hip_field in
                   qcd_hip_field b, int rb, double m, double tm, double *partials, hipStream_t stream, int *grid_out) {
   TuneVal t;
   const bool have = tune_get(key_of(in, g), &t);
-  if (have && t.split && !red && (epi == EPI_D || epi == EPI_Q))
+  if (have && !red && (epi == EPI_D || epi == EPI_Q) && takes_split(t, in->lat->V, 1))
     return dslash_split_launch(epi, batch_args(in->lat, m, tm, kOne), out, ro, in, ri, g, stream);
   const int map = have ? t.map : kDefaultMap, occ = have ? t.occ : 0;
   return launch_cfg(epi, red, map, occ, out, ro, in, ri, g, b, rb, m, tm, partials, stream, grid_out);
@@ -1007,11 +1017,8 @@ int dslash_launch_batch(int epi, bool red, qcd_hip_field out, int ro, int out_rs
   const bool two = have && count >= 2 && t.bmap != 0 && timed;
   const int map = two ? t.bmap : have ? t.map : kDefaultMap, occ = two ? t.bocc : have ? t.occ : 0;
   const Batch bt{ids, count, in_rs, out_rs, b_rs};
-  // (batches of a lattice tuned on one rhs: only while they are small as well)
-  const bool split = have && !red && (epi == EPI_D || epi == EPI_Q) &&
-                     (count == 1 ? t.split : t.btimed ? t.bsplit && count <= kSplitRhs
-                                                      : t.split && in->lat->V * count <= (1L << 16));
-  if (split) return dslash_split_launch(epi, batch_args(in->lat, m, tm, bt), out, ro, in, ri, g, stream);
+  if (have && !red && (epi == EPI_D || epi == EPI_Q) && takes_split(t, in->lat->V, count))
+    return dslash_split_launch(epi, batch_args(in->lat, m, tm, bt), out, ro, in, ri, g, stream);
   return launch_cfg(epi, red, map, occ, out, ro, in, ri, g, b, rb, m, tm, partials, stream, grid_out, bt);
 }
 
@@ -1209,26 +1216,38 @@ int qcd_hip_dslash_candidates(int *maps, int max) {
 // 1 y-slab per XCD, 2 | (n << 8) z-march of n steps, 3 | (n << 8) z-march of
 // n steps with LDS-staged t and x neighbours, 4 | (n << 8) z-march with the
 // forward z neighbour carried in LDS, 5 | (n << 8) z-march with two rhs per
-// lane (batches of FP32/FP16 D or Q; otherwise the one-rhs z-march); occ = 0
-// compiler default, 2 or 3 minimum waves per SIMD, 16 scheduling fence
+// lane (batches of FP32/FP16 D or Q; otherwise the one-rhs z-march), 6 matrix
+// cores, 7 one wavefront per hop (D and Q of equal precisions and up to 2^20
+// (site, rhs) pairs; otherwise the z-march of 6 steps); occ = 0 compiler default, 2 or 3 minimum waves per SIMD, 16 scheduling fence
 // between hop directions.
 int qcd_hip_dslash_set_config(qcd_hip_field in, qcd_hip_field gauge, int map, int occ) {
   QH_TRY(ensure_init());
   const int m0 = map & 0xff;
-  if (!in || !gauge || m0 < 0 || m0 > 6 || (m0 >= 2 && m0 <= 5 && (map >> 8) < 1) ||
+  if (!in || !gauge || m0 < 0 || m0 > 7 || (m0 >= 2 && m0 <= 5 && (map >> 8) < 1) ||
       (occ != 0 && occ != 2 && occ != 3 && occ != 16)) {
     set_error("dslash_set_config: bad arguments");
     return 1;
   }
   const TuneKey k = key_of(in, gauge);
+  TuneVal t{m0 == 7 ? kDefaultMap : map, occ, 0.f};   // forced: batches use the same traversal
+  t.forced = m0 == 7 && in->prec == gauge->prec;
   std::lock_guard<std::recursive_mutex> lock(state_mutex());
   for (auto &e : g_tune)
     if (e.first == k) {
-      e.second = TuneVal{map, occ, 0.f};
+      e.second = t;
       return 0;
     }
-  g_tune.push_back({k, TuneVal{map, occ, 0.f}});   // forced: batches use the same traversal
+  g_tune.push_back({k, t});
   return 0;
+}
+
+// The traversal that D and Q over count rhs take now (7: one wavefront per hop),
+// -1 before they are tuned.
+int qcd_hip_dslash_chosen(qcd_hip_field in, qcd_hip_field gauge, int count) {
+  TuneVal t;
+  if (!in || !gauge || count < 1 || !tune_get(key_of(in, gauge), &t)) return -1;
+  if (takes_split(t, in->lat->V, count)) return 7;
+  return count >= 2 && t.bmap != 0 ? t.bmap : t.map;
 }
 
 }  // extern "C"
