@@ -70,6 +70,7 @@ std::recursive_mutex &state_mutex();
 int ensure_init();
 // copy between device and pageable host memory (up: to the device), on st
 hipError_t host_copy(void *dev, void *host, size_t bytes, bool up, hipStream_t st);
+void host_slots_free();               // the pinned memory host_copy keeps
 int dev_alloc(void **p, size_t bytes);
 void dev_free(void *p, size_t bytes);
 int gauge_create_unfilled(qcd_hip_field *f, qcd_hip_lattice lat);
