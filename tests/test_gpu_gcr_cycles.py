@@ -151,3 +151,34 @@ def test_a_cycle_reaches_the_least_residual(gpu, prec, eps, op, eo, kappa, mu, p
         r = _one_cycle(Q, L, b, kappa, mu, op, eo, prec, n)
         assert r <= 1.02 * ref[n] + 4 * eps * np.sqrt((ref[:n]**2).sum()) + 1e-15
         assert r >= 0.98 * ref[n] - 2 * eps - 1e-15   # (1e-15: the reference's own rounding)
+
+
+# 12 288 sites, the longest short vectors of FP32 and FP64, and longer ones whose
+# last tile has 60, 58, 4 and (half lattice) 56 of 64 sites
+@pytest.mark.parametrize("L,op,eo", [((16, 16, 6, 8), "D", 0), ((14, 21, 6, 7), "D", 0), ((15, 13, 9, 14), "Q", 0),
+                                     ((30, 21, 18, 11), "D", 0), ((10, 6, 14, 30), "D", 1)])
+@pytest.mark.parametrize("prec,eps", [("f64", 2.0**-53), ("f32", 2.0**-24), ("f16", 2.0**-11)])
+def test_long_vectors_with_partial_tiles(gpu, L, op, eo, prec, eps):
+    """Blocks of 8 (FP16: 4), 4, 2 and 1: the least residual, and the same bits
+    alone and in a batch."""
+    Q = gpu
+    kappa, mu, n = 0.12, 0.04, 15
+    lat, g = Q.Lattice(L), Q.Gauge(Q.Lattice(L)).upload(O.gauge_generate(L, EPS, 61))
+    b = [_source(L, 0), O.spinor_gaussian(L, 63)]
+    fb, sols = Q.Spinor(lat, nrhs=2), []
+    for r in range(2):
+        fb.upload(b[r], rhs=r)
+    # (a tuned FP16 batch may take the matrix cores, which round differently)
+    Q.dslash_set_config(Q.Spinor(lat, Q.PREC[prec]), Q.Gauge(lat, Q.PREC[prec]), 2 | (4 << 8), 0)
+    for batch in (1, 2):
+        fx = Q.Spinor(lat, nrhs=2)
+        S = Q.Solver(lat, g, n_restart=n, tol=1e-15, inner_prec=prec, op=op, eo=eo, max_outer=1, batch=batch)
+        S.solve(fx, fb, kappa, mu, check=False)
+        S.close()
+        sols.append([fx.download(r) for r in range(2)])
+    for r in range(2):
+        assert np.array_equal(sols[0][r], sols[1][r])
+    ref = _least_residuals(L, op, eo, kappa, mu, 0, n)
+    res = O.b_minus_Dx(O.Geometry(L), sols[0][0], b[0], O.gauge_generate(L, EPS, 61), kappa, mu)
+    assert res <= 1.02 * ref[n] + 4 * eps * np.sqrt((ref[:n]**2).sum()) + 1e-15
+    assert res >= 0.98 * ref[n] - 2 * eps
