@@ -22,7 +22,9 @@ __device__ __forceinline__ C cm(C a, C b) { return C{fma(a.re, b.re, -(a.im * b.
 __device__ __forceinline__ C cj(C a) { return C{a.re, -a.im}; }
 
 // c (+)= a b (DA: a^+, DB: b^+; ADD: added to c): a chain of fused
-// multiply-adds per element, 108 instructions
+// multiply-adds per element, 108 instructions.  An element's product is summed
+// from zero and then added: a chain that starts from c rounds each of its terms
+// at the size of a whole staple sum.
 template <bool DA, bool DB, bool ADD = false>
 __device__ __forceinline__ void mm3(C c[9], const C a[9], const C b[9]) {
 #pragma unroll
@@ -34,31 +36,21 @@ __device__ __forceinline__ void mm3(C c[9], const C a[9], const C b[9]) {
       for (int k = 0; k < 3; k++) {
         const C x = DA ? cj(a[3 * k + i]) : a[3 * i + k];
         const C y = DB ? cj(b[3 * j + k]) : b[3 * k + j];
-        if (k == 0 && !ADD) {
-          re = x.re * y.re;
-          im = x.re * y.im;
-        } else {
-          re = fma(x.re, y.re, k == 0 ? c[3 * i + j].re : re);
-          im = fma(x.re, y.im, k == 0 ? c[3 * i + j].im : im);
-        }
+        re = k == 0 ? x.re * y.re : fma(x.re, y.re, re);
+        im = k == 0 ? x.re * y.im : fma(x.re, y.im, im);
         re = fma(-x.im, y.im, re);
         im = fma(x.im, y.re, im);
       }
-      c[3 * i + j] = C{re, im};
+      c[3 * i + j] = ADD ? C{c[3 * i + j].re + re, c[3 * i + j].im + im} : C{re, im};
     }
 }
 
-// 1 / x and 1 / sqrt(x) for normal x > 0: the hardware's approximation and
-// two Newton steps.  Zero, infinity and NaN give infinity, zero or NaN.
+// 1 / x for normal x > 0: the hardware's approximation and two Newton steps.
+// Zero, infinity and NaN give NaN.
 __device__ __forceinline__ double recip(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(fma(-x, r, 1.0), r, r);
   return fma(fma(-x, r, 1.0), r, r);
-}
-__device__ __forceinline__ double rsqrt_pos(double x) {
-  double r = __builtin_amdgcn_rsq(x);
-  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
-  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
 }
 
 // cofactor of element (r, c) of a 3x3 matrix
@@ -80,13 +72,19 @@ __device__ __forceinline__ C cof3(const C x[9], int r, int c) {
 //  * an unscaled step that changed X by D leaves an error of |D|^2 / 2, so
 //    the loop ends at |D|^2 <= 1e-17 without a step that confirms it;
 //  * the phase exp(-i arg(det M) / 3) starts from single precision and takes two
-//    Newton steps z <- z (4 - z^3 conj(w)) / 3 for z^3 = w, |w| = 1.
-// 24^3x48: an APE step 446-468 -> 322 us with these and the fused products.
+//    Newton steps z <- z + z (1 - z^3 det X) / 3 on the determinant of the X
+//    reached, not of M: every step's rounding turns X by a common phase too, and
+//    leaves a common factor, which z takes out.
+// 24^3x48: an APE step 446-468 -> 322 us with these and the fused products.  Error
+// of a step on generated fields (eps 0.1, 0.3, 1.0), rms over the links: 4.0, 5.3,
+// 10.1e-17; with the phase of det M, the last factor as z (4 - t) / 3 and the
+// products added into the staple sum term by term 7.3, 8.7, 15.6e-17; with sin, cos
+// and atan2 and a confirming step 5.6, 6.9, 12.3e-17.
 __device__ __forceinline__ void project_su3(C m[9]) {
   C x[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) x[k] = m[k];
-  C w{0.0, 0.0};   // conj(det M) / |det M|
+  C w{0.0, 0.0};   // det M, normalised for the range of FP32
   double diff = 1.0;
   for (int it = 0; it < 100; it++) {
     // y = (x^-1)^+ = conj(cofactor(x)) / conj(det x)
@@ -101,8 +99,8 @@ __device__ __forceinline__ void project_su3(C m[9]) {
       d = C{fma(x[c].re, y[c].re, fma(-x[c].im, y[c].im, d.re)), fma(x[c].re, y[c].im, fma(x[c].im, y[c].re, d.im))};
     const double dd = fma(d.re, d.re, d.im * d.im);
     if (it == 0) {
-      const double rd = rsqrt_pos(dd);
-      w = C{d.re * rd, -(d.im * rd)};
+      const double rd = __builtin_amdgcn_rsq(dd);
+      w = C{d.re * rd, d.im * rd};
     }
     const double rdd = recip(dd);
     double g = 0.5, rg = 0.5;
@@ -137,12 +135,19 @@ __device__ __forceinline__ void project_su3(C m[9]) {
     }
     if (!scale && diff <= 1e-17) break;
   }
-  const float ph = -atan2f((float)-w.im, (float)w.re) / 3.0f;
+  C d{0.0, 0.0};   // det X
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const C y = cof3(x, 0, c);
+    d = C{fma(x[c].re, y.re, fma(-x[c].im, y.im, d.re)), fma(x[c].re, y.im, fma(x[c].im, y.re, d.im))};
+  }
+  const float ph = -atan2f((float)w.im, (float)w.re) / 3.0f;
   C z{(double)__cosf(ph), (double)__sinf(ph)};
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const C t = cm(cm(cm(z, z), z), cj(w));
-    z = cm(z, C{(4.0 - t.re) * (1.0 / 3.0), t.im * (-1.0 / 3.0)});
+    const C t = cm(cm(cm(z, z), z), d);
+    const C e{(1.0 - t.re) * (1.0 / 3.0), t.im * (-1.0 / 3.0)};
+    z = C{fma(z.re, e.re, fma(-z.im, e.im, z.re)), fma(z.re, e.im, fma(z.im, e.re, z.im))};
   }
 #pragma unroll
   for (int k = 0; k < 9; k++) m[k] = cm(x[k], z);
