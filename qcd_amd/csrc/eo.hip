@@ -649,8 +649,13 @@ static int eo_launch_pp(int epi, bool red, const EoArgs &e, dim3 gr, qcd_hip_fie
   // 16^3x32, one rhs (65 536 items) FP64 6.31 -> 6.25, FP32 3.68 -> 3.59, FP16
   // 2.67 -> 2.76.
   const double items = (double)e.d.count * e.Vh;
+  // Not FP64 launches that fill the 256 CUs with one round of one-site workgroups:
+  // 8 rhs of 16x12x10x8 (240 workgroups) 3.35 against 3.24 ms, 3 of 12^3x24 (243) 3.49
+  // and 3.39, 2 of 16^4 (256) 3.69 and 3.53; 12 of 8^3x16 (192) 2.81 and 2.84, 3 of
+  // 16^4 (384) 4.90 and 5.11.
   const bool may_split = !red && eo_zlen_setting().load() == 0;
-  if (may_split && items < (PS == QCD_HIP_F16 ? 65536.0 : 131072.0))
+  const bool one_round = PS == QCD_HIP_F64 && gr.x > 208 && gr.x <= 256;
+  if (may_split && !one_round && items < (PS == QCD_HIP_F16 ? 65536.0 : 131072.0))
     return eo_split_launch(epi, e, out, ro, in, ri, g, b, rb, st);
   const bool two = PS != QCD_HIP_F64 && e.d.count >= 2 && !red && (epi == EO_MINV || epi == EO_SCHUR) &&
                    eo_two_rhs();
