@@ -341,17 +341,23 @@ __global__ void __launch_bounds__(kBlock) k_gauss_gather_links(GaussArgs g, cons
 // z steps per lane of k_gauss for a launch over `sites` (site, rhs) pairs: the
 // march saves loads but divides the wavefronts, so it is as long as leaves about
 // 4096 of them (four per SIMD): one step below kGaussTile, a few for whole FP16
-// fields.  Calls of 50 iterations with their sources, ms: 16^3, 12 FP64 rhs 0.77
+// fields, but four at most (10 iterations, us, 1, 2, 4, 8 steps: 12 rhs of 16^3x32 985,
+// 909, 882, 910; 5 of 32^3x16 1652, 1517, 1466, 1523; 12 of 24^3x48 4810, 4300, 4058,
+// 4102; one of 24^3x48 501, 484, 479, 582).  Calls of 50 iterations with their sources, ms: 16^3, 12 FP64 rhs 0.77
 // with 1 step, 1.23 with 4; 32^3, one rhs 0.58 with 1, 1.99 with 8.  (Lanes of one
 // spin each, without a march and with every hop's loads in flight, gain on 8^3
 // only.)  QCD_HIP_GAUSS_ZLEN overrides it, for launches of every size.
-static unsigned gauss_zlen(unsigned Z, long sites) {
+static int gauss_zlen_set() {   // 0: not set
   static const int env = [] {
     const char *e = std::getenv("QCD_HIP_GAUSS_ZLEN");
     return e ? std::atoi(e) : 0;
   }();
+  return env > 0 ? env : 0;
+}
+static unsigned gauss_zlen(unsigned Z, long sites) {
+  const int env = gauss_zlen_set();
   const long per = 4096L * 64;
-  const unsigned r = env > 0 ? (unsigned)env : (unsigned)std::max(1L, std::min((sites + per / 2) / per, (long)Z));
+  const unsigned r = env > 0 ? (unsigned)env : (unsigned)std::max(1L, std::min((sites + per / 2) / per, 4L));
   return r > Z ? Z : r;
 }
 
@@ -439,7 +445,7 @@ static int gauss_run(qcd_hip_field v, qcd_hip_field gauge, qcd_hip_field buf, in
   const GaugeIn<P> U = GaugeIn<P>::of(links);
   const unsigned nb = (unsigned)grid_for(g.n);
   const long pairs = (long)g.n * std::min(rows, v->nrhs), columns = (long)g.tn * g.X * g.Y;
-  const bool tile = pairs >= kGaussTile && !(P == QCD_HIP_F16 && g.tn > 1) && !std::getenv("QCD_HIP_GAUSS_ZLEN");
+  const bool tile = pairs >= kGaussTile && !(P == QCD_HIP_F16 && g.tn > 1) && gauss_zlen_set() == 0;
   const int block = tile ? kGaussBlock : kBlock;
   g.ncb = (unsigned)grid_for(columns, block);
   g.zlen = tile ? gauss_tile_zlen(P, g.Z, (long)g.ncb * std::min(rows, v->nrhs)) : gauss_zlen(g.Z, pairs);
