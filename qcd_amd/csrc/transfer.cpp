@@ -7,6 +7,8 @@
 // one is on the bus while the other is filled or emptied.  75 MB up 2530 -> 1800
 // us (chunks of 4 MB; 1 MB 2440, 8 MB 1810; one thread 2640, four 1810), 25 MB
 // up 673 -> 650, down 1416 -> 742 (chunks of 2 MB; 4 MB 771; one thread 970).
+// The shortest that gain, us: up 8.8 MB 271 -> 310, 9.8 300 -> 350, 11.8 378 -> 387,
+// 13.8 495 -> 433; down 8.8 MB 519 -> 364.
 // The slots (16 MB) are kept and given back by qcd_hip_release_cache.  All calls
 // hold state_mutex.  The calling thread's current device need not be the library's
 // (streams name their device; memory and events take the current one), and is left
@@ -17,7 +19,8 @@
 
 namespace qcdhip {
 
-constexpr size_t kSlotBytes = (size_t)4 << 20, kDownChunk = (size_t)2 << 20, kHostMin = (size_t)8 << 20;
+constexpr size_t kSlotBytes = (size_t)4 << 20, kDownChunk = (size_t)2 << 20;
+constexpr size_t kUpMin = (size_t)12 << 20, kDownMin = (size_t)8 << 20;
 struct HostSlots {
   char *mem = nullptr;   // four slots: two of the caller, two of the helper
   hipEvent_t ev[4] = {};
@@ -99,7 +102,7 @@ static hipError_t copy_chunks(char *dev, char *host, size_t bytes, size_t chunk,
 // Copy between device and host on st.  The caller holds state_mutex and waits
 // for st before it touches or frees either side.
 hipError_t host_copy(void *dev, void *host, size_t bytes, bool up, hipStream_t st) {
-  if (bytes < kHostMin || !pageable(host) || !slots_ready())
+  if (bytes < (up ? kUpMin : kDownMin) || !pageable(host) || !slots_ready())
     return up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st)
               : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
   const size_t chunk = up ? kSlotBytes : kDownChunk;

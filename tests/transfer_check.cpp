@@ -49,16 +49,19 @@ int main() {
   context.device = 1;
   for (int pass = 0; pass < 3; pass++) {
     no_memory = pass == 2;   // the runtime's copy
-    for (size_t n : {(size_t)1000, (size_t)8 << 20, ((size_t)8 << 20) + 24, (size_t)20971528}) {
+    const size_t MB = (size_t)1 << 20;
+    for (size_t n : {(size_t)1000, 8 * MB - 24, 8 * MB, 12 * MB - 24, 12 * MB, 12 * MB + 24, (size_t)20971528}) {
       std::vector<char> host(n), dev(n, 0), back(n, 0);
       for (size_t i = 0; i < n; i++) host[i] = (char)(i * 2654435761u >> 13);
       copies = 0;
       CHECK(qcdhip::host_copy(dev.data(), host.data(), n, true, &stream) == hipSuccess);
       CHECK(dev == host);
+      CHECK((copies > 1) == (n >= 12 * MB && !no_memory));
+      copies = 0;
       CHECK(qcdhip::host_copy(dev.data(), back.data(), n, false, &stream) == hipSuccess);
       CHECK(back == host);
       CHECK(current == 0);
-      CHECK((copies > 2) == (n >= ((size_t)8 << 20) && !no_memory));
+      CHECK((copies > 1) == (n >= 8 * MB && !no_memory));
     }
     CHECK(allocations == (no_memory ? 0 : 1) && events == (no_memory ? 0 : 4));
     qcdhip::host_slots_free();
