@@ -973,8 +973,10 @@ namespace {
 //     one FP64 rhs, GCR(32) 1.31 / 1.70, three FP32, GCR(16) 0.98 / 1.05.  9216
 //     sites: FP64 1.55 / 1.81, FP32 1.28 / 1.30; 16 128 sites: both 2% slower.
 //   FP16 vectors: one chunk per lane at every length; a tile's three wavefronts
-//     share a workgroup, which finds the site norms.  (One vector in flight in the
-//     update against two: 0.1 to 1% slower up to 8^3x16, as much faster from 12^3x24.)
+//     share a workgroup, which finds the site norms.  Two vectors in flight in the
+//     dots; in the kernels without sums too up to 4096 sites, one from there (8^3x16,
+//     twelve, GCR(32): k_solution 17.5 against 23.0 us, the solve 2.82 against 2.84 ms;
+//     16^3x32 20.45 against 20.14).
 //   Long ones: what measured best, us per launch (12 FP16 rhs, GCR(12), 24^3x48;
 //     one FP64 rhs, GCR(32), 16^3x32; three FP32, GCR(16), 16^3x24, even-odd).
 //     FP16 dots: a third of a site, two vectors 496, one 508, three 618, a whole
@@ -1036,8 +1038,10 @@ void gcr_launch(long V, int count, F f) {
   using G = GcrShapes<P>;
   auto call = [&](auto sh) { f(sh, dim3(gcr_blocks<decltype(sh)>(P, V), (unsigned)count)); };
   constexpr long kShort = 12288;
-  if constexpr (P == QCD_HIP_F16) call(std::conditional_t<DOTS, typename G::Dots, typename G::Update>{});
-  else if constexpr (ST == 8) {
+  if constexpr (P == QCD_HIP_F16) {
+    if (DOTS || V <= 4096) call(typename G::Dots{});
+    else call(typename G::Update{});
+  } else if constexpr (ST == 8) {
     if (V <= kShort) call(typename G::Short8{});
     else call(std::conditional_t<DOTS, typename G::Dots8, typename G::Update8>{});
   } else {
