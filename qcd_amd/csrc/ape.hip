@@ -313,9 +313,10 @@ __device__ __forceinline__ unsigned bwd_dir(unsigned mu, const Site &st, const D
 // holds the planes z - 1, z, z + 1 of its slab and the links that the
 // directions share in its L2.  24^3x48, against site order with the directions
 // as separate passes and the same arithmetic (us a step): APE 322 -> 286,
-// stout 440 -> 415.  What bounds them now is traffic between L2 and the fabric
-// (1.6 GB read for 0.29 GB of spatial links an APE step) together with the
-// FP64 pipes, busy 42% of the time.  Tried and slower: rows of the products
+// stout 440 -> 415.  What bounds APE now is traffic between L2 and the fabric
+// (1.6 GB read for 0.29 GB of spatial links a step, 6.3 TB/s with the writes)
+// together with the FP64 pipes, busy 48% of the time; a 4d stout step reads 1.5 GB
+// for 0.38 at 4.0 TB/s, pipes 44%, with two wavefronts per SIMD (224 VGPRs).  Tried and slower: rows of the products
 // formed one at a time (fewer registers, 3-4 wavefronts per SIMD), separate
 // loops over backward and forward stout staples (3 wavefronts).
 struct SlabOrder {

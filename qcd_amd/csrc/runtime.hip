@@ -1,4 +1,4 @@
-// runtime.hip -- context, errors, lattices, fields, host<->device transfer,
+// runtime.hip -- context, errors, lattices, fields and their transfer,
 // precision conversion and the synthetic-input generator.
 #include "internal.h"
 #include "generator.h"

@@ -291,19 +291,27 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
 // them and formed in a second one, where single steps take 2 S passes, and these
 // passes are what a cycle spends its time on (bound by the rate of the fabric, 6.0-6.7 TB/s).  Solves with blocks of 1, 2, 4
 // and 8, ms: one FP64 rhs, Q, GCR(32) on 16^3x32 204, 126, 87, 69; one FP32 rhs
-// 4: 20.8, 8: 17.3; 12 FP16 rhs, GCR(12) on 24^3x48 132, 107, 96, 97, on 16^3x32
-// 21.0, 16.9, 15.0, 16.0.  FP16 stays at 4: its dots are bound by arithmetic, which
-// blocks do not save, and eight steps carry up to twice the rounding of single
-// ones into long cycles.
+// 4: 20.8, 8: 17.3; 12 FP16 rhs, GCR(12), 1, 2, 4 steps: on 24^3x48 136, 111, 98, on
+// 16^3x32 21.8, 17.5, 15.4.  FP16 stays at 4: its dots are bound by arithmetic, which
+// blocks do not save (8 steps, with cheaper dots, 97 against 96 and 16.0 against
+// 15.0), and eight steps carry up to twice the rounding of single ones into long
+// cycles.
 //
 // theta is the local term m + 4 of D and of the Schur complement (0 for Q): the
 // d_a are then, but for factors, the residuals of Richardson's iteration, about
 // as independent of each other as the residuals of single steps, and a long FP16
 // cycle reaches the same residual: GCR(32) on 8^3x16, kappa 0.125, 4.0e-4 of the
-// one before, single steps 4.9e-4 (d_1 without theta 8.1e-4).  The outer step
-// counts are those of single steps for FP64, FP32 and FP16, Q and D, GCR(4) to
-// GCR(64), kappa 0.1 to 0.139, random and point sources, where single steps
-// converge (FP16 with 64 steps: one cycle more or less).
+// one before, single steps 4.9e-4 (d_1 without theta 8.1e-4).  A cycle reaches
+// the least residual of its Krylov space to 2% and the rounding of the stored w_j,
+// but for Q beyond 27 steps in FP16 and 40 in FP32, where they lose orthogonality.
+// Outer steps against the earlier single steps, which took them from the stored
+// w_k: 672 solves each, GCR(8) to GCR(64), kappa 0.1 to 0.139, mu 0 to 0.2, D, Q and
+// the Schur complement, random and point sources: FP64 the same or fewer; FP32 one
+// more in 3, fewer in 57; FP16 more in 33, all Q, fewer in 278.  Most of the 33 are
+// restarted cycles at kappa 0.139 that came out shorter with the rounding of those
+// single steps (8^3x16, GCR(24): 97; in blocks of 1, 2 and 4 141, as in FP64).  Heavy quarks on Q
+// leave directions of a block out: FP64, kappa 0.005, GCR(16) takes 2 cycles of
+// blocks for one of single steps.
 
 // Smallest |w_{k+a}|^2 / |v_a|^2 that is told from rounding of the stored vectors:
 // a v_a with less to itself is left out of the cycle
@@ -342,8 +350,8 @@ __device__ __forceinline__ double norm2(double2 a) { return a.x * a.x + a.y * a.
 // block cannot take more off |res_k|^2 than there is (Bessel): sums that claim so
 // by more than kExcess of it come from vectors that are not orthogonal, and leave
 // their own block and the rest out.  (FP16, Q, mu = 0.04, point source, 8x6x4x6,
-// one cycle of 40 steps: 0.36 of the residual without this, 0.016 with it; a
-// block that is too long without claiming too much can still double |res|.)  A
+// one cycle of 40 steps: 0.36 of the residual without this, 0.016 with it.)  What
+// neither sees is a last block that is too long without claiming too much.  A
 // residual of exactly 0 (heavy quarks: FP16 vectors of a few steps) ends the
 // cycle as well.  prev: steps of the block before.
 //
