@@ -1218,8 +1218,9 @@ int qcd_hip_dslash_candidates(int *maps, int max) {
 // forward z neighbour carried in LDS, 5 | (n << 8) z-march with two rhs per
 // lane (batches of FP32/FP16 D or Q; otherwise the one-rhs z-march), 6 matrix
 // cores, 7 one wavefront per hop (D and Q of equal precisions and up to 2^20
-// (site, rhs) pairs; otherwise the z-march of 6 steps); occ = 0 compiler default, 2 or 3 minimum waves per SIMD, 16 scheduling fence
-// between hop directions.
+// (site, rhs) pairs; otherwise the z-march of 6 steps); occ = 0 compiler
+// default, 2 or 3 minimum waves per SIMD, 16 scheduling fence between hop
+// directions.
 int qcd_hip_dslash_set_config(qcd_hip_field in, qcd_hip_field gauge, int map, int occ) {
   QH_TRY(ensure_init());
   const int m0 = map & 0xff;

@@ -613,8 +613,8 @@ static int eo_launch_z(int epi, bool red, const EoArgs &e, unsigned zlen, bool t
 // (row, half-site) items that may run twice (not under graph capture, out
 // aliasing neither in nor b) times chunks of 1 to 12 planes and keeps the
 // fastest; smaller launches take one wavefront per hop or one site per lane
-// (eo_launch_pp).  All give bit-identical results.  Timing rather than a formula: how the grid fills the 256 CUs
-// decides (24^3x48, one FP64 rhs: 289 us at 6 steps, 423 at 5, 383 at 1).
+// (eo_launch_pp).  All give bit-identical results.  Timing rather than a
+// formula: how the grid fills the 256 CUs decides (24^3x48, one FP64 rhs: 289 us at 6 steps, 423 at 5, 383 at 1).
 struct EoZKey {
   int L[4], ps, nr;
   unsigned rows;

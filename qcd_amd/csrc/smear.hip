@@ -343,7 +343,8 @@ __global__ void __launch_bounds__(kBlock) k_gauss_gather_links(GaussArgs g, cons
 // 4096 of them (four per SIMD): one step below kGaussTile, a few for whole FP16
 // fields, but four at most (10 iterations, us, 1, 2, 4, 8 steps: 12 rhs of 16^3x32 985,
 // 909, 882, 910; 5 of 32^3x16 1652, 1517, 1466, 1523; 12 of 24^3x48 4810, 4300, 4058,
-// 4102; one of 24^3x48 501, 484, 479, 582).  Calls of 50 iterations with their sources, ms: 16^3, 12 FP64 rhs 0.77
+// 4102; one of 24^3x48 501, 484, 479, 582).  Calls of 50 iterations with their
+// sources, ms: 16^3, 12 FP64 rhs 0.77
 // with 1 step, 1.23 with 4; 32^3, one rhs 0.58 with 1, 1.99 with 8.  (Lanes of one
 // spin each, without a march and with every hop's loads in flight, gain on 8^3
 // only.)  QCD_HIP_GAUSS_ZLEN overrides it, for launches of every size.

@@ -309,9 +309,9 @@ __device__ __forceinline__ void sum_parts(const double *part, unsigned np, unsig
 // the Schur complement, random and point sources: FP64 the same or fewer; FP32 one
 // more in 3, fewer in 57; FP16 more in 33, all Q, fewer in 278.  Most of the 33 are
 // restarted cycles at kappa 0.139 that came out shorter with the rounding of those
-// single steps (8^3x16, GCR(24): 97; in blocks of 1, 2 and 4 141, as in FP64).  Heavy quarks on Q
-// leave directions of a block out: FP64, kappa 0.005, GCR(16) takes 2 cycles of
-// blocks for one of single steps.
+// single steps (8^3x16, GCR(24): 97; in blocks of 1, 2 and 4 141, as in FP64).
+// Heavy quarks on Q leave directions of a block out: FP64, kappa 0.005, GCR(16)
+// takes 2 cycles of blocks for one of single steps.
 
 // Smallest |w_{k+a}|^2 / |v_a|^2 that is told from rounding of the stored vectors:
 // a v_a with less to itself is left out of the cycle
